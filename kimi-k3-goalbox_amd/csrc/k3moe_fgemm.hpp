@@ -271,6 +271,11 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
   const uint32_t wlane = (uint32_t)i * KB * 16 + q * 16;                 // row i of a tile, block q
   const size_t wtile = (size_t)16 * KB * 16;                             // tile stride
   const int sci = l >> 2, scp = 16 * (l & 3);
+  // Scale rows that are not whole 16-byte words (KB % 16 == 8: a reduction
+  // length of 256 mod 512) go in 4-byte loads, kScWide times as many: a 16-byte
+  // load of such a row's last 8 bytes would run past the tensor after its last row.
+  const bool sc_wide = KB % 16 == 0;
+  constexpr int kScWide = 4;
   const uint8_t *const sbase = l < 32 ? a.shi : a.slo;
   const int NSC = (KS + kFScSteps - 1) / kFScSteps;  // scale chunks of a unit
   // chunk c lands with the loads of step sc_step(c): 0 for the first, 2 steps
@@ -278,7 +283,7 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
   // c - 2, whose last step is done once that step's barrier has passed)
   auto chunk_at = [&](int s) { return s == 0 || (s >= 2 && (s - 2) % kFScSteps == 0 && (s - 2) / kFScSteps + 1 < NSC); };
   constexpr int kNR = kFRowsL / 8;                  // 8-row loads per term
-  constexpr int kLoads = 2 * kNR + 1 + kFTiles;     // a loader's loads per step (and kFTiles more with a chunk)
+  constexpr int kLoads = 2 * kNR + 1 + kFTiles;     // a loader's loads per step (and kFTiles, or kScWide kFTiles, more with a chunk)
   struct LoadP {  // one unit's load addresses for this lane
     size_t wrow;
     uint32_t aoffs[kNR];
@@ -309,12 +314,17 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
     char *base = lds + (g % kFRing) * kFSlot;
     if (chunk_at(ks)) {
       const int c = ks == 0 ? 0 : (ks - 2) / kFScSteps + 1;
-      const bool cin = 64 * c + scp < KB;  // lane L: bytes 64c + 16 (L % 4) .. of row L / 4 (zero area past the row)
+      char *const scd = lds + kFOffSc + ((cb0 + c) & 1) * kFScBuf + kFTiles * w * 1024;
 #pragma unroll
       for (int r = 0; r < kFTiles; ++r) {
-        const uint8_t *sp = GU ? (r < 2 ? scl0 : scl1) + (P.wrow + 16 * (r & 1) + sci) * KB + 64 * c + scp
-                               : scl0 + (P.wrow + 16 * r + sci) * KB + 64 * c + scp;
-        load_lds<16>(cin ? sp : zero, lds + kFOffSc + ((cb0 + c) & 1) * kFScBuf + (kFTiles * w + r) * 1024);
+        const uint8_t *tile = (GU && r >= 2 ? scl1 : scl0) + (P.wrow + 16 * (GU ? r & 1 : r)) * KB + 64 * c;
+        if (sc_wide) {  // lane L: bytes 64c + 16 (L % 4) .. of row L / 4 (zero area past the row)
+          load_lds<16>(64 * c + scp < KB ? tile + (size_t)sci * KB + scp : zero, scd + r * 1024);
+        } else {  // lane L of load u: bytes 64c + 4 (L % 16) .. of row 4u + L / 16
+#pragma unroll
+          for (int u = 0; u < kScWide; ++u)
+            load_lds<4>(64 * c + 4 * i < KB ? tile + (size_t)(4 * u + q) * KB + 4 * i : zero, scd + r * 1024 + u * 256);
+        }
       }
     }
 #pragma unroll
@@ -364,10 +374,12 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
         for (int ks = 0; ks < KS; ++ks) {
           // step ks landed (the loads of the step after it may be in flight)
           if (ks + 1 < KS) {
-            if (chunk_at(ks + 1)) wait_vm<kLoads + kFTiles>();
-            else wait_vm<kLoads>();
-          } else if (have_n) {
-            wait_vm<kLoads + kFTiles>();  // the next unit's step 0 carries its first chunk
+            if (!chunk_at(ks + 1)) wait_vm<kLoads>();
+            else if (sc_wide) wait_vm<kLoads + kFTiles>();
+            else wait_vm<kLoads + kScWide * kFTiles>();
+          } else if (have_n) {  // the next unit's step 0 carries its first chunk
+            if (sc_wide) wait_vm<kLoads + kFTiles>();
+            else wait_vm<kLoads + kScWide * kFTiles>();
           } else {
             wait_vm<0>();
           }

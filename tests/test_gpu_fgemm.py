@@ -147,3 +147,15 @@ def test_fp4_and_bf16_grouped_gemms_agree(gpu, seed):
     assert torch.equal(a['route_weights'], b['route_weights'])
     assert bool(torch.isfinite(a['expert_sum']).all())
     assert moe_ref.rel_l2(a['expert_sum'].cpu(), b['expert_sum'].cpu()) < 2e-3
+
+
+@pytest.mark.parametrize('inter', [256, 768])
+def test_grouped_gemms_agree_on_narrow_scale_rows(gpu, inter):
+    """Down-projection scale rows of 8 and 24 bytes (not whole 16-byte words): the
+    FP4-MFMA path against the bf16-MFMA one."""
+    cfg = MoEConfig(f'fgemm-i{inter}', 16, 4, 512, inter, 96, gating='softmax')
+    say(f'case: {cfg.name} seed=2 grouped (FP4 MFMA) vs grouped_bf16')
+    outs = {p: run_step(cfg, 2, gpu, p)[1] for p in ('grouped', 'grouped_bf16')}
+    a, b = outs['grouped'], outs['grouped_bf16']
+    assert torch.equal(a['expert_ids'], b['expert_ids'])
+    assert moe_ref.rel_l2(a['expert_sum'].cpu(), b['expert_sum'].cpu()) < 2e-3

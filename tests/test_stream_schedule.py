@@ -61,6 +61,40 @@ def test_fgemm_stream_schedule(KS, nunits):
     fgemm_stream(KS, nunits)
 
 
+def fgemm_scale_reads(KB, rows, steps_per_chunk=16):
+    """(row, first byte, bytes) of every weight-scale load of a row tile whose rows are KB bytes, per chunk."""
+    nsc = (KB // 4 + steps_per_chunk - 1) // steps_per_chunk
+    for c in range(nsc):
+        if KB % 16 == 0:
+            for lane in range(64):
+                b = 64*c + 16*(lane % 4)
+                if b < KB:
+                    yield lane // 4, b, 16
+        else:
+            for u in range(4):
+                for lane in range(64):
+                    b = 64*c + 4*(lane % 16)
+                    if b < KB:
+                        yield 4*u + lane // 16, b, 4
+
+
+@pytest.mark.parametrize('KB', [8, 16, 24, 40, 48, 56, 64, 72, 112, 224])
+def test_fgemm_scale_loads_stay_in_their_rows(KB):
+    """Every scale byte of the tile is loaded once and no load leaves its row (the last row ends the tensor)."""
+    seen = [[0]*KB for _ in range(16)]
+    for row, b, n in fgemm_scale_reads(KB, 16):
+        assert b + n <= KB, (KB, row, b, n)
+        for j in range(b, b + n):
+            seen[row][j] += 1
+    assert all(v == 1 for row in seen for v in row)
+
+
+@pytest.mark.parametrize('KS', [2, 6, 10, 18])
+def test_fgemm_stream_schedule_narrow_scales(KS):
+    """Rows that are not whole 16-byte words: four times the loads per chunk, the same order."""
+    fgemm_stream(KS, 3, ktiles=16)
+
+
 def sk_order(lo, hi, KS):
     """k_latent_sk's processing order of a run's (tile, step) items: the last
     tile's head when that tile is cut, the first tile's tail when that one is,
