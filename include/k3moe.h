@@ -42,15 +42,16 @@ extern "C" {
  * batches (tokens <= 64, tokens*topk <= 1024) and the multi-kernel path
  * otherwise; the other values force one (DECODE fails with K3MOE_EINVAL when
  * the shape does not fit it). All give the same expert sets. The multi-kernel
- * path (GENERAL) runs the expert projections as grouped GEMMs (weights read
- * once per 128 tokens of an expert) when the experts average at least 16
- * tokens and hidden/latent and inter are multiples of 128, and as per-16-token
- * streams otherwise; GROUPED and STREAMED force one of the two (GROUPED fails
- * with K3MOE_EINVAL when the widths are not multiples of 128). The grouped
- * GEMMs run on the scaled FP4 MFMA (MXFP4 weights as stored, activations as
- * two E4M3 terms with E8M0 block scales, which represent the bf16 values) when
- * latent is a multiple of 512 and inter of 256, and on bf16 MFMA after an
- * in-register decode otherwise; GROUPED_BF16 forces the latter. A single token
+ * path (GENERAL) runs the expert projections as grouped GEMMs when
+ * hidden/latent and inter are multiples of 128: streaming ones (bf16 MFMA on
+ * the weights decoded in registers, units of 32 or 64 tokens of an expert; from
+ * a latent of 512 on) while the experts average fewer than 64 tokens, then, when
+ * latent is a multiple of 512 and inter of 256, GEMMs on the scaled FP4 MFMA
+ * (MXFP4 weights as stored, activations as two E4M3 terms with E8M0 block
+ * scales, which represent the bf16 values); other widths run as per-16-token
+ * streams. GROUPED forces the FP4-MFMA GEMMs (on bf16 MFMA where the widths do
+ * not fit them; fails with K3MOE_EINVAL when they are not multiples of 128),
+ * GROUPED_BF16 the bf16 ones, STREAMED the per-16-token streams. A single token
  * runs on its own persistent kernel when its shape fits (SINGLE below); AUTO
  * picks it then, DECODE forces the general persistent kernel. */
 #define K3MOE_PATH_AUTO 0

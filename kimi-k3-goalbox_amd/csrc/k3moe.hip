@@ -5,8 +5,8 @@
 // (megabench/tasks/quantization.py:40-51). Declarations: include/k3moe.h.
 //
 // Dispatch: B <= 64 tokens (and B*k <= 1024) runs the persistent decode
-// kernel (k3moe_decode.hpp); larger batches run the six-kernel general path
-// (k3moe_general.hpp). Both are enqueued on the caller's stream with no host
+// kernel (k3moe_decode.hpp); larger batches run the general path, a chain of
+// kernels (k3moe_general.hpp, k3moe_sgemm.hpp, k3moe_fgemm.hpp, k3moe_xgemm.hpp). Both are enqueued on the caller's stream with no host
 // synchronisation and no device allocation.
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
@@ -25,6 +25,7 @@
 #include "k3moe_general.hpp"
 #include "k3moe_latent.hpp"
 #include "k3moe_plan.hpp"
+#include "k3moe_sgemm.hpp"
 #include "k3moe_single.hpp"
 #include "k3moe_xgemm.hpp"
 
@@ -179,6 +180,26 @@ int allow_fgemm_lds() {
   static int granted_gu = 0, granted_dn = 0;
   int rc = grant_lds(reinterpret_cast<const void *>(&k_fgemm<true>), kFLds, granted_gu, "FP4 gate/up GEMM");
   if (!rc) rc = grant_lds(reinterpret_cast<const void *>(&k_fgemm<false>), kFLds, granted_dn, "FP4 down GEMM");
+  return rc;
+}
+
+// The streaming grouped GEMMs' instantiations of a plan (pl.sgemm pairs per unit).
+typedef void (*StreamGemm)(Plan, const uint16_t *, const uint8_t *, const uint8_t *, const uint8_t *, const uint8_t *,
+                           char *);
+struct StreamGemms {
+  StreamGemm gu, dn;
+  int lds;
+};
+template <int SM, int Ring, int ScSteps>
+StreamGemms stream_gemms_of() {
+  return {k_sgemm<true, SM, Ring, ScSteps>, k_sgemm<false, SM, Ring, ScSteps>, SGeom<SM, Ring, ScSteps>::lds};
+}
+int stream_gemms(const Plan &p, StreamGemms &g) {
+  static int granted[2][2] = {{0, 0}, {0, 0}};
+  const int v = p.sgemm == 32 ? 0 : 1;
+  g = v == 0 ? stream_gemms_of<32, 5, 16>() : stream_gemms_of<64, 4, 8>();
+  int rc = grant_lds(reinterpret_cast<const void *>(g.gu), g.lds, granted[v][0], "streaming gate/up GEMM");
+  if (!rc) rc = grant_lds(reinterpret_cast<const void *>(g.dn), g.lds, granted[v][1], "streaming down GEMM");
   return rc;
 }
 
@@ -628,6 +649,15 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
     hipLaunchKernelGGL(k_xgemm<false>, dim3(p.G), dim3(kXThreads), kXLds, st, p,
                        reinterpret_cast<const uint16_t *>(ws + p.o_h), down_blocks, down_scales, nullptr, nullptr, ws);
     if ((rc = launch_check("down GEMM"))) return rc;
+  } else if (p.sgemm) {  // few tokens per expert: grouped GEMMs built around the weight stream
+    StreamGemms sg;
+    if ((rc = stream_gemms(p, sg))) return rc;
+    hipLaunchKernelGGL(sg.gu, dim3(p.G), dim3(kSThreads), sg.lds, st, p, xin, gate_blocks, gate_scales, up_blocks,
+                       up_scales, ws);
+    if ((rc = launch_check("streaming gate/up GEMM"))) return rc;
+    hipLaunchKernelGGL(sg.dn, dim3(p.G), dim3(kSThreads), sg.lds, st, p,
+                       reinterpret_cast<const uint16_t *>(ws + p.o_h), down_blocks, down_scales, nullptr, nullptr, ws);
+    if ((rc = launch_check("streaming down GEMM"))) return rc;
   } else {
     const long ng = (long)p.Dmax * p.RTg * p.Sg;
     hipLaunchKernelGGL(k_gateup, dim3(cdiv(ng, kWavesPerBlock)), dim3(kThreads), 0, st, p, xin, gate_blocks,

@@ -23,6 +23,12 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
+// A compile-time int as a value (an unrolled variant's parameter).
+template <int N>
+struct IntC {
+  static constexpr int value = N;
+};
+
 constexpr int kWave = 64;
 constexpr int kBlockK = 32;  // MXFP4 block (quantization.py:10)
 constexpr int kStepK = 128;  // k covered by one k-step of a wave

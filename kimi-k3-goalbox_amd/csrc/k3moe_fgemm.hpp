@@ -158,11 +158,6 @@ __device__ __forceinline__ f32x4 mfma_fp4x8(const u32x4 &a, const i32x8 &b, uint
 // s_waitcnt with lgkmcnt(0) and the other counters at their maxima (no wait on them)
 constexpr int kLgkmZero = 0xC07F;
 
-template <int N>
-struct IntC {
-  static constexpr int value = N;
-};
-
 // Activation operand arrays of one GEMM: rows of two E4M3 terms and their scales.
 struct MxAct {
   const uint8_t *hi, *lo, *shi, *slo;

@@ -230,12 +230,14 @@ __global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restr
 // layout is deterministic.
 //   k_group_count  one workgroup per chunk: the chunk's expert histogram
 //                  (LDS atomics) -> cnt[chunk][e]
-//   k_group_scan   one workgroup: per expert the chunks' counts summed in
-//                  chunk order (exclusive prefix per chunk), then a scan over
-//                  the experts of the totals and of the active flags; writes
-//                  the active list, offsets and counts, and turns cnt into the
-//                  absolute first position of each (chunk, expert) run; clears
-//                  the gate/up split arrival counters for this step
+//   k_group_scan   one workgroup, thread e for expert e: the chunks' counts
+//                  summed (8 loads in flight: one after the other, 32 chunks
+//                  took 17 us), then a scan over the experts of the totals,
+//                  the active flags and the numbers of groups; writes the
+//                  active list, offsets and counts and the streaming GEMMs'
+//                  group table, and turns cnt into the absolute first position
+//                  of each (chunk, expert) run; clears the gate/up split
+//                  arrival counters of the per-16-token streams
 //   k_group_place  one workgroup per chunk: a pair's rank among its expert's
 //                  pairs in the chunk, from per-expert token bitmaps (popcounts
 //                  of the bits below it), gives its position
@@ -252,45 +254,79 @@ __global__ __launch_bounds__(256) void k_group_count(Plan pl, char *ws) {
   for (int e = tid; e < pl.E; e += 256) cnt[e] = s_cnt[e];
 }
 
+// Inclusive scans of three values over the workgroup's 1024 threads.
+__device__ __forceinline__ void block_scan3(int v[3], int (*s_sum)[3]) {
+  const int l = threadIdx.x & 63, w = wave_id();
+#pragma unroll
+  for (int j = 0; j < 3; ++j) v[j] = wave_incl_scan(v[j]);
+  if (l == 63) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s_sum[w][j] = v[j];
+  }
+  __syncthreads();
+  for (int ww = 0; ww < w; ++ww) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) v[j] += s_sum[ww][j];
+  }
+}
+
 __global__ __launch_bounds__(1024) void k_group_scan(Plan pl, char *ws) {
-  __shared__ int s_off[kMaxExperts];
-  __shared__ int s_act[kMaxExperts];
+  static_assert(kMaxExperts == 1024, "one thread per expert");
+  constexpr int kBatch = 8;  // chunk counts in flight per thread
+  __shared__ int s_sum[16][3];
   const int tid = threadIdx.x, E = pl.E;
   const int nch = cdiv(pl.B, kGroupChunk);
   int *cnt = reinterpret_cast<int *>(ws + pl.o_gchunk);
-  // per expert: chunk counts -> exclusive prefixes (relative to the expert's first pair)
   int total = 0;
   if (tid < E)
-    for (int c = 0; c < nch; ++c) {
-      const int v = cnt[(size_t)c * E + tid];
-      cnt[(size_t)c * E + tid] = total;
-      total += v;
+    for (int c0 = 0; c0 < nch; c0 += kBatch) {
+      int v[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) v[j] = c0 + j < nch ? cnt[(size_t)(c0 + j) * E + tid] : 0;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) total += v[j];
     }
-  // inclusive Hillis-Steele scans of the totals (s_off) and active flags (s_act);
-  // the block has exactly kMaxExperts threads, one per expert slot
-  s_off[tid] = total;
-  s_act[tid] = total > 0 ? 1 : 0;
-  __syncthreads();
-  for (int d = 1; d < kMaxExperts; d <<= 1) {
-    const int vo = tid >= d ? s_off[tid - d] : 0;
-    const int va = tid >= d ? s_act[tid - d] : 0;
-    __syncthreads();
-    s_off[tid] += vo;
-    s_act[tid] += va;
-    __syncthreads();
+  // the expert's groups: as few as pl.sgemm pairs each allow, of equal size up to whole 16-token tiles
+  int groups = 0, size = 16;
+  if (pl.sgemm && total > 0) {
+    size = cdiv(cdiv(total, cdiv(total, pl.sgemm)), 16) * 16;
+    groups = cdiv(total, size);
   }
-  if (tid == kMaxExperts - 1) *reinterpret_cast<int *>(ws + pl.o_nact) = s_act[tid];
-  const int first = s_off[tid] - total;
+  int sc[3] = {total, total > 0 ? 1 : 0, groups};
+  block_scan3(sc, s_sum);
+  if (tid == kMaxExperts - 1) {
+    int *n = reinterpret_cast<int *>(ws + pl.o_nact);
+    n[0] = sc[1];
+    n[1] = sc[2];
+  }
+  const int first = sc[0] - total;
   if (tid < E && total > 0) {
-    const int d = s_act[tid] - 1;  // exclusive index of this active expert
+    const int d = sc[1] - 1;  // exclusive index of this active expert
     reinterpret_cast<int *>(ws + pl.o_active)[d] = tid;
     reinterpret_cast<int *>(ws + pl.o_aoff)[d] = first;
     reinterpret_cast<int *>(ws + pl.o_acnt)[d] = total;
+    u32x4 *tab = reinterpret_cast<u32x4 *>(ws + pl.o_gtab) + (sc[2] - groups);
+    for (int j = 0; j < groups; ++j)
+      tab[j] = u32x4{(uint32_t)tid, (uint32_t)(first + j * size), (uint32_t)min(size, total - j * size), 0u};
   }
-  if (tid < E)
-    for (int c = 0; c < nch; ++c) cnt[(size_t)c * E + tid] += first;
-  int *gcnt = reinterpret_cast<int *>(ws + pl.o_gcnt);
-  for (int i = tid; i < pl.Dmax * pl.RTg; i += 1024) gcnt[i] = 0;
+  // chunk counts -> the absolute first position of each (chunk, expert) run
+  if (tid < E) {
+    int at = first;
+    for (int c0 = 0; c0 < nch; c0 += kBatch) {
+      int v[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) v[j] = c0 + j < nch ? cnt[(size_t)(c0 + j) * E + tid] : 0;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        if (c0 + j < nch) cnt[(size_t)(c0 + j) * E + tid] = at;
+        at += v[j];
+      }
+    }
+  }
+  if (!pl.xgemm && !pl.sgemm) {
+    int *gcnt = reinterpret_cast<int *>(ws + pl.o_gcnt);
+    for (int i = tid; i < pl.Dmax * pl.RTg; i += 1024) gcnt[i] = 0;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_group_place(Plan pl, char *ws) {

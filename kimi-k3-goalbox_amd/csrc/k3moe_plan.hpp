@@ -26,7 +26,9 @@ constexpr int kThreads = kWavesPerBlock * 64;
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTopk = 32;
 constexpr int kGroupChunk = 128;   // tokens per placement chunk in k_group
-constexpr int kXMinPairsPerExpert = 16;  // general path: grouped GEMMs from this many token-expert pairs per expert
+constexpr int kXMinPairsPerExpert = 16;  // general path: token-expert pairs per expert from which units hold more than 32
+constexpr int kSMaxPairsPerExpert = 64;  // ... and from which the FP4-MFMA GEMMs take over
+constexpr int kSMinWidth = 512;  // general path: least K of the streaming grouped GEMMs (their loads run up to 4 k-steps ahead)
 constexpr int kMaxRouterSplits = 8;      // general path: router k-splits (partials summed by the top-k kernel)
 
 constexpr int kDecWaves = 8;       // decode path: waves per workgroup
@@ -131,6 +133,7 @@ struct Plan {
   int single;     // 1: the single-token kernel runs the step (k3moe_single.hpp)
   int redundant;  // 1: every workgroup routes every token (no barrier before grouping)
   int xgemm;      // general path: 1 = grouped-GEMM expert kernels, 0 = per-16-token streams
+  int sgemm;      // general path: the streaming grouped GEMMs (k3moe_sgemm.hpp) and their pairs per unit; 0: not them
   int fgemm;      // grouped GEMMs on the scaled FP4 MFMA with two-term E4M3 activations (k3moe_fgemm.hpp)
   int lat_in;     // single-token or decode kernel: 1 = it also computes the latent block's inputs (latent, shared_h)
   int lat_S;      // ... the shared experts' width S
@@ -138,7 +141,7 @@ struct Plan {
   // workspace byte offsets (o_ebf: the decode kernel's bf16 copy of the expert
   // sum, B x K, which the latent block's output phase reads)
   size_t o_ctl, o_zero, o_logit, o_ids, o_w, o_nact, o_active, o_aoff, o_acnt, o_ptok, o_pw, o_pof, o_gpart, o_gcnt,
-      o_gchunk, o_h, o_y, o_xq, o_hq, o_ebf, o_trace, total;
+      o_gchunk, o_gtab, o_h, o_y, o_xq, o_hq, o_ebf, o_trace, total;
 };
 
 __host__ __device__ inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
@@ -353,14 +356,27 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
       p.B <= kDecMaxTokens && p.P <= kDecMaxPairs && (long)p.B * p.Epad * 8 <= part_room &&
       decode_lds(p) <= kDecMaxLds - kDecStaticLds)
     p.path = kPathDecode;
-  // general path expert kernels: grouped GEMMs when the experts average at
-  // least kXMinPairsPerExpert tokens (and the widths allow 128-k steps)
-  const bool widths = p.K % 128 == 0 && p.I % 128 == 0;
-  p.xgemm = d.path == K3MOE_PATH_GROUPED || d.path == K3MOE_PATH_GROUPED_BF16 ||
-            (d.path != K3MOE_PATH_STREAMED && widths && (long)p.P >= (long)kXMinPairsPerExpert * p.E);
-  // the FP4-MFMA grouped GEMMs take whole units of output rows: 256 of I for gate/up, 512 of K for down
-  // and whole 128-k steps
-  p.fgemm = p.xgemm && d.path != K3MOE_PATH_GROUPED_BF16 && p.K % 512 == 0 && p.I % 256 == 0;
+  // general path expert kernels (widths allowing 128-k steps). By the pairs per
+  // expert n = P / E: the streaming GEMMs with 32 pairs per unit below
+  // kXMinPairsPerExpert and with 64 below kSMaxPairsPerExpert (or above it, where
+  // the widths do not fit the FP4-MFMA GEMMs), the FP4-MFMA GEMMs from there.
+  // Gate/up + down us on a TP8 rank's shard, 32 / 64 / FP4: n = 4: 149 + 82 /
+  // 154 + 89 / -, n = 15: 209 + 102 / 182 + 114 / -, n = 31: 271 + 156 / 262 +
+  // 158 / 262 + 231, n = 62: 386 + 248 / 329 + 239 / 314 + 303; unsharded experts,
+  // n = 85: - / 2700 + 1223 / 2678 + 1209. The Kimi rank, n = 14: 302 + 165 /
+  // 314 + 161, n = 27: 363 + 209 / 361 + 179.
+  const bool widths = p.K % 128 == 0 && p.I % 128 == 0, fp4_widths = p.K % 512 == 0 && p.I % 256 == 0;
+  const bool grouped = d.path == K3MOE_PATH_GROUPED || d.path == K3MOE_PATH_GROUPED_BF16;
+  const bool many = (long)p.P >= (long)kXMinPairsPerExpert * p.E;
+  p.sgemm = 0;
+  if (!grouped && d.path != K3MOE_PATH_STREAMED && widths && p.K >= kSMinWidth) {
+    if (!many) p.sgemm = 32;
+    else if ((long)p.P < (long)kSMaxPairsPerExpert * p.E || !fp4_widths) p.sgemm = 64;
+  }
+  // the other grouped GEMMs, on the FP4 MFMA where the widths are whole units of
+  // output rows (256 of I for gate/up, 512 of K for down) and whole 128-k steps
+  p.xgemm = grouped || (d.path != K3MOE_PATH_STREAMED && widths && many && !p.sgemm);
+  p.fgemm = p.xgemm && d.path != K3MOE_PATH_GROUPED_BF16 && fp4_widths;
   p.Srw = (int)(p.G / p.RTr);  // decode router units: (row tile, split), every token tile
   if (p.Srw > srw_cap) p.Srw = srw_cap;
   if (p.Srw < 1) p.Srw = 1;
@@ -388,7 +404,7 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   p.o_logit = take((size_t)logit_splits * p.B * p.Epad * 4);
   p.o_ids = take((size_t)p.P * 4);
   p.o_w = take((size_t)p.P * 4);
-  p.o_nact = take(4);
+  p.o_nact = take(16);  // {active experts, groups}
   p.o_active = take((size_t)p.E * 4);
   p.o_aoff = take((size_t)p.E * 4);
   p.o_acnt = take((size_t)p.E * 4);
@@ -396,9 +412,12 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   p.o_pw = take((size_t)p.P * 4);
   p.o_pof = take((size_t)p.P * 4);
   const bool general = p.path == kPathGeneral;
-  p.o_gpart = take(general && p.Sg > 1 ? (size_t)p.Sg * p.P * 2 * p.I * 4 : 0);
-  p.o_gcnt = take(general ? (size_t)p.Dmax * p.RTg * 4 : 0);
+  const bool streams = general && !p.xgemm && !p.sgemm;
+  p.o_gpart = take(streams && p.Sg > 1 ? (size_t)p.Sg * p.P * 2 * p.I * 4 : 0);
+  p.o_gcnt = take(streams ? (size_t)p.Dmax * p.RTg * 4 : 0);
   p.o_gchunk = take(general ? (size_t)cdiv(p.B, kGroupChunk) * p.E * 4 : 0);  // grouping: per-chunk counts
+  // the streaming GEMMs' group table: {expert, first pair, pairs, -} per group
+  p.o_gtab = take(general && p.sgemm ? (size_t)(p.P / p.sgemm + p.Dmax) * 16 : 0);
   const bool fg = general && p.fgemm;
   p.o_h = take(fg ? 0 : (size_t)p.P * p.I * 2);
   // two-term E4M3 activations of the FP4-MFMA GEMMs: expert inputs [B, K] and h [P, I]

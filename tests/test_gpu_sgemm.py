@@ -1,0 +1,65 @@
+"""GPU checks of the streaming grouped GEMMs (k_sgemm; run with -m gpu).
+
+Batches past the decode kernel's whose experts average fewer than 16 tokens run
+them on the general path. Checked against the per-16-token streams on the same
+routing (the same products, summed in fp32 in another order, so the bf16
+roundings of gate, up, h and y flip now and then: the bar of the grouped GEMMs'
+comparison) at the edges of the units: 1 to 33 and 64 to 65 tokens of an expert
+(one or two 16-token tiles, one to three groups), reductions of 1 to 8 k-steps,
+odd counts, scale rows that are not whole 16-byte words, a partial row block,
+and no expert active twice in a row.
+"""
+
+import pytest
+import torch
+
+import k3moe
+from k3moe import synthetic
+from k3moe.configs import MoEConfig
+from oracle import moe_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def both(cfg, seed, dev, routes=None):
+    g = {k: (v.to(dev) if isinstance(v, torch.Tensor) else v) for k, v in
+         synthetic.moe_layer_inputs(cfg, seed, scale_mode='kimi').items()}
+    kw = dict(topk=cfg.topk, gating=cfg.gating, activation=cfg.activation, routes=routes, latent=g.get('latent'))
+    outs = {p: k3moe.moe_step(*synthetic.step_args(g), path=p, **kw) for p in ('general', 'streamed')}
+    torch.cuda.synchronize(dev)
+    return outs['general'], outs['streamed']
+
+
+def check(a, b):
+    assert torch.equal(a['expert_ids'], b['expert_ids'])
+    assert torch.equal(a['route_weights'], b['route_weights'])
+    assert bool(torch.isfinite(a['expert_sum']).all())
+    assert moe_ref.rel_l2(a['expert_sum'].cpu(), b['expert_sum'].cpu()) < 2e-3
+
+
+@pytest.mark.parametrize('cfg', [
+    MoEConfig('sgemm-i128', 24, 4, 512, 128, 70),                               # 4 and 1 k-steps
+    MoEConfig('sgemm-k640-i384', 32, 4, 640, 384, 100, activation='silu'),      # narrow scales, a partial row block
+    MoEConfig('sgemm-i512', 16, 2, 1024, 512, 90, gating='softmax'),            # whole scale words in both
+    MoEConfig('sgemm-k3584-i384', 48, 16, 512, 384, 66, latent=3584),    # two scale chunks
+    MoEConfig('sgemm-b800', 896, 16, 256, 128, 800, latent=512),                # many groups
+], ids=lambda c: c.name)
+def test_streaming_gemms_match_the_streams(gpu, cfg):
+    say(f'case: {cfg.name} seed=6 general (k_sgemm) vs streamed')
+    check(*both(cfg, 6, gpu))
+
+
+@pytest.mark.parametrize('counts', [(1, 16, 17, 32, 33), (64, 65, 2, 1), (15, 31, 48)])
+def test_streaming_gemms_token_counts(gpu, counts):
+    """Forced routes that give experts exactly these token counts; every token's second expert spreads over the rest."""
+    B, E = sum(counts), 64
+    cfg = MoEConfig('sgemm-counts', E, 2, 768, 256, max(B, 65))
+    first = [e for e, n in enumerate(counts) for _ in range(n)] + [len(counts)]*(cfg.tokens - B)
+    lo = len(counts) + 1
+    routes = torch.tensor([[e, lo + t % (E - lo)] for t, e in enumerate(first)], dtype=torch.int64, device=gpu)
+    say(f'case: {cfg.name} tokens per expert {counts} seed=1')
+    check(*both(cfg, 1, gpu, routes))
