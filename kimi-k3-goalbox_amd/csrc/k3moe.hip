@@ -24,6 +24,7 @@
 #include "k3moe_fgemm.hpp"
 #include "k3moe_general.hpp"
 #include "k3moe_latent.hpp"
+#include "k3moe_lgemm.hpp"
 #include "k3moe_plan.hpp"
 #include "k3moe_sgemm.hpp"
 #include "k3moe_single.hpp"
@@ -215,17 +216,10 @@ int check_latent_dims(const k3moe_latent_dims *d) {
   return K3MOE_OK;
 }
 
-// Plans of both latent kernels for a launch of min(tokens, kLatMaxTokens)
-// tokens (larger batches run as consecutive launches of up to that many; the
-// workspace covers the larger plan of the full launch, which also covers a
-// shorter last one).
+// Plans of both latent kernels for up to kLatMaxTokens tokens.
 int latent_plans(const k3moe_latent_dims *d, int n_cus, LatPlan &pin, LatPlan &pout) {
-  int rc = check_latent_dims(d);
-  if (rc) return rc;
-  k3moe_latent_dims c = *d;
-  if (c.tokens > kLatMaxTokens) c.tokens = kLatMaxTokens;
-  const char *why = latent_plan(c, n_cus, 0, pin);
-  if (!why) why = latent_plan(c, n_cus, 1, pout);
+  const char *why = latent_plan(*d, n_cus, 0, pin);
+  if (!why) why = latent_plan(*d, n_cus, 1, pout);
   if (why) return fail(K3MOE_EINVAL, "latent block geometry B=%d h=%d lh=%d S=%d: %s", d->tokens, d->hidden,
                        d->latent, d->shared, why);
   if (trace_enabled()) {  // one trace area for both kernels, the last 1024 x kTraceSlots x 8 bytes
@@ -233,6 +227,31 @@ int latent_plans(const k3moe_latent_dims *d, int n_cus, LatPlan &pin, LatPlan &p
     pin.o_trace = pout.o_trace = at;
     pin.total = pout.total = at + 1024L * kTraceSlots * 8;
   }
+  return K3MOE_OK;
+}
+
+// Workspace bytes of the block's projections.
+int latent_bytes(const k3moe_latent_dims *d, int n_cus, size_t &need) {
+  int rc = check_latent_dims(d);
+  if (rc) return rc;
+  long in, out;
+  if (d->tokens > kLatMaxTokens) {
+    k3moe_latent_dims c = *d;  // (the geometries are those the 64-token kernels take)
+    c.tokens = kLatMaxTokens;
+    LatPlan sin, sout;
+    if ((rc = latent_plans(&c, n_cus, sin, sout))) return rc;
+    LgPlan pin, pout;
+    lgemm_plan(*d, kDefaultCus, 0, pin);
+    lgemm_plan(*d, kDefaultCus, 1, pout);
+    in = pin.total;
+    out = pout.total;
+  } else {
+    LatPlan pin, pout;
+    if ((rc = latent_plans(d, n_cus, pin, pout))) return rc;
+    in = pin.total;
+    out = pout.total;
+  }
+  need = (size_t)(in > out ? in : out);
   return K3MOE_OK;
 }
 
@@ -246,42 +265,66 @@ int allow_latent_lds(int out, int sk, int bytes) {
   return grant_lds(fn, kLatMaxLds, granted[sk][out], "latent block");
 }
 
-int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size_t workspace_bytes, void *stream) {
-  LatPlan pin, pout;
-  int rc = latent_plans(dims, device_cus(), pin, pout);
+// More than kLatMaxTokens tokens: the GEMMs of k3moe_lgemm.hpp.
+template <int OUT, int RW, int TW>
+int lgemm_launch_as(const LgPlan &p, const LatArgs &a, hipStream_t st) {
+  typedef LgGeom<RW, TW> Geo;
+  static int granted = 0;
+  int rc = grant_lds(reinterpret_cast<const void *>(&k_lgemm<OUT, RW, TW>), Geo::lds, granted, "latent GEMM");
   if (rc) return rc;
-  const size_t need = (size_t)(pin.total > pout.total ? pin.total : pout.total);
+  uint16_t *en = reinterpret_cast<uint16_t *>(a.ws + p.o_en);
+  float *part = reinterpret_cast<float *>(a.ws + p.o_part);
+  if (OUT) {
+    hipLaunchKernelGGL(k_lnorm, dim3(p.B), dim3(256), 0, st, p.lh, a.esum, a.norm, en);
+    if ((rc = launch_check("latent norm"))) return rc;
+  }
+  hipLaunchKernelGGL((k_lgemm<OUT, RW, TW>), dim3(p.G), dim3(kLgThreads), Geo::lds, st, p, OUT ? en : a.x, a.x, a.wa,
+                     a.wb, a.wc, a.ya, a.yb, part);
+  if ((rc = launch_check("latent GEMM"))) return rc;
+  if (p.splits > 1) {
+    hipLaunchKernelGGL(k_lreduce<OUT>, dim3(cdiv((long)p.B * (p.N / 4), 256)), dim3(256), 0, st, p, part, a.ya, a.yb);
+    if ((rc = launch_check("latent GEMM sums"))) return rc;
+  }
+  return K3MOE_OK;
+}
+
+template <int OUT, int RW>
+int lgemm_launch_rows(const LgPlan &p, const LatArgs &a, hipStream_t st) {
+  if (p.TW == 4) return lgemm_launch_as<OUT, RW, 4>(p, a, st);
+  if (p.TW == 3) return lgemm_launch_as<OUT, RW, 3>(p, a, st);
+  return lgemm_launch_as<OUT, RW, 2>(p, a, st);
+}
+
+template <int OUT>
+int lgemm_launch(const k3moe_latent_dims *dims, const LatArgs &a, hipStream_t st) {
+  LgPlan p;
+  lgemm_plan(*dims, kDefaultCus, OUT, p);
+  p.G = 1;
+  while (p.G * 2 <= device_cus() && p.G * 2 <= 1024) p.G *= 2;
+  if (p.RW == 8) return lgemm_launch_rows<OUT, 8>(p, a, st);
+  if (p.RW == 5) return lgemm_launch_rows<OUT, 5>(p, a, st);
+  if (p.RW == 4) return lgemm_launch_rows<OUT, 4>(p, a, st);
+  return lgemm_launch_rows<OUT, 2>(p, a, st);
+}
+
+int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size_t workspace_bytes, void *stream) {
+  size_t need = 0;
+  int rc = latent_bytes(dims, device_cus(), need);
+  if (rc) return rc;
   if (!a.ws || workspace_bytes < need)
     return fail(K3MOE_EWORKSPACE, "workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if (reinterpret_cast<uintptr_t>(a.ws) % 256) return fail(K3MOE_EWORKSPACE, "workspace must be 256-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const long h = dims->hidden, lh = dims->latent, S = dims->shared;
-  for (int b0 = 0; b0 < dims->tokens; b0 += kLatMaxTokens) {  // token rows b0 .. b0 + nb - 1
-    k3moe_latent_dims c = *dims;
-    c.tokens = dims->tokens - b0 < kLatMaxTokens ? dims->tokens - b0 : kLatMaxTokens;
-    LatPlan p;
-    const char *why = latent_plan(c, device_cus(), out, p);
-    if (why) return fail(K3MOE_EINVAL, "latent block geometry B=%d h=%d lh=%d S=%d: %s", c.tokens, c.hidden,
-                         c.latent, c.shared, why);
-    p.o_trace = (out ? pout : pin).o_trace;
-    LatArgs ac = a;
-    if (!out) {
-      ac.x = a.x + b0 * h;
-      ac.ya = a.ya + b0 * lh;
-      ac.yb = a.yb + b0 * S;
-    } else {
-      ac.x = a.x + b0 * S;
-      ac.esum = a.esum + b0 * lh;
-      ac.ya = a.ya + b0 * h;
-    }
-    if ((rc = allow_latent_lds(out, p.sk, p.lds_total))) return rc;
-    if (p.sk && out) hipLaunchKernelGGL(k_latent_sk<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
-    else if (p.sk) hipLaunchKernelGGL(k_latent_sk<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
-    else if (out) hipLaunchKernelGGL(k_latent<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
-    else hipLaunchKernelGGL(k_latent<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
-    if ((rc = launch_check(out ? "latent_out" : "latent_in"))) return rc;
-  }
-  return K3MOE_OK;
+  if (dims->tokens > kLatMaxTokens) return out ? lgemm_launch<1>(dims, a, st) : lgemm_launch<0>(dims, a, st);
+  LatPlan pin, pout;
+  if ((rc = latent_plans(dims, device_cus(), pin, pout))) return rc;
+  const LatPlan &p = out ? pout : pin;
+  if ((rc = allow_latent_lds(out, p.sk, p.lds_total))) return rc;
+  if (p.sk && out) hipLaunchKernelGGL(k_latent_sk<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
+  else if (p.sk) hipLaunchKernelGGL(k_latent_sk<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
+  else if (out) hipLaunchKernelGGL(k_latent<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
+  else hipLaunchKernelGGL(k_latent<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
+  return launch_check(out ? "latent_out" : "latent_in");
 }
 
 // The expert GEMMs' activation, elementwise (debug entry point k3moe_activation).
@@ -675,11 +718,11 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
 
 int k3moe_latent_workspace_bytes(const k3moe_latent_dims *dims, size_t *bytes) {
   g_err[0] = 0;
-  LatPlan pin, pout;
-  int rc = latent_plans(dims, kDefaultCus, pin, pout);
+  size_t need = 0;
+  int rc = latent_bytes(dims, kDefaultCus, need);
   if (rc) return rc;
   if (!bytes) return fail(K3MOE_EINVAL, "bytes is NULL");
-  *bytes = (size_t)(pin.total > pout.total ? pin.total : pout.total);
+  *bytes = need;
   return K3MOE_OK;
 }
 

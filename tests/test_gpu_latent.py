@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 # reference's batches, and small or ragged shapes (token tiles, splits and row tiles partly filled)
 SHAPES = [(1, 7168, 3584, 768), (8, 7168, 3584, 768), (64, 7168, 3584, 768), (3, 256, 128, 128),
           (17, 512, 256, 128), (33, 1024, 512, 256), (40, 2048, 1024, 384), (1, 128, 128, 128),
-          (100, 1024, 512, 256), (130, 512, 256, 128),   # more than 64 tokens: launches of 64 rows
+          (100, 1024, 512, 256), (130, 512, 256, 128),   # more than 64 tokens: the GEMMs
           (40, 5120, 2560, 384)]  # latent_out streamed with cut row tiles (320 tiles of 23 steps, 256 runs)
 
 
