@@ -768,11 +768,19 @@ int k3moe_mxfp4_decode(const uint8_t *blocks, const uint8_t *scales, int64_t n_b
     return fail(K3MOE_EINVAL, "out_dtype must be f32 or bf16, got %d", out_dtype);
   if (n_blocks == 0) return K3MOE_OK;
   if (!blocks || !scales || !out) return fail(K3MOE_EINVAL, "a required pointer is NULL");
-  const int64_t n = n_blocks * 16;
-  long grid = (long)((n + 255) / 256);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const bool f32 = out_dtype == K3MOE_DTYPE_F32;
+  if (reinterpret_cast<uintptr_t>(blocks) % (f32 ? 2 : 4) == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+    // one pass of kDecUnroll words per thread up to kDecGrid workgroups
+    long grid = (long)((n_blocks * (f32 ? 8 : 4) + 256 * kDecUnroll - 1) / (256 * kDecUnroll));
+    if (grid > kDecGrid) grid = kDecGrid;
+    if (f32) hipLaunchKernelGGL(k_decode<true>, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out);
+    else hipLaunchKernelGGL(k_decode<false>, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out);
+    return launch_check("decode");
+  }
+  long grid = (long)((n_blocks * 16 + 255) / 256);
   if (grid > 65536) grid = 65536;
-  hipLaunchKernelGGL(k_decode, dim3((unsigned)grid), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), blocks,
-                     scales, n_blocks, out_dtype, out);
+  hipLaunchKernelGGL(k_decode_bytes, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out_dtype, out);
   return launch_check("decode");
 }
 
@@ -800,10 +808,16 @@ int k3moe_mxfp4_encode(const void *in, int32_t in_dtype, int64_t n_blocks, uint8
   if (!in || !blocks || !scales) return fail(K3MOE_EINVAL, "a required pointer is NULL");
   if (reinterpret_cast<uintptr_t>(in) % 16 || reinterpret_cast<uintptr_t>(blocks) % 4)
     return fail(K3MOE_EINVAL, "in must be 16-byte aligned and blocks 4-byte aligned");
-  long grid = (long)((n_blocks + kEncThreads / 4 - 1) / (kEncThreads / 4));
-  if (grid > 16384) grid = 16384;
-  hipLaunchKernelGGL(k_encode, dim3((unsigned)grid), dim3(kEncThreads), 0, reinterpret_cast<hipStream_t>(stream), in,
-                     in_dtype, n_blocks, blocks, scales);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int per = kEncThreads / (in_dtype == K3MOE_DTYPE_F32 ? 8 : 4);  // blocks per workgroup and pass
+  long grid = (long)((n_blocks + per - 1) / per);
+  if (grid > kEncGrid) grid = kEncGrid;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kEncThreads), 0, st, in, n_blocks, blocks, scales);
+  };
+  if (in_dtype == K3MOE_DTYPE_F32) launch(k_encode<K3MOE_DTYPE_F32>);
+  else if (in_dtype == K3MOE_DTYPE_BF16) launch(k_encode<K3MOE_DTYPE_BF16>);
+  else launch(k_encode<K3MOE_DTYPE_F16>);
   return launch_check("encode");
 }
 

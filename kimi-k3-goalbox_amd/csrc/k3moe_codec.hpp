@@ -1,7 +1,8 @@
-// MXFP4 encoder: pack_mxfp4 of megabench/tasks/quantization.py:13-37 on the
-// GPU, bit for bit with its torch CPU chain (fp32 throughout).
+// MXFP4 codec on the GPU: unpack_mxfp4 (megabench/tasks/quantization.py:40-51,
+// k_decode*) and pack_mxfp4 (:13-37, k_encode), bit for bit with their torch CPU
+// chains.
 //
-// Per block of 32 values along the last axis:
+// Encoder (fp32 throughout). Per block of 32 values along the last axis:
 //   e      = ceil(log2(max(max|x| / 6, 2^-126))), clamped to [-126, 127]
 //            (:24-26). log2 is torch's fp32 logarithm, which rounds to the
 //            nearest fp32: for a quotient v = 2^n (1 + j 2^-23) with j > 0 the
@@ -21,23 +22,38 @@
 // int32 as INT_MIN, so the scale byte wraps to 127 and ldexp scales by
 // 2^INT_MIN = 0 (NaN and infinite elements then take code 7, finite ones 0).
 //
-// Layout: 4 lanes per block, lane s of the group holding elements 8s .. 8s+7
-// (one 16-byte load of bf16 / fp16, two of fp32), so a wave reads 16
-// consecutive blocks with contiguous 16-byte loads and writes their 256 packed
-// bytes with contiguous 4-byte stores and their 16 scale bytes with one byte
-// store per block; the block maximum is two xor-shuffles.
-// HBM-bound: per block 32 input values in, 17 bytes out.
+// Layout: a lane takes one 16-byte load, 8 bf16 / fp16 values (4 lanes per
+// block) or 4 fp32 values (8 lanes), so a wave reads contiguous 16-byte words
+// and writes contiguous packed bytes; the block's maximum magnitude meets in the
+// lanes' xor-shuffles as integers (packed 16-bit ones for the 16-bit types),
+// whose order is the magnitudes' and which see a NaN as the largest. The values
+// are rounded by the hardware's fp32 -> E2M1 conversion (nearest, ties to even,
+// saturating), which keeps the sign of a zero: the product is added to +0 first,
+// so that -0 and a product that underflows give code 0 as a < 0 does. The
+// quotient amax / 6 is only needed where its mantissa is next to a power of two:
+// elsewhere amax x (1/6), a few ulps off, has the same exponent.
+// HBM-bound: per block 32 input values in, 17 bytes out. A TP8 rank's bf16 gate
+// weights [384, 256, 7168]: 320 us, 5.6 TB/s (550 us with the seven
+// boundary comparisons per element and the division per lane).
 #pragma once
 
+#include "k3moe.h"
 #include "k3moe_device.hpp"
 
 namespace k3moe {
 
 constexpr int kEncThreads = 256;
+// Workgroups, at most (the rest by a grid stride). The gate weights below in us, encode and
+// decode: 2048 workgroups 362 / 359, 16384 398 / 381, 65536 320 / 310, no limit 361 / 316.
+constexpr long kEncGrid = 65536, kDecGrid = 65536;
 
 // The block exponent e (before the +127 bias) of a finite or infinite block
 // maximum, as torch's chain computes it (see the file comment).
 __device__ __forceinline__ int mx_block_exponent(float amax) {
+  // amax x fp32(1/6) is within 2 ulps of the IEEE quotient: 4 mantissa steps away from a power
+  // of two, and above the 64 steps past one that need the logarithm, both lie in one binade
+  const uint32_t qb = __float_as_uint(__fmul_rn(amax, 1.0f / 6.0f)), qj = qb & 0x7FFFFFu;
+  if (qj >= 68u && qj <= 0x7FFFFBu && qb >= 0x01000000u && qb < 0x7F000000u) return (int)(qb >> 23) - 126;
   float v = amax / 6.0f;  // IEEE fp32 division
   if (!(v >= 0x1p-126f)) v = 0x1p-126f;
   const uint32_t b = __float_as_uint(v);
@@ -64,56 +80,128 @@ __device__ __forceinline__ float pow2_neg(int e) {
   return e == 127 ? __uint_as_float(0x00400000u) : __uint_as_float((uint32_t)(127 - e) << 23);
 }
 
-// in_dtype: K3MOE_DTYPE_F32 / _BF16 / _F16 (values converted to fp32 exactly)
-__global__ __launch_bounds__(kEncThreads) void k_encode(const void *__restrict__ in, int in_dtype, int64_t n_blocks,
+// DT: K3MOE_DTYPE_BF16 / _F32 / _F16 (values converted to fp32 exactly)
+template <int DT>
+__global__ __launch_bounds__(kEncThreads) void k_encode(const void *__restrict__ in, int64_t n_blocks,
                                                         uint8_t *__restrict__ blocks, uint8_t *__restrict__ scales) {
-  const int s = threadIdx.x & 3;
-  const int64_t stride = (int64_t)gridDim.x * (kEncThreads / 4);
-  for (int64_t blk = (int64_t)blockIdx.x * (kEncThreads / 4) + (threadIdx.x >> 2); blk < n_blocks; blk += stride) {
-    float v[8];
-    if (in_dtype == 1) {  // fp32
-      const float *src = reinterpret_cast<const float *>(in) + blk * 32 + 8 * s;
-      const u32x4 w0 = *reinterpret_cast<const u32x4 *>(src), w1 = *reinterpret_cast<const u32x4 *>(src + 4);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        v[t] = __uint_as_float(w0[t]);
-        v[4 + t] = __uint_as_float(w1[t]);
-      }
+  constexpr int V = DT == K3MOE_DTYPE_F32 ? 4 : 8;  // values per lane
+  constexpr int LPB = 32 / V;                       // lanes per block
+  const int s = threadIdx.x & (LPB - 1);
+  const int64_t stride = (int64_t)gridDim.x * (kEncThreads / LPB);
+  for (int64_t blk = (int64_t)blockIdx.x * (kEncThreads / LPB) + threadIdx.x / LPB; blk < n_blocks; blk += stride) {
+    const u32x4 w = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(in) + (blk * LPB + s) * 16);
+    // the largest magnitude's bits, in the type's own format
+    uint32_t mag;
+    if constexpr (DT == K3MOE_DTYPE_F32) {
+      mag = max(max(w[0] & 0x7FFFFFFFu, w[1] & 0x7FFFFFFFu), max(w[2] & 0x7FFFFFFFu, w[3] & 0x7FFFFFFFu));
     } else {
-      const u32x4 w = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint16_t *>(in) + blk * 32 + 8 * s);
+      typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
+      u16x2 m = __builtin_bit_cast(u16x2, w[0] & 0x7FFF7FFFu);
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const uint32_t h = (w[t >> 1] >> (16 * (t & 1))) & 0xFFFFu;
-        v[t] = in_dtype == 0 ? __uint_as_float(h << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)h);
+      for (int t = 1; t < 4; ++t) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[t] & 0x7FFF7FFFu));
+      mag = max((uint32_t)m[0], (uint32_t)m[1]);
+    }
+#pragma unroll
+    for (int m = 1; m < LPB; m <<= 1) mag = max(mag, shfl_xor(mag, m));
+    float v[V];
+#pragma unroll
+    for (int t = 0; t < V; ++t) {
+      if constexpr (DT == K3MOE_DTYPE_F32) {
+        v[t] = __uint_as_float(w[t]);
+      } else if constexpr (DT == K3MOE_DTYPE_BF16) {
+        v[t] = __uint_as_float(t & 1 ? w[t >> 1] & 0xFFFF0000u : w[t >> 1] << 16);
+      } else {
+        v[t] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[t >> 1] >> (16 * (t & 1))));
       }
     }
-    float amax = 0.f;
-    int nan = 0;
+    constexpr uint32_t inf = DT == K3MOE_DTYPE_F32 ? 0x7F800000u : DT == K3MOE_DTYPE_BF16 ? 0x7F80u : 0x7C00u;
+    uint32_t sbyte = 127u, packed = 0u;
+    if (mag > inf) {  // a NaN in the block
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      amax = fmaxf(amax, fabsf(v[t]));
-      nan |= v[t] != v[t];
-    }
-#pragma unroll
-    for (int m = 1; m < 4; m <<= 1) {
-      amax = fmaxf(amax, shfl_xor(amax, m));
-      nan |= shfl_xor(nan, m);
-    }
-    uint32_t sbyte;
-    float step;
-    if (nan) {
-      sbyte = 127u;
-      step = 0.f;
+      for (int t = 0; t < V; ++t) packed |= e2m1_code(__fmul_rn(v[t], 0.f)) << (4 * t);
     } else {
+      const float amax = DT == K3MOE_DTYPE_F32    ? __uint_as_float(mag)
+                         : DT == K3MOE_DTYPE_BF16 ? __uint_as_float(mag << 16)
+                                                  : (float)__builtin_bit_cast(_Float16, (uint16_t)mag);
       const int e = mx_block_exponent(amax);
       sbyte = (uint32_t)(e + 127);
-      step = pow2_neg(e);
-    }
-    uint32_t packed = 0u;
+      const float step = pow2_neg(e);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) packed |= e2m1_code(__fmul_rn(v[t], step)) << (4 * t);
-    *reinterpret_cast<uint32_t *>(blocks + blk * 16 + 4 * s) = packed;
+      for (int t = 0; t < V; ++t) v[t] = __fadd_rn(__fmul_rn(v[t], step), 0.f);
+      packed = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(packed, v[0], v[1], 1.0f, 0);
+      packed = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(packed, v[2], v[3], 1.0f, 1);
+      if constexpr (V == 8) {
+        packed = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(packed, v[4], v[5], 1.0f, 2);
+        packed = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(packed, v[6], v[7], 1.0f, 3);
+      }
+    }
+    if constexpr (V == 8) *reinterpret_cast<uint32_t *>(blocks + blk * 16 + 4 * s) = packed;
+    else *reinterpret_cast<uint16_t *>(blocks + blk * 16 + 2 * s) = (uint16_t)packed;
     if (s == 0) scales[blk] = (uint8_t)sbyte;
+  }
+}
+
+// Exact MXFP4 decode (quantization.py:40-51): a lane takes the codes of one
+// 16-byte store, 4 packed bytes for bf16 (8 values) and 2 for fp32 (4), through
+// the hardware conversion (exact for every scale byte but 255, whose values are
+// the quiet NaN), kDecUnroll of them a grid apart in flight. HBM-bound: 17 bytes
+// in, 64 or 128 out per block, stored past the caches (a larger output would only
+// evict the input: 310 -> 301 us, at 90000 x 2048 83 -> 66). A TP8 rank's gate
+// weights to bf16: 301 us, 5.9 TB/s (774 us with a byte per thread and the bit
+// construction).
+constexpr int kDecUnroll = 4;
+template <bool F32>
+__global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ blocks, const uint8_t *__restrict__ scales,
+                                                int64_t n_blocks, void *__restrict__ out) {
+  constexpr int LPB = F32 ? 8 : 4;  // lanes per block
+  const int64_t n = n_blocks * LPB, stride = (int64_t)gridDim.x * 256;
+  for (int64_t u0 = (int64_t)blockIdx.x * 256 + threadIdx.x; u0 < n; u0 += stride * kDecUnroll) {
+    uint32_t w[kDecUnroll], s[kDecUnroll];
+#pragma unroll
+    for (int j = 0; j < kDecUnroll; ++j) {
+      const int64_t u = u0 + j * stride < n ? u0 + j * stride : u0;
+      if constexpr (F32) w[j] = reinterpret_cast<const uint16_t *>(blocks)[u];
+      else w[j] = reinterpret_cast<const uint32_t *>(blocks)[u];
+      s[j] = scales[u / LPB];
+    }
+#pragma unroll
+    for (int j = 0; j < kDecUnroll; ++j) {
+      const int64_t u = u0 + j * stride;
+      if (u >= n) break;
+      const float sc = e8m0_to_f32(s[j]);
+      u32x4 o;
+      if constexpr (F32) {
+        typedef __attribute__((ext_vector_type(2))) float f32x2;
+        const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w[j], sc, 0);
+        const f32x2 b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w[j], sc, 1);
+        o = u32x4{__float_as_uint(a[0]), __float_as_uint(a[1]), __float_as_uint(b[0]), __float_as_uint(b[1])};
+      } else {
+        o = __builtin_bit_cast(u32x4, fp4x8_to_bf16(w[j], sc));
+      }
+      if (!scale_is_plain(s[j])) {
+        const uint32_t nan = F32 ? 0x7FC00000u : 0x7FC07FC0u;
+        o = u32x4{nan, nan, nan, nan};
+      }
+      __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(out) + u);
+    }
+  }
+}
+
+// The same one byte per thread by bit construction, for arrays that are not
+// aligned for k_decode's loads and stores.
+__global__ __launch_bounds__(256) void k_decode_bytes(const uint8_t *__restrict__ blocks,
+                                                const uint8_t *__restrict__ scales, int64_t n_blocks,
+                                                int out_dtype, void *out) {
+  const int64_t n = n_blocks * 16;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t byte = blocks[i];
+    const uint32_t s = scales[i / 16];
+    const uint32_t lo = mxfp4_bits(byte & 15u, s), hi = mxfp4_bits(byte >> 4, s);
+    if (out_dtype == K3MOE_DTYPE_F32) {
+      reinterpret_cast<u32x2 *>(out)[i] = u32x2{lo, hi};
+    } else {
+      reinterpret_cast<uint32_t *>(out)[i] = (lo >> 16) | (hi & 0xFFFF0000u);
+    }
   }
 }
 

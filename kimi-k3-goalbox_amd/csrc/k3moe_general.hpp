@@ -7,7 +7,6 @@
 //              registers, MFMA, activation epilogue -> bf16 h          (kimi.py:321-322)
 //   k_down     down projection of every active expert -> bf16 y       (kimi.py:322)
 //   k_combine  FP32 routing-weighted sum in ascending expert order    (kimi.py:318,323)
-// plus k_decode, the exact MXFP4 decode (quantization.py:40-51).
 #pragma once
 
 #include "k3moe_device.hpp"
@@ -552,23 +551,6 @@ __global__ __launch_bounds__(256) void k_combine(Plan pl, char *ws, float *__res
   float *o = out + (size_t)t * pl.K + c;
   *reinterpret_cast<f32x4 *>(o) = f32x4{acc[0], acc[1], acc[2], acc[3]};
   *reinterpret_cast<f32x4 *>(o + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
-}
-
-// Exact MXFP4 decode, one thread per block byte (quantization.py:40-51).
-__global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ blocks,
-                                                const uint8_t *__restrict__ scales, int64_t n_blocks,
-                                                int out_dtype, void *out) {
-  const int64_t n = n_blocks * 16;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t byte = blocks[i];
-    const uint32_t s = scales[i / 16];
-    const uint32_t lo = mxfp4_bits(byte & 15u, s), hi = mxfp4_bits(byte >> 4, s);
-    if (out_dtype == K3MOE_DTYPE_F32) {
-      reinterpret_cast<u32x2 *>(out)[i] = u32x2{lo, hi};
-    } else {
-      reinterpret_cast<uint32_t *>(out)[i] = (lo >> 16) | (hi & 0xFFFF0000u);
-    }
-  }
 }
 
 }  // namespace k3moe

@@ -119,3 +119,38 @@ def test_encode_tp8_rank_gate_round_trip(gpu):
     ref_dec = moe_ref.unpack_mxfp4(p[7].cpu(), s[7].cpu())
     err = (ref_dec - w[7].float().cpu()).abs()
     assert float(err.max()) <= float(w[7].float().abs().amax().cpu())/3    # half a code step at most
+
+
+def test_encode_exponents_next_to_the_fast_range(gpu):
+    """Block maxima whose quotient by 6 is 56 to 76 and 2^23 - 12 to 2^23 - 1 mantissa steps above a power of two:
+    the exponent taken from amax x (1/6) starts and ends there."""
+    say('case: encode exponents around 64 mantissa steps and the next binade, every binade')
+    steps = np.concatenate([np.arange(56, 77), np.arange(2**23 - 12, 2**23)])
+    n = np.arange(-126, 126)
+    amax = (6.0*2.0**n[:, None]*(1.0 + steps[None, :]*2.0**-23)).astype(np.float32).reshape(-1)
+    amax = np.concatenate([amax, np.nextafter(amax, np.float32(0)), np.nextafter(amax, np.float32(np.inf))])
+    amax = amax[np.isfinite(amax)]
+    x = torch.from_numpy(amax)[:, None]*torch.linspace(-1, 1, 32)[None, :]
+    x[:, 3] = -0.0
+    p, s = gpu_pack(x, gpu)
+    q, t = pack_ref.pack_mxfp4(x)
+    assert torch.equal(s, t)
+    assert torch.equal(p, q)
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('offset', [0, 1, 2, 4])
+@pytest.mark.parametrize('n', [1, 5, 1027])
+def test_decode_of_unaligned_blocks(gpu, n, offset, dtype):
+    """Packed bytes that start off a 4- or 2-byte word take the byte-wise decoder; whole-word ones the wide one."""
+    say(f'case: decode {n} blocks at byte offset {offset} to {dtype}')
+    g = torch.Generator().manual_seed(n + offset)
+    raw = torch.randint(0, 256, (offset + 16*n,), generator=g, dtype=torch.uint8).to(gpu)
+    scales = torch.randint(0, 256, (n,), generator=g, dtype=torch.uint8)
+    scales[0] = 255
+    blocks = raw[offset:].view(n, 16)
+    got = k3moe.mxfp4_decode(blocks, scales.to(gpu), dtype).cpu()
+    want = moe_ref.unpack_mxfp4(blocks.cpu(), scales).to(dtype)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(torch.where(got.isnan(), 0, got.view(bits)), torch.where(want.isnan(), 0, want.view(bits)))
