@@ -233,7 +233,8 @@ int k3moe_workspace_status(const void *workspace, int32_t *status, void *stream)
 /* Geometry of the latent MoE block around the routed experts of a Kimi K3
  * layer (kimi.py:317, 325-328; weight shapes kimi.py:112-121):
  *   tokens      B: rows of x (up to 64: kernels that stream the weights once;
- *               more: bf16 GEMMs, whose workspace grows with B)
+ *               more: bf16 GEMMs in the 64-token kernels' workspace, or in
+ *               k3moe_latent_block and k3moe_latent_moe_step the MoE step's)
  *   hidden      h: width of x and of the block's output (7168)
  *   latent      lh: width of the experts' input and of expert_sum (3584)
  *   shared      S: this rank's shared-expert width (intermediate x

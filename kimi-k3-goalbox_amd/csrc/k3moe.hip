@@ -230,28 +230,15 @@ int latent_plans(const k3moe_latent_dims *d, int n_cus, LatPlan &pin, LatPlan &p
   return K3MOE_OK;
 }
 
-// Workspace bytes of the block's projections.
+// Workspace bytes of the block's projections: the 64-token kernels' for any larger batch.
 int latent_bytes(const k3moe_latent_dims *d, int n_cus, size_t &need) {
   int rc = check_latent_dims(d);
   if (rc) return rc;
-  long in, out;
-  if (d->tokens > kLatMaxTokens) {
-    k3moe_latent_dims c = *d;  // (the geometries are those the 64-token kernels take)
-    c.tokens = kLatMaxTokens;
-    LatPlan sin, sout;
-    if ((rc = latent_plans(&c, n_cus, sin, sout))) return rc;
-    LgPlan pin, pout;
-    lgemm_plan(*d, kDefaultCus, 0, pin);
-    lgemm_plan(*d, kDefaultCus, 1, pout);
-    in = pin.total;
-    out = pout.total;
-  } else {
-    LatPlan pin, pout;
-    if ((rc = latent_plans(d, n_cus, pin, pout))) return rc;
-    in = pin.total;
-    out = pout.total;
-  }
-  need = (size_t)(in > out ? in : out);
+  k3moe_latent_dims c = *d;
+  if (c.tokens > kLatMaxTokens) c.tokens = kLatMaxTokens;
+  LatPlan pin, pout;
+  if ((rc = latent_plans(&c, n_cus, pin, pout))) return rc;
+  need = (size_t)(pin.total > pout.total ? pin.total : pout.total);
   return K3MOE_OK;
 }
 
@@ -266,39 +253,33 @@ int allow_latent_lds(int out, int sk, int bytes) {
 }
 
 // More than kLatMaxTokens tokens: the GEMMs of k3moe_lgemm.hpp.
+struct LgemmArgs {
+  const uint16_t *x, *x2, *wa, *wb, *wc;
+  uint16_t *ya, *yb;
+  float *part;
+};
+
 template <int OUT, int RW, int TW>
-int lgemm_launch_as(const LgPlan &p, const LatArgs &a, hipStream_t st) {
+int lgemm_launch_as(const LgPlan &p, const LgemmArgs &a, hipStream_t st) {
   typedef LgGeom<RW, TW> Geo;
   static int granted = 0;
   int rc = grant_lds(reinterpret_cast<const void *>(&k_lgemm<OUT, RW, TW>), Geo::lds, granted, "latent GEMM");
   if (rc) return rc;
-  uint16_t *en = reinterpret_cast<uint16_t *>(a.ws + p.o_en);
-  float *part = reinterpret_cast<float *>(a.ws + p.o_part);
-  if (OUT) {
-    hipLaunchKernelGGL(k_lnorm, dim3(p.B), dim3(256), 0, st, p.lh, a.esum, a.norm, en);
-    if ((rc = launch_check("latent norm"))) return rc;
-  }
-  hipLaunchKernelGGL((k_lgemm<OUT, RW, TW>), dim3(p.G), dim3(kLgThreads), Geo::lds, st, p, OUT ? en : a.x, a.x, a.wa,
-                     a.wb, a.wc, a.ya, a.yb, part);
-  if ((rc = launch_check("latent GEMM"))) return rc;
-  if (p.splits > 1) {
-    hipLaunchKernelGGL(k_lreduce<OUT>, dim3(cdiv((long)p.B * (p.N / 4), 256)), dim3(256), 0, st, p, part, a.ya, a.yb);
-    if ((rc = launch_check("latent GEMM sums"))) return rc;
-  }
-  return K3MOE_OK;
+  hipLaunchKernelGGL((k_lgemm<OUT, RW, TW>), dim3(p.G), dim3(kLgThreads), Geo::lds, st, p, a.x, a.x2, a.wa, a.wb, a.wc,
+                     a.ya, a.yb, a.part);
+  return launch_check(OUT == 2 ? "router" : "latent GEMM");
 }
 
 template <int OUT, int RW>
-int lgemm_launch_rows(const LgPlan &p, const LatArgs &a, hipStream_t st) {
+int lgemm_launch_rows(const LgPlan &p, const LgemmArgs &a, hipStream_t st) {
   if (p.TW == 4) return lgemm_launch_as<OUT, RW, 4>(p, a, st);
   if (p.TW == 3) return lgemm_launch_as<OUT, RW, 3>(p, a, st);
   return lgemm_launch_as<OUT, RW, 2>(p, a, st);
 }
 
+// The plan's k_lgemm variant, on a grid of the device's compute units.
 template <int OUT>
-int lgemm_launch(const k3moe_latent_dims *dims, const LatArgs &a, hipStream_t st) {
-  LgPlan p;
-  lgemm_plan(*dims, kDefaultCus, OUT, p);
+int lgemm_launch(LgPlan p, const LgemmArgs &a, hipStream_t st) {
   p.G = 1;
   while (p.G * 2 <= device_cus() && p.G * 2 <= 1024) p.G *= 2;
   if (p.RW == 8) return lgemm_launch_rows<OUT, 8>(p, a, st);
@@ -307,7 +288,47 @@ int lgemm_launch(const k3moe_latent_dims *dims, const LatArgs &a, hipStream_t st
   return lgemm_launch_rows<OUT, 2>(p, a, st);
 }
 
-int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size_t workspace_bytes, void *stream) {
+// One half of the latent block for more than kLatMaxTokens tokens, in `avail` bytes of workspace.
+template <int OUT>
+int latent_gemm(const k3moe_latent_dims *dims, const LatArgs &a, long avail, hipStream_t st) {
+  LgPlan full;
+  lgemm_plan(*dims, kLgCus, OUT, avail, full);
+  for (int b0 = 0; b0 < dims->tokens; b0 += full.B) {  // token rows b0 .. b0 + p.B - 1
+    LgPlan p = full;
+    if (dims->tokens - b0 < full.B) {
+      k3moe_latent_dims c = *dims;
+      c.tokens = dims->tokens - b0;
+      lgemm_plan(c, kLgCus, OUT, avail, p);
+    }
+    uint16_t *en = reinterpret_cast<uint16_t *>(a.ws + p.o_en);
+    float *part = reinterpret_cast<float *>(a.ws + p.o_part);
+    LgemmArgs g{};
+    g.wa = a.wa; g.wb = a.wb; g.wc = a.wc;
+    g.part = part;
+    int rc;
+    if (OUT) {
+      hipLaunchKernelGGL(k_lnorm, dim3(p.B), dim3(256), 0, st, p.lh, a.esum + (size_t)b0 * p.lh, a.norm, en);
+      if ((rc = launch_check("latent norm"))) return rc;
+      g.x = en;
+      g.x2 = a.x + (size_t)b0 * p.S;
+      g.ya = a.ya + (size_t)b0 * p.h;
+    } else {
+      g.x = a.x + (size_t)b0 * p.h;
+      g.ya = a.ya + (size_t)b0 * p.lh;
+      g.yb = a.yb + (size_t)b0 * p.S;
+    }
+    if ((rc = lgemm_launch<OUT>(p, g, st))) return rc;
+    if (p.splits > 1) {
+      hipLaunchKernelGGL(k_lreduce<OUT>, dim3(cdiv((long)p.B * (p.N / 4), 256)), dim3(256), 0, st, p, part, g.ya, g.yb);
+      if ((rc = launch_check("latent GEMM sums"))) return rc;
+    }
+  }
+  return K3MOE_OK;
+}
+
+// `room`: the workspace bytes that the caller's dimensions grant beyond the latent block's own (0: none)
+int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size_t workspace_bytes, size_t room,
+                  void *stream) {
   size_t need = 0;
   int rc = latent_bytes(dims, device_cus(), need);
   if (rc) return rc;
@@ -315,7 +336,11 @@ int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size
     return fail(K3MOE_EWORKSPACE, "workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if (reinterpret_cast<uintptr_t>(a.ws) % 256) return fail(K3MOE_EWORKSPACE, "workspace must be 256-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dims->tokens > kLatMaxTokens) return out ? lgemm_launch<1>(dims, a, st) : lgemm_launch<0>(dims, a, st);
+  if (dims->tokens > kLatMaxTokens) {
+    if (room > workspace_bytes) room = workspace_bytes;
+    const long avail = (long)(room > need ? room : need);
+    return out ? latent_gemm<1>(dims, a, avail, st) : latent_gemm<0>(dims, a, avail, st);
+  }
   LatPlan pin, pout;
   if ((rc = latent_plans(dims, device_cus(), pin, pout))) return rc;
   const LatPlan &p = out ? pout : pin;
@@ -477,6 +502,18 @@ struct LatInArgs {
   void *out;
   bool *did_out;
 };
+static int latent_in_impl(const k3moe_latent_dims *dims, const void *x, const void *latent_down,
+                          const void *shared_gate, const void *shared_up, void *latent, void *shared_h,
+                          void *workspace, size_t workspace_bytes, size_t room, void *stream);
+static int latent_out_impl(const k3moe_latent_dims *dims, const float *expert_sum, const void *latent_norm,
+                           const void *latent_up, const void *shared_h, const void *shared_down, void *out,
+                           void *workspace, size_t workspace_bytes, size_t room, void *stream);
+// The MoE step's workspace bytes (valid dims), which the block's projections may use before and after it.
+static size_t step_room(const k3moe_dims *dims) {
+  Plan p;
+  make_plan(*dims, kDefaultCus, p, trace_enabled());
+  return p.total;
+}
 constexpr int kNotFused = -1000;  // moe_step_impl: the plan has no one-launch latent path
 
 static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *latent, const void *router,
@@ -517,8 +554,8 @@ int k3moe_latent_moe_step(const k3moe_dims *dims, int32_t shared, const void *x,
   if (rc != kNotFused) return rc;
   // two launches: the input projections, then the step on their latent
   const k3moe_latent_dims ld{dims->tokens, dims->hidden, dims->latent, shared, dims->activation};
-  if ((rc = k3moe_latent_in(&ld, x, latent_down, shared_gate, shared_up, latent, shared_h, workspace,
-                            workspace_bytes, stream)))
+  if ((rc = latent_in_impl(&ld, x, latent_down, shared_gate, shared_up, latent, shared_h, workspace,
+                           workspace_bytes, step_room(dims), stream)))
     return rc;
   return k3moe_moe_step(dims, x, latent, router, router_bias, gate_blocks, gate_scales, up_blocks, up_scales,
                         down_blocks, down_scales, routes, expert_sum, expert_ids, route_weights, shortfall,
@@ -546,16 +583,16 @@ int k3moe_latent_block(const k3moe_dims *dims, int32_t shared, const void *x, co
                          workspace, workspace_bytes, stream, &lat);
   const k3moe_latent_dims ld{dims->tokens, dims->hidden, dims->latent, shared, dims->activation};
   if (rc == kNotFused) {  // the input projections, then the step on their latent
-    if ((rc = k3moe_latent_in(&ld, x, latent_down, shared_gate, shared_up, latent, shared_h, workspace,
-                              workspace_bytes, stream)))
+    if ((rc = latent_in_impl(&ld, x, latent_down, shared_gate, shared_up, latent, shared_h, workspace,
+                             workspace_bytes, step_room(dims), stream)))
       return rc;
     rc = k3moe_moe_step(dims, x, latent, router, router_bias, gate_blocks, gate_scales, up_blocks, up_scales,
                         down_blocks, down_scales, routes, expert_sum, expert_ids, route_weights, shortfall,
                         workspace, workspace_bytes, stream);
   }
   if (rc || did_out) return rc;
-  return k3moe_latent_out(&ld, expert_sum, latent_norm, latent_up, shared_h, shared_down, out, workspace,
-                          workspace_bytes, stream);
+  return latent_out_impl(&ld, expert_sum, latent_norm, latent_up, shared_h, shared_down, out, workspace,
+                         workspace_bytes, step_room(dims), stream);
 }
 
 static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *latent, const void *router,
@@ -651,12 +688,28 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
     return launch_check("decode step");
   }
 
-  const int nr = cdiv(p.B, kRM) * cdiv(p.E, kRExperts) * p.Sr;
-  hipLaunchKernelGGL(k_router, dim3(nr), dim3(kRWaves * 64), 0, st, p, reinterpret_cast<const uint16_t *>(x),
-                     reinterpret_cast<const uint16_t *>(router), ws);
-  if ((rc = launch_check("router"))) return rc;
-  hipLaunchKernelGGL(k_topk, dim3(cdiv(p.B, kWavesPerBlock)), dim3(kThreads), 0, st, p, router_bias, routes, ws,
-                     expert_ids, route_weights, shortfall);
+  if (p.rgemm) {
+    LgPlan lp;
+    lgemm_router_plan(p.B, p.h, p.E, p.Epad, kLgCus, lp);
+    rc = lgemm_launch<2>(lp, LgemmArgs{reinterpret_cast<const uint16_t *>(x), nullptr,
+                                       reinterpret_cast<const uint16_t *>(router), nullptr, nullptr, nullptr, nullptr,
+                                       reinterpret_cast<float *>(ws + p.o_logit)}, st);
+    if (rc) return rc;
+  } else {
+    const int nr = cdiv(p.B, kRM) * cdiv(p.E, kRExperts) * p.Sr;
+    hipLaunchKernelGGL(k_router, dim3(nr), dim3(kRWaves * 64), 0, st, p, reinterpret_cast<const uint16_t *>(x),
+                       reinterpret_cast<const uint16_t *>(router), ws);
+    if ((rc = launch_check("router"))) return rc;
+  }
+  auto topk = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(cdiv(p.B, kWavesPerBlock)), dim3(kThreads), 0, st, p, router_bias, routes, ws,
+                       expert_ids, route_weights, shortfall);
+  };
+  if (p.E <= 128) topk(k_topk<2>);
+  else if (p.E <= 256) topk(k_topk<4>);
+  else if (p.E <= 384) topk(k_topk<6>);
+  else if (p.E <= 512) topk(k_topk<8>);
+  else topk(k_topk<16>);
   if ((rc = launch_check("topk"))) return rc;
   const int nch = cdiv(p.B, kGroupChunk);
   hipLaunchKernelGGL(k_group_count, dim3(nch), dim3(256), 0, st, p, ws);
@@ -726,10 +779,9 @@ int k3moe_latent_workspace_bytes(const k3moe_latent_dims *dims, size_t *bytes) {
   return K3MOE_OK;
 }
 
-int k3moe_latent_in(const k3moe_latent_dims *dims, const void *x, const void *latent_down, const void *shared_gate,
-                    const void *shared_up, void *latent, void *shared_h, void *workspace, size_t workspace_bytes,
-                    void *stream) {
-  g_err[0] = 0;
+static int latent_in_impl(const k3moe_latent_dims *dims, const void *x, const void *latent_down,
+                          const void *shared_gate, const void *shared_up, void *latent, void *shared_h,
+                          void *workspace, size_t workspace_bytes, size_t room, void *stream) {
   if (!x || !latent_down || !shared_gate || !shared_up || !latent || !shared_h)
     return fail(K3MOE_EINVAL, "a required pointer is NULL");
   LatArgs a{};
@@ -740,13 +792,12 @@ int k3moe_latent_in(const k3moe_latent_dims *dims, const void *x, const void *la
   a.ya = reinterpret_cast<uint16_t *>(latent);
   a.yb = reinterpret_cast<uint16_t *>(shared_h);
   a.ws = reinterpret_cast<char *>(workspace);
-  return latent_launch(dims, 0, a, workspace_bytes, stream);
+  return latent_launch(dims, 0, a, workspace_bytes, room, stream);
 }
 
-int k3moe_latent_out(const k3moe_latent_dims *dims, const float *expert_sum, const void *latent_norm,
-                     const void *latent_up, const void *shared_h, const void *shared_down, void *out,
-                     void *workspace, size_t workspace_bytes, void *stream) {
-  g_err[0] = 0;
+static int latent_out_impl(const k3moe_latent_dims *dims, const float *expert_sum, const void *latent_norm,
+                           const void *latent_up, const void *shared_h, const void *shared_down, void *out,
+                           void *workspace, size_t workspace_bytes, size_t room, void *stream) {
   if (!expert_sum || !latent_norm || !latent_up || !shared_h || !shared_down || !out)
     return fail(K3MOE_EINVAL, "a required pointer is NULL");
   LatArgs a{};
@@ -757,7 +808,23 @@ int k3moe_latent_out(const k3moe_latent_dims *dims, const float *expert_sum, con
   a.wb = reinterpret_cast<const uint16_t *>(shared_down);
   a.ya = reinterpret_cast<uint16_t *>(out);
   a.ws = reinterpret_cast<char *>(workspace);
-  return latent_launch(dims, 1, a, workspace_bytes, stream);
+  return latent_launch(dims, 1, a, workspace_bytes, room, stream);
+}
+
+int k3moe_latent_in(const k3moe_latent_dims *dims, const void *x, const void *latent_down, const void *shared_gate,
+                    const void *shared_up, void *latent, void *shared_h, void *workspace, size_t workspace_bytes,
+                    void *stream) {
+  g_err[0] = 0;
+  return latent_in_impl(dims, x, latent_down, shared_gate, shared_up, latent, shared_h, workspace, workspace_bytes, 0,
+                        stream);
+}
+
+int k3moe_latent_out(const k3moe_latent_dims *dims, const float *expert_sum, const void *latent_norm,
+                     const void *latent_up, const void *shared_h, const void *shared_down, void *out,
+                     void *workspace, size_t workspace_bytes, void *stream) {
+  g_err[0] = 0;
+  return latent_out_impl(dims, expert_sum, latent_norm, latent_up, shared_h, shared_down, out, workspace,
+                         workspace_bytes, 0, stream);
 }
 
 int k3moe_mxfp4_decode(const uint8_t *blocks, const uint8_t *scales, int64_t n_blocks, int32_t out_dtype,

@@ -552,6 +552,22 @@ __device__ __forceinline__ uint64_t wave_sort_desc(uint64_t v) {
   return v;
 }
 
+// The same for 32-bit values.
+template <int K, int J>
+__device__ __forceinline__ uint32_t bitonic_merge32(uint32_t v, int l) {
+  const uint32_t o = xor_lane<J>(v);
+  const bool keep_max = ((l & J) == 0) == ((l & K) == 0);
+  v = keep_max ? max(o, v) : min(o, v);
+  if constexpr (J > 1) v = bitonic_merge32<K, J / 2>(v, l);
+  return v;
+}
+template <int K = 2>
+__device__ __forceinline__ uint32_t wave_sort_desc32(uint32_t v) {
+  v = bitonic_merge32<K, K / 2>(v, __lane_id());
+  if constexpr (K < 64) v = wave_sort_desc32<K * 2>(v);
+  return v;
+}
+
 // Top 32 of two lists sorted descending in lanes 0..31 (a and b), sorted
 // descending in lanes 0..31: b reversed into lanes 32..63 makes a bitonic
 // sequence of 64, which one 6-stage merge sorts.

@@ -137,44 +137,101 @@ __global__ __launch_bounds__(kRWaves * 64, 1) void k_router(Plan pl, const uint1
   }
 }
 
-// Gating and top-k, one wave per token (kimi.py:308-316; distributed.py:174-176).
-__global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restrict__ bias,
-                                                    const int64_t *__restrict__ routes, char *ws,
-                                                    int64_t *__restrict__ out_ids, float *__restrict__ out_w,
-                                                    float *__restrict__ out_short) {
-  __shared__ float s_score[kWavesPerBlock][kMaxExperts];
-  __shared__ float s_key[kWavesPerBlock][kMaxExperts];
-  __shared__ uint32_t s_keyu[kWavesPerBlock][kMaxExperts];
-  __shared__ int s_sel[kWavesPerBlock][kMaxTopk];
-  const int wave = threadIdx.x / kWave, l = threadIdx.x % kWave;
-  const int t = blockIdx.x * kWavesPerBlock + wave;
-  if (t >= pl.B) return;
-  const float *part = reinterpret_cast<const float *>(ws + pl.o_logit);
-  const int E = pl.E, k = pl.k;
-  for (int e = l; e < E; e += kWave) {
-    float ps[kMaxRouterSplits];
+// Top-k of the wave's keys (lane l, register m: expert l + 64 m; 0 past E), 1 <= k <=
+// min(E, 32), larger keys first and equal ones by ascending expert: sel[0..k) in
+// rank order. The k-th largest of the lanes' maxima is at most the k-th largest
+// key (k distinct lanes hold a key as large), so the candidates, the keys from it
+// on, hold the top k: a few more than k of them when scores do not cluster. Up to
+// 64 are listed and sorted across the wave; more (many equal keys, or the best
+// experts in one residue class mod 64) take wave_topk on the keys in LDS.
+template <int MM>
+__device__ __forceinline__ void wave_topk_list(const uint32_t key[MM], const uint32_t *keys_lds, int E, int k,
+                                               uint64_t *list, int *sel) {
+  const int l = __lane_id();
+  uint32_t best = key[0];
 #pragma unroll
-    for (int s = 0; s < kMaxRouterSplits; ++s) ps[s] = s < pl.Sr ? part[((size_t)s * pl.B + t) * pl.Epad + e] : 0.f;
-    float logit = ps[0];
+  for (int m = 1; m < MM; ++m) best = max(best, key[m]);
+  const uint32_t threshold = lane_u32((uint32_t)wave_sort_desc32(best), k - 1);
+  int n = 0;
 #pragma unroll
-    for (int s = 1; s < kMaxRouterSplits; ++s)
-      if (s < pl.Sr) logit += ps[s];
-    float score, kv;
-    if (pl.gating == K3MOE_GATING_SIGMOID_BIAS) {
-      score = 1.0f / (1.0f + expf(-logit));
-      kv = bias ? __fadd_rn(score, bias[e]) : score;
-    } else {
-      score = logit;
-      kv = logit;
-    }
-    s_score[wave][e] = score;
-    s_key[wave][e] = kv;
-    s_keyu[wave][e] = ordered_key(kv);
+  for (int m = 0; m < MM; ++m) {
+    const bool in = l + 64 * m < E && key[m] >= threshold;
+    const uint64_t mask = __ballot(in);
+    const int at = n + __popcll(mask & ((1ull << l) - 1ull));
+    if (in && at < 64) list[at] = ((uint64_t)key[m] << 32) | (uint32_t)~(l + 64 * m);
+    n += __popcll(mask);
+  }
+  if (n > 64) {  // wave-uniform
+    wave_topk(keys_lds, E, k, sel);
+    return;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  wave_topk(s_keyu[wave], E, k, s_sel[wave]);
+  const uint64_t v = wave_sort_desc(l < n ? list[l] : 0ull);
+  if (l < k) sel[l] = (int)~(uint32_t)v;
+}
+
+// Gating and top-k, one wave per token (kimi.py:308-316; distributed.py:174-176), MM
+// experts per lane. The partial logits of four splits are loaded together: one
+// split after the other the loads' latency was most of the kernel (384 experts, 8
+// splits: 14.6 us; 896, with the selection by sorting every key: 36).
+template <int MM>
+__global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restrict__ bias,
+                                                    const int64_t *__restrict__ routes, char *ws,
+                                                    int64_t *__restrict__ out_ids, float *__restrict__ out_w,
+                                                    float *__restrict__ out_short) {
+  __shared__ float s_score[kWavesPerBlock][64 * MM];
+  __shared__ float s_key[kWavesPerBlock][64 * MM];
+  __shared__ uint32_t s_keyu[kWavesPerBlock][64 * MM];
+  __shared__ uint64_t s_list[kWavesPerBlock][64];
+  __shared__ int s_sel[kWavesPerBlock][kMaxTopk];
+  const int wave = threadIdx.x / kWave, l = threadIdx.x % kWave;
+  const int t = blockIdx.x * kWavesPerBlock + wave;
+  if (t >= pl.B) return;
+  const float *part = reinterpret_cast<const float *>(ws + pl.o_logit) + (size_t)t * pl.Epad;
+  const int E = pl.E, k = pl.k;
+  const size_t split = (size_t)pl.B * pl.Epad;
+  constexpr int kBatch = MM <= 8 ? 4 : 2;  // splits in flight
+  float logit[MM];
+  uint32_t keyu[MM];
+#pragma unroll
+  for (int m = 0; m < MM; ++m) logit[m] = l + 64 * m < E ? part[l + 64 * m] : 0.f;
+  for (int s0 = 1; s0 < pl.Sr; s0 += kBatch) {
+    float ps[kBatch][MM];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const float *src = part + (s0 + j < pl.Sr ? s0 + j : 0) * split;  // (past the last: an unused value)
+#pragma unroll
+      for (int m = 0; m < MM; ++m) ps[j][m] = l + 64 * m < E ? src[l + 64 * m] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (s0 + j >= pl.Sr) break;
+#pragma unroll
+      for (int m = 0; m < MM; ++m) logit[m] += ps[j][m];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < MM; ++m) {
+    const int e = l + 64 * m;
+    float score, kv;
+    if (pl.gating == K3MOE_GATING_SIGMOID_BIAS) {
+      score = 1.0f / (1.0f + expf(-logit[m]));
+      kv = bias && e < E ? __fadd_rn(score, bias[e]) : score;
+    } else {
+      score = logit[m];
+      kv = logit[m];
+    }
+    keyu[m] = e < E ? ordered_key(kv) : 0u;
+    s_score[wave][e] = score;
+    s_key[wave][e] = kv;
+    s_keyu[wave][e] = keyu[m];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  wave_topk_list<MM>(keyu, s_keyu[wave], E, k, s_list[wave], s_sel[wave]);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");

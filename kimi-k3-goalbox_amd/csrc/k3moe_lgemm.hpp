@@ -25,10 +25,15 @@
 // multiplied first and stored as bf16, and the same lanes add it to the routed
 // part when that is done.
 //
+//   k_lgemm<2>  the general path's router logits, x @ router.T as fp32 partials
+//               per k split, which the top-k kernel sums (kimi.py:308)
+//
 // Work is (row block, k split, token group); RW, TW and the number of splits
 // are chosen by lgemm_plan from the rounds of the grid and a step's cost. With
 // splits, fp32 partials go to the workspace and k_lreduce sums them in split
-// order: results do not depend on timing.
+// order: results do not depend on timing. The latent entry points' workspace is the
+// 64-token kernels' for every batch; inside the block the MoE step's, free before
+// and after it, takes the partials and the normalised rows.
 //
 // Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 26 + 7 us at 65
 // tokens (62 in two skinny launches), 109 at 777 (407), 213 at 2048 (988); <1> 24
@@ -46,21 +51,22 @@
 namespace k3moe {
 
 constexpr int kLgThreads = 512;
+constexpr int kLgCus = 256;  // the plans' compute units: tiles, splits and so the workspace do not depend on the device
 constexpr int kLgStepK = 64;
-constexpr int kLgMaxSplits = 8;
+constexpr int kLgMaxSplits = 8;         // (<2>: kMaxRouterSplits)
 constexpr long kLgMaxPartials = 64L << 20;  // bytes of fp32 partials, at most
 
 struct LgPlan {
   int B, h, lh, S, act, out;
   int RW, TW;    // MFMA tiles of a wave: 16 RW rows x 16 TW tokens
-  int N;         // weight rows: <0> lh + 2 S, <1> h
+  int N;         // weight rows: <0> lh + 2 S, <1> h, <2> the experts up to a whole tile (Plan::Epad)
   int NRB, NTG;  // row blocks, token groups
   int TG;        // tokens per group (a multiple of 16)
-  int splits;    // k splits of x (<0>) or en (<1>); 1: a workgroup does all of a tile and stores the outputs
-  int segs;      // k segments of a tile: <0> splits, <1> 1 + splits (the shared part first)
+  int splits;    // k splits of x (<0>, <2>) or en (<1>); 1: a workgroup does all of a tile and stores the outputs
+  int segs;      // k segments of a tile: <0>, <2> splits, <1> 1 + splits (the shared part first)
   int items;     // work items of the grid
   int G;
-  long o_en, o_part, total;
+  long o_en, o_part;
 };
 
 // Cycles of one 64-k step: the MFMAs, or the LDS traffic (8 (RW + TW) KiB read,
@@ -70,14 +76,12 @@ inline long lgemm_step_cost(int RW, int TW) {
   return (mfma > lds ? mfma : lds) + 60;
 }
 
-// Plan of k_lgemm<out>: the variant and split count of the least estimated time on
-// n_cus compute units (the launch's grid follows the device; the choice, and so the
-// workspace, does not).
-inline void lgemm_plan(const k3moe_latent_dims &d, int n_cus, int out, LgPlan &p) {
-  p.B = d.tokens; p.h = d.hidden; p.lh = d.latent; p.S = d.shared; p.act = d.activation; p.out = out;
+// The variant and split count of the least estimated time on n_cus compute units
+// (the launch's grid follows the device).
+inline void lgemm_choose(LgPlan &p, int n_cus, int max_splits, long max_part) {
   p.G = 1;
   while (p.G * 2 <= n_cus && p.G * 2 <= 1024) p.G *= 2;
-  p.N = out ? p.h : p.lh + 2 * p.S;
+  const bool out = p.out == 1;
   const int KS = (out ? p.lh : p.h) / kLgStepK, KS0 = out ? p.S / kLgStepK : 0;
   const int TT = cdiv(p.B, 16);
   const int rws[4] = {8, 5, 4, 2}, tws[3] = {4, 3, 2};
@@ -85,25 +89,58 @@ inline void lgemm_plan(const k3moe_latent_dims &d, int n_cus, int out, LgPlan &p
   long best = -1;
   for (int rw : rws)
     for (int tw : tws)
-      for (int s = 1; s <= kLgMaxSplits && s <= KS; ++s) {
+      for (int s = 1; s <= max_splits && s <= KS; ++s) {
         const int nrb = cdiv(p.N, 32 * rw), ntg = cdiv(TT, 2 * tw);
         const int segs = out ? 1 + s : s;
         const long items = (long)nrb * ntg * (s > 1 ? segs : 1);
-        if (s > 1 && (long)segs * p.B * p.N * 4 > kLgMaxPartials) break;
+        if (s > 1 && (long)segs * p.B * p.N * 4 > max_part) break;
         const long rounds = cdiv(cdiv(items, xcds), nslot);
         long t = rounds * ((s > 1 ? cdiv(KS, s) : KS + KS0) * lgemm_step_cost(rw, tw) + 2000);
-        if (s > 1) t += 12000 + (long)segs * p.B * p.N / 2000;  // the partials out and in, and a launch
+        if (s > 1 || p.out == 2) t += (long)segs * p.B * p.N / 2000;  // the partials out and in
+        if (s > 1 && p.out != 2) t += 12000;                          // and a launch
         if (best < 0 || t < best) {
           best = t;
           p.RW = rw; p.TW = tw; p.splits = s; p.segs = segs; p.NRB = nrb; p.NTG = ntg; p.items = (int)items;
           p.TG = cdiv(TT, ntg) * 16;
         }
       }
+}
+
+// Plan of k_lgemm<out> in `avail` bytes of workspace (at least the 64-token kernels',
+// whose area holds 64 normalised rows): the partials of its splits fit, and <1>
+// takes as many of the d.tokens rows at a time (p.B) as it can hold normalised, in
+// launches of equal size. avail follows from the dimensions alone, and so do the
+// splits and the order of the sums.
+inline void lgemm_plan(const k3moe_latent_dims &d, int n_cus, int out, long avail, LgPlan &p) {
+  p = LgPlan{};
+  p.B = d.tokens; p.h = d.hidden; p.lh = d.latent; p.S = d.shared; p.act = d.activation; p.out = out;
+  p.N = out ? p.h : p.lh + 2 * p.S;
   long o = kInitBytes;
-  auto take = [&](long bytes) { long at = o; o = (long)align256((size_t)(o + bytes)); return at; };
-  p.o_en = out ? take((long)p.B * p.lh * 2) : 0;
-  p.o_part = p.splits > 1 ? take((long)p.segs * p.B * p.N * 4) : 0;
-  p.total = o;
+  if (out) {
+    const long fit = (avail - o - 256) / (2L * p.lh) / 16 * 16;
+    const int launches = cdiv(p.B, fit);
+    p.B = cdiv(cdiv(p.B, launches), 16) * 16;
+    if (p.B > d.tokens) p.B = d.tokens;
+    p.o_en = o;
+    o = (long)align256((size_t)(o + (long)p.B * p.lh * 2));
+  }
+  p.o_part = o;
+  const long room = avail - o;
+  lgemm_choose(p, n_cus, kLgMaxSplits, room < kLgMaxPartials ? room : kLgMaxPartials);
+}
+
+// Plan of the router's k_lgemm<2> for a general-path step: B tokens of width h (a
+// multiple of 64) against E experts.
+inline void lgemm_router_plan(int B, int h, int E, int Epad, int n_cus, LgPlan &p) {
+  p = LgPlan{};
+  p.B = B; p.h = h; p.lh = E; p.N = Epad; p.out = 2;  // (lh: the weights' rows)
+  lgemm_choose(p, n_cus, kMaxRouterSplits, kLgMaxPartials);
+}
+
+inline int router_splits(int B, int h, int E, int Epad) {
+  LgPlan p;
+  lgemm_router_plan(B, h, E, Epad, kLgCus, p);
+  return p.splits;
 }
 
 template <int RW, int TW>
@@ -116,7 +153,8 @@ struct LgGeom {
 };
 
 // x: <0> x [B, h], <1> en [B, lh]; x2: <1> shared_h [B, S]; wa: latent_down / latent_up;
-// wb: shared_gate / shared_down; wc: shared_up; ya: latent / out; yb: shared_h.
+// wb: shared_gate / shared_down; wc: shared_up; ya: latent / out; yb: shared_h. <2>: x,
+// wa = router, part = the logits' partials [split][B][N].
 template <int OUT, int RW, int TW>
 __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16_t *__restrict__ x,
                                                         const uint16_t *__restrict__ x2,
@@ -133,7 +171,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
   const int xcds = gridDim.x < 8 ? (int)gridDim.x : 8;
   const int xcd = blockIdx.x % xcds, nslot = gridDim.x / xcds, slot = blockIdx.x / xcds;
   const int j0 = (int)((long)pl.items * xcd / xcds), j1 = (int)((long)pl.items * (xcd + 1) / xcds);
-  const int spi = pl.splits > 1 ? 1 : pl.segs;  // segments a workgroup runs one after the other per item
+  const int spi = OUT != 1 || pl.splits > 1 ? 1 : pl.segs;  // segments a workgroup runs one after the other per item
   const int nu = j1 - j0 > slot ? ((j1 - j0 - slot + nslot - 1) / nslot) * spi : 0;
   if (nu == 0) return;
 
@@ -153,12 +191,12 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
       U.seg = u % spi;
       U.rb = (int)v;
     }
-    const int KS = (OUT ? pl.lh : pl.h) / kLgStepK;
-    if (OUT && U.seg == 0) {
+    const int KS = (OUT == 1 ? pl.lh : pl.h) / kLgStepK;
+    if (OUT == 1 && U.seg == 0) {
       U.k0 = 0;
       U.k1 = pl.S / kLgStepK;
     } else {
-      const int s = OUT ? U.seg - 1 : U.seg;
+      const int s = OUT == 1 ? U.seg - 1 : U.seg;
       U.k0 = (int)((long)KS * s / pl.splits);
       U.k1 = (int)((long)KS * (s + 1) / pl.splits);
     }
@@ -174,13 +212,15 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
     };
     auto load_params = [&](const UnitP &U) {
       LoadP P;
-      const bool shared = OUT && U.seg == 0;
+      const bool shared = OUT == 1 && U.seg == 0;
 #pragma unroll
       for (int u = 0; u < RW; ++u) {
         const int r = 8 * (w + 4 * u) + (l >> 3);
         const int c = ((l & 7) ^ ((r >> 1) & 7)) * 8 + U.k0 * kLgStepK;
-        const int row = min(U.rb * 32 * RW + r, pl.N - 1);
-        if (OUT) {
+        const int row = min(U.rb * 32 * RW + r, (OUT == 2 ? pl.lh : pl.N) - 1);
+        if (OUT == 2) {
+          P.a[u] = wa + (size_t)row * pl.h + c;
+        } else if (OUT == 1) {
           P.a[u] = shared ? wb + (size_t)row * pl.S + c : wa + (size_t)row * pl.lh + c;
         } else {
           const int sr = row - pl.lh;  // pair tile sr / 16: 8 gate rows, then the same 8 up rows
@@ -193,7 +233,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
         const int r = 8 * (w + 4 * u) + (l >> 3);
         const int c = ((l & 7) ^ ((r >> 1) & 7)) * 8 + U.k0 * kLgStepK;
         const int t = min(U.tg * pl.TG + r, pl.B - 1);
-        P.b[u] = shared ? x2 + (size_t)t * pl.S + c : x + (size_t)t * (OUT ? pl.lh : pl.h) + c;
+        P.b[u] = shared ? x2 + (size_t)t * pl.S + c : x + (size_t)t * (OUT == 1 ? pl.lh : pl.h) + c;
       }
       return P;
     };
@@ -300,9 +340,9 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
         const int row = row0 + 16 * r;
         if (row >= pl.N) break;  // wave-uniform (N: whole tiles)
         const f32x4 c = acc[r][t];
-        if (pl.splits > 1) {
+        if (OUT == 2 || pl.splits > 1) {
           if (ok) *reinterpret_cast<f32x4 *>(part + ((size_t)U.seg * pl.B + tok) * pl.N + row + 4 * q) = c;
-        } else if constexpr (OUT) {
+        } else if constexpr (OUT == 1) {
           u32x2 *dst = reinterpret_cast<u32x2 *>(ya + (size_t)(ok ? tok : 0) * pl.h + row + 4 * q);
           if (U.seg == 0) {
             if (ok) *dst = pack_bf16x4(c[0], c[1], c[2], c[3]);

@@ -29,7 +29,7 @@ constexpr int kGroupChunk = 128;   // tokens per placement chunk in k_group
 constexpr int kXMinPairsPerExpert = 16;  // general path: token-expert pairs per expert from which units hold more than 32
 constexpr int kSMaxPairsPerExpert = 64;  // ... and from which the FP4-MFMA GEMMs take over
 constexpr int kSMinWidth = 512;  // general path: least K of the streaming grouped GEMMs (their loads run up to 4 k-steps ahead)
-constexpr int kMaxRouterSplits = 8;      // general path: router k-splits (partials summed by the top-k kernel)
+constexpr int kMaxRouterSplits = 16;     // general path: router k-splits (partials summed by the top-k kernel)
 
 constexpr int kDecWaves = 8;       // decode path: waves per workgroup
 constexpr int kDecThreads = kDecWaves * 64;
@@ -132,6 +132,7 @@ struct Plan {
   int trace;      // 1: the decode kernel records phase timestamps at o_trace
   int single;     // 1: the single-token kernel runs the step (k3moe_single.hpp)
   int redundant;  // 1: every workgroup routes every token (no barrier before grouping)
+  int rgemm;      // general path: router logits by k_lgemm<2> (k3moe_lgemm.hpp)
   int xgemm;      // general path: 1 = grouped-GEMM expert kernels, 0 = per-16-token streams
   int sgemm;      // general path: the streaming grouped GEMMs (k3moe_sgemm.hpp) and their pairs per unit; 0: not them
   int fgemm;      // grouped GEMMs on the scaled FP4 MFMA with two-term E4M3 activations (k3moe_fgemm.hpp)
@@ -313,6 +314,8 @@ inline bool lat_out_plan(Plan &p) {
   return ok;
 }
 
+inline int router_splits(int B, int h, int E, int Epad);  // of lgemm_router_plan (k3moe_lgemm.hpp)
+
 // n_cus: compute units of the device (the persistent grid size); trace: reserve
 // a timestamp area (kTraceSlots x 8 bytes per workgroup, up to 1024 groups).
 inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
@@ -382,12 +385,15 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   if (p.Srw < 1) p.Srw = 1;
   decode_lds(p);
 
-  // general path splits: router tiles of 64 tokens x 384 experts, at least 256 workgroups
-  // (at most 8 splits), gate/up about 2048 waves
+  // general path: the router's splits (rgemm, k3moe_lgemm.hpp: widths of whole
+  // 64-k steps; otherwise tiles of 64 tokens x 384 experts, at least 256
+  // workgroups, at most 8 splits), gate/up streams about 2048 waves
+  p.rgemm = p.h % 64 == 0;
   p.Sr = cdiv(256, (long)cdiv(p.B, 64) * cdiv(p.E, 384));
-  if (p.Sr > kMaxRouterSplits) p.Sr = kMaxRouterSplits;
+  if (p.Sr > 8) p.Sr = 8;
   if (p.Sr > p.KSr) p.Sr = p.KSr;
   if (p.Sr < 1) p.Sr = 1;
+  if (p.rgemm && p.path == kPathGeneral) p.Sr = router_splits(p.B, p.h, p.E, p.Epad);
   base = (long)p.Dmax * p.RTg;
   p.Sg = cdiv(2048, base);
   if (p.Sg > p.KSg) p.Sg = p.KSg;
