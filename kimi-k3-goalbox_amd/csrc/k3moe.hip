@@ -709,6 +709,7 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
   else if (p.E <= 256) topk(k_topk<4>);
   else if (p.E <= 384) topk(k_topk<6>);
   else if (p.E <= 512) topk(k_topk<8>);
+  else if (p.E <= 896) topk(k_topk<14>);
   else topk(k_topk<16>);
   if ((rc = launch_check("topk"))) return rc;
   const int nch = cdiv(p.B, kGroupChunk);

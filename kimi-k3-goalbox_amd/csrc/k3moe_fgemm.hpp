@@ -52,6 +52,7 @@
 
 #include "k3moe_device.hpp"
 #include "k3moe_plan.hpp"
+#include "k3moe_sgemm.hpp"
 
 namespace k3moe {
 
@@ -263,7 +264,7 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
   // then differ from the next tile's by a constant. Every load is issued (rows
   // without a token read the zero area), so that every k-step issues the same
   // number of them (and kFTiles more with a weight-scale chunk).
-  const uint32_t wlane = (uint32_t)i * KB * 16 + q * 16;                 // row i of a tile, block q
+  const uint32_t wlane = (uint32_t)(l >> 2) * KB * 16 + ((l & 3) ^ a_swizzle(l >> 2)) * 16;  // the lane's row of a tile and its block
   const size_t wtile = (size_t)16 * KB * 16;                             // tile stride
   const int sci = l >> 2, scp = 16 * (l & 3);
   // Scale rows that are not whole 16-byte words (KB % 16 == 8: a reduction
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(kFThreads, 1) void k_fgemm(Plan pl, MxAct a, const 
         uint32_t sa[kFTiles];
 #pragma unroll
         for (int r = 0; r < kFTiles; ++r) {
-          wa[r] = *reinterpret_cast<const u32x4 *>(base + kFOffW + (kFTiles * w + r) * 1024 + 16 * l);
+          wa[r] = *reinterpret_cast<const u32x4 *>(base + kFOffW + (kFTiles * w + r) * 1024 + (4 * i + (q ^ a_swizzle(i))) * 16);
           sa[r] = *reinterpret_cast<const uint8_t *>(scb + r * 1024);
         }
         // token tile t's B operands (both terms) and scales; the reads of tile

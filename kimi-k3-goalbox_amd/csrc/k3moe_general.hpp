@@ -173,9 +173,9 @@ __device__ __forceinline__ void wave_topk_list(const uint32_t key[MM], const uin
 }
 
 // Gating and top-k, one wave per token (kimi.py:308-316; distributed.py:174-176), MM
-// experts per lane. The partial logits of four splits are loaded together: one
-// split after the other the loads' latency was most of the kernel (384 experts, 8
-// splits: 14.6 us; 896, with the selection by sorting every key: 36).
+// experts per lane. The partial logits of several splits and the biases are loaded
+// together: one split after the other the loads' latency was most of the kernel
+// (384 experts, 8 splits: 14.6 us; 896, with the selection by sorting every key: 36).
 template <int MM>
 __global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restrict__ bias,
                                                     const int64_t *__restrict__ routes, char *ws,
@@ -192,11 +192,14 @@ __global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restr
   const float *part = reinterpret_cast<const float *>(ws + pl.o_logit) + (size_t)t * pl.Epad;
   const int E = pl.E, k = pl.k;
   const size_t split = (size_t)pl.B * pl.Epad;
-  constexpr int kBatch = MM <= 8 ? 4 : 2;  // splits in flight
-  float logit[MM];
+  constexpr int kBatch = MM <= 8 ? 8 : 4;  // splits in flight after the first
+  float logit[MM], bs[MM];
   uint32_t keyu[MM];
 #pragma unroll
-  for (int m = 0; m < MM; ++m) logit[m] = l + 64 * m < E ? part[l + 64 * m] : 0.f;
+  for (int m = 0; m < MM; ++m) {
+    logit[m] = l + 64 * m < E ? part[l + 64 * m] : 0.f;
+    bs[m] = bias && l + 64 * m < E ? bias[l + 64 * m] : 0.f;
+  }
   for (int s0 = 1; s0 < pl.Sr; s0 += kBatch) {
     float ps[kBatch][MM];
 #pragma unroll
@@ -218,7 +221,7 @@ __global__ __launch_bounds__(kThreads) void k_topk(Plan pl, const float *__restr
     float score, kv;
     if (pl.gating == K3MOE_GATING_SIGMOID_BIAS) {
       score = 1.0f / (1.0f + expf(-logit[m]));
-      kv = bias && e < E ? __fadd_rn(score, bias[e]) : score;
+      kv = bias ? __fadd_rn(score, bs[m]) : score;
     } else {
       score = logit[m];
       kv = logit[m];

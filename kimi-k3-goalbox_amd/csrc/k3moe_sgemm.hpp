@@ -18,8 +18,8 @@
 // their waits allow exactly the loads issued after the awaited step's.
 //
 // LDS slot: activation rows (SM x 256 bytes, the 16-byte chunk c of row r at
-// position c ^ (r & 15)), then the 16 weight tiles (lane (row i, block q) at
-// position 16 q + i, one MXFP4 block each). Only the 4-row blocks that hold
+// position c ^ s_swizzle(r)), then the 16 weight tiles (block q of row i at
+// position 4 i + (q ^ a_swizzle(i)), one MXFP4 block each). Only the 4-row blocks that hold
 // tokens are loaded; columns without a token multiply whatever the slot held
 // and are never stored (an MFMA's columns are independent). Weight scales:
 // rows of whole 16-byte words (KB % 16 == 0) go through two buffers in chunks
@@ -45,7 +45,8 @@
 
 namespace k3moe {
 
-constexpr int kSThreads = 512;
+constexpr int kSMfma = 8;                        // MFMA waves: 4 row groups x 2 halves of the token tiles
+constexpr int kSThreads = (kSMfma + 4) * 64;     // and 4 loaders
 
 // LDS layout of a variant: SM pairs per unit, Ring slots, ScSteps k-steps per weight-scale chunk.
 template <int SM, int Ring, int ScSteps>
@@ -74,6 +75,23 @@ __device__ __forceinline__ GroupEntry group_entry(const char *tab, int j) {
   const cint *src = reinterpret_cast<const cint *>(reinterpret_cast<uint64_t>(tab) + (uint64_t)(uint32_t)j * 16u);
   return GroupEntry{src[0], src[1], src[2]};
 }
+
+// Position of a 256-byte activation row's 16-byte chunk c: c ^ s_swizzle(row). A
+// b128 LDS read takes its lanes sixteen at a time (0-3, 12-15, 20-23, 24-27 and the
+// complements), four rows of one k quarter with four others' of the next: those
+// fall on distinct banks this way (with c ^ row they meet two by two).
+__device__ __forceinline__ int s_swizzle(int row) {
+  const int r = row & 15;
+  return r ^ ((((r >> 3) ^ (r >> 2)) & 1) << 2);
+}
+
+// A weight tile's 1 KiB in LDS: block q of row i at position 4 i + (q ^
+// a_swizzle(i)). A direct-to-LDS load puts lane L's 16 bytes at position L, so four
+// lanes in a row read a row's 64 contiguous bytes: with the A operand's lane order
+// (16 rows, then the next block) as the order of the load, every 16 lanes touch 16
+// lines, which the address unit takes at 16 bytes a cycle instead of over 60. The
+// swizzle keeps the operand's LDS reads, in that order, on distinct banks.
+__device__ __forceinline__ int a_swizzle(int row) { return (0 - (row >> 2)) & 3; }
 
 // Waits until at most n (wave-uniform, 0 .. 40) of this wave's loads are in flight.
 __device__ __forceinline__ void wait_vm_upto(int n) {
@@ -153,7 +171,7 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
     return UnitP{g.e, g.p0, g.m, (int)(v - jj * (unsigned)NB)};
   };
 
-  if (wv >= 4) {  // ------------------------------------------------ loader
+  if (wv >= kSMfma) {  // ------------------------------------------- loader
     const int *ptok = reinterpret_cast<const int *>(ws + pl.o_ptok);
     int *rows = reinterpret_cast<int *>(lds + Geo::off_row) + w * 2 * kRowWords;  // [2][kRowWords]
     // the token rows of unit U into buffer buf (lanes past its pairs repeat the last one's)
@@ -163,7 +181,7 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         load_lds<4>(ptok + U.p0 + min(64 * u + l, U.m - 1), reinterpret_cast<char *>(rows + buf * kRowWords + 64 * u));
     };
     struct LoadP {  // one unit's load addresses for this lane
-      const uint8_t *w[4], *s[4];  // weight tile rows (block q of row i), scale rows
+      const uint8_t *w[4], *s[4];  // weight tile rows (the lane's block of its row), scale rows
       const uint8_t *sn;           // scale row of the lane's row (tile q, row i), for rows of no whole words
       const uint16_t *x[kSRowLoads];
       int nx;                      // activation loads of this loader
@@ -174,7 +192,7 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
       for (int r = 0; r < 4; ++r) {
         const int orow = min(U.nb * RPB + (GU ? 32 * w + 16 * (r & 1) : 64 * w + 16 * r), Nout - 16);
         const size_t row = (size_t)U.e * Nout + orow;
-        P.w[r] = (GU && r >= 2 ? blk1 : blk0) + (row + i) * KB * 16 + q * 16;
+        P.w[r] = (GU && r >= 2 ? blk1 : blk0) + (row + (l >> 2)) * KB * 16 + ((l & 3) ^ a_swizzle(l >> 2)) * 16;
         P.s[r] = (GU && r >= 2 ? scl1 : scl0) + row * KB;
       }
       {
@@ -188,7 +206,7 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         P.nx += r0 < U.m ? 1 : 0;
         const int rc = min(r, U.m - 1);
         const size_t arow = GU ? (size_t)rows[buf * kRowWords + rc] : (size_t)(U.p0 + rc);
-        P.x[u] = act + arow * Kd + ((i ^ (r & 15)) * 8);
+        P.x[u] = act + arow * Kd + ((i ^ s_swizzle(r)) * 8);
       }
       return P;
     };
@@ -205,17 +223,18 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         n += 1;
       } else if (chunk_at(ks)) {
         // lane L: 16 bytes of one row's chunk (zero area past the row). ScSteps 16: row L / 4,
-        // one tile a load; 8: row L / 2 of 32, two tiles a load. The chunk replaces chunk
-        // c - 2, whose last step's reads are done at this step's issue.
+        // one tile a load; 8: row L / 2 of 32, two tiles a load; a row's words rotated by its
+        // number, so that 16 rows' bytes of one step lie in distinct banks. The chunk
+        // replaces chunk c - 2, whose last step's reads are done at this step's issue.
         const int c = ks == 0 ? 0 : (ks - kSAhead) / ScSteps + 1;
         char *const dst = lds + kSOffSc + ((cb0 + c) & 1) * kSScBuf + 4 * w * (64 * ScSteps);
         if constexpr (ScSteps == 16) {
-          const int at = 64 * c + 16 * (l & 3);
+          const int at = 64 * c + 16 * ((l & 3) ^ ((l >> 4) & 3));
 #pragma unroll
           for (int r = 0; r < 4; ++r) load_lds<16>(at < KB ? P.s[r] + (size_t)(l >> 2) * KB + at : zero, dst + r * 1024);
           n += 4;
         } else {
-          const int at = 32 * c + 16 * (l & 1);
+          const int at = 32 * c + 16 * ((l & 1) ^ ((l >> 4) & 1));
 #pragma unroll
           for (int r = 0; r < 4; r += 2) {
             const uint8_t *row = (l < 32 ? P.s[r] : P.s[r + 1]) + (size_t)((l >> 1) & 15) * KB;
@@ -279,61 +298,59 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
   }
 
   // ---------------------------------------------------------- MFMA wave
-  // A step is 2 NT items of 8 MFMAs, (half of the step's 128 k, token tile),
-  // tiles inside halves: a half's decoded weights are 32 registers, a whole
-  // step's would be 64. The B operands are read two items ahead (256 cycles of
-  // MFMAs cover the LDS latency) and the weights are decoded between the MFMAs
-  // of the half before, so that the matrix unit waits for neither. The barrier
-  // of the next step falls two items before the end of a step, when every read
-  // of the step's slot has been made; at a unit's end the next step is the next
-  // unit's first, read before the epilogue (after the last unit the same reads
-  // find stale slots and go unused: the loop keeps no branch).
+  // Wave w + 4 half takes the row group w's four tiles for the token tiles t = 2 j +
+  // half: two waves per SIMD, so that one's LDS reads and decodes run beside the
+  // other's MFMAs. A step is 2 NT items of 8 MFMAs, (half of the step's 128 k, token
+  // tile), tiles inside halves: a half's decoded weights are 32 registers, a whole
+  // step's would be 64. The B operands are read an item ahead and the weights
+  // decoded between the MFMAs of the half before. The barrier of the next step falls
+  // two items before the end of a step, when every read of the step's slot has been
+  // made; at a unit's end the next step is the next unit's first, read before the
+  // epilogue (after the last unit the same reads find stale slots and go unused: the
+  // loop keeps no branch).
+  const int half = wv >> 2;
   uint16_t *out = reinterpret_cast<uint16_t *>(ws + (GU ? pl.o_h : pl.o_y));
   u32x4 wa[4];         // a step's weights as stored, and their scale bytes
   uint32_t sa[4];
   bf16x8 av[4][2];     // the decoded half
-  u32x4 bb[4][2];      // B operands of item n of the running count in slot n & 3
+  u32x4 bb[2][2];      // B operands of item n in slot n & 1
   int g = 0;           // ring slot of the step read last
   // LDS offsets of this lane, as values the compiler keeps whole (it would
   // otherwise hoist one address per tile and spill them): everything else of an
   // address is wave-uniform or an immediate
-  int la = kSOffW + 4 * w * 1024 + 16 * l;
+  int la = kSOffW + 4 * w * 1024 + (4 * i + (q ^ a_swizzle(i))) * 16;
   int ls = wide ? kSOffSc + (4 * w * 16 + i) * (4 * ScSteps) + q : kSOffSc + w * 256 + i * 4 + q;
   const int tile_scales = wide ? 64 * ScSteps : 64;  // bytes from one tile's scales to the next's
-  int lb[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) lb[kk] = i * 256 + (((4 * q + kk) ^ i) * 16);
-  asm("" : "+v"(la), "+v"(ls), "+v"(lb[0]), "+v"(lb[1]), "+v"(lb[2]), "+v"(lb[3]));
+  const int lx = !wide ? 0 : ScSteps == 16 ? 16 * (i >> 2) : 16 * (i >> 3);  // the row's rotation
+  int lb = half * 4096 + i * 256 + (((4 * q) ^ s_swizzle(i)) * 16);  // chunk 4q; chunk 4q + kk: ^ 16 kk
+  asm("" : "+v"(la), "+v"(ls), "+v"(lb));
   auto read_a = [&](int sl, int c, int ks) {
     const char *base = lds + (sl * kSSlot + la);
 #pragma unroll
     for (int r = 0; r < 4; ++r) wa[r] = *reinterpret_cast<const u32x4 *>(base + r * 1024);
-    const int so = wide ? (c & 1) * kSScBuf + 4 * (ks % ScSteps) : sl * 1024;
+    const int so = wide ? (c & 1) * kSScBuf : sl * 1024, word = wide ? 4 * (ks % ScSteps) : 0;
+    const int at = (word ^ lx) + ls;  // (words of 16 bytes: the xor leaves the byte in the word)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sa[r] = *reinterpret_cast<const uint8_t *>(lds + (so + r * tile_scales + ls));
+    for (int r = 0; r < 4; ++r) sa[r] = *reinterpret_cast<const uint8_t *>(lds + (so + r * tile_scales + at));
   };
-  auto decode = [&](int r, int half) {
+  auto decode = [&](int r, int kh) {
     const float sc = e8m0_to_f32(sa[r]);
-    av[r][0] = fp4x8_to_bf16(wa[r][2 * half], sc);
-    av[r][1] = fp4x8_to_bf16(wa[r][2 * half + 1], sc);
+    av[r][0] = fp4x8_to_bf16(wa[r][2 * kh], sc);
+    av[r][1] = fp4x8_to_bf16(wa[r][2 * kh + 1], sc);
   };
-  auto read_b = [&](int sl, int half, int t, u32x4 (&b)[2]) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) b[k] = *reinterpret_cast<const u32x4 *>(lds + (sl * kSSlot + lb[2 * half + k]) + t * 4096);
-  };
-  // item 1 of a step: the second tile's first half, or the only tile's second half
-  auto read_b1 = [&](int sl, bool two, u32x4 (&b)[2]) {
+  // the wave's j-th token tile (2 j + half), k half kh
+  auto read_b = [&](int sl, int kh, int j, u32x4 (&b)[2]) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
-      b[k] = *reinterpret_cast<const u32x4 *>(lds + (sl * kSSlot + (two ? lb[k] + 4096 : lb[2 + k])));
+      b[k] = *reinterpret_cast<const u32x4 *>(lds + (sl * kSSlot + (lb ^ (16 * (2 * kh + k)))) + j * 8192);
   };
+  auto tiles_of = [&](const UnitP &U) { return (((U.m + 15) >> 4) + 1 - half) >> 1; };  // the wave's token tiles of a unit
 
   UnitP U = unit_at(0);
   int cb0 = 0;
   ring_barrier();
   read_a(0, 0, 0);
   read_b(0, 0, 0, bb[0]);
-  read_b1(0, U.m > 16, bb[1]);
 #pragma unroll
   for (int r = 0; r < 4; ++r) decode(r, 0);
   for (int u = 0; u < nu; ++u) {
@@ -347,23 +364,21 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      auto step = [&](auto sub, int ks) {
-        constexpr int S0 = decltype(sub)::value * N2;  // the step's first item in the running count (mod 4)
+      for (int ks = 0; ks < KS; ++ks) {
         const bool inner = ks + 1 < KS;
 #pragma unroll
         for (int n = 0; n < N2; ++n) {
-          const int half = n / NT, t = n % NT;
+          const int kh = n / NT, t = n % NT;
+          if (n + 1 < N2) read_b(g, (n + 1) / NT, (n + 1) % NT, bb[(n + 1) & 1]);
           if (n == N2 - 2) {
             ring_barrier();
             g = g + 1 == Ring ? 0 : g + 1;
           }
           if (n == (NT > 1 ? N2 - 2 : 1))
             read_a(g, inner ? cb0 + (ks + 1) / ScSteps : cb0 + NSC, inner ? ks + 1 : 0);
-          if (n + 2 < N2) read_b(g, (n + 2) / NT, (n + 2) % NT, bb[(S0 + n + 2) & 3]);
-          else if (n + 2 == N2) read_b(g, 0, 0, bb[(S0 + n + 2) & 3]);
-          else read_b1(g, inner ? NT > 1 : Un.m > 16, bb[(S0 + n + 2) & 3]);
+          if (n + 1 == N2) read_b(g, 0, 0, bb[0]);
           __builtin_amdgcn_sched_barrier(0);
-          u32x4(&b)[2] = bb[(S0 + n) & 3];
+          u32x4(&b)[2] = bb[n & 1];
           if (t + 1 < NT) {
 #pragma unroll
             for (int k = 0; k < 2; ++k)
@@ -377,27 +392,10 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
 #pragma unroll
                 for (int r = r0; r < r0 + 2; ++r) acc[r][t] = mfma16(av[r][k], as_bf16x8(b[k]), acc[r][t]);
 #pragma unroll
-              for (int r = r0; r < r0 + 2; ++r) decode(r, half ^ 1);
+              for (int r = r0; r < r0 + 2; ++r) decode(r, kh ^ 1);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
-        }
-      };
-      if constexpr (NT % 2 == 0) {
-        for (int ks = 0; ks < KS; ++ks) step(IntC<0>{}, ks);
-      } else {  // the running item count is even or odd twos by turns
-        int ks = 0;
-        for (; ks + 1 < KS; ks += 2) {
-          step(IntC<0>{}, ks);
-          step(IntC<1>{}, ks + 1);
-        }
-        if (ks < KS) {
-          step(IntC<0>{}, ks);
-#pragma unroll
-          for (int k = 0; k < 2; ++k) {  // the next unit's items count from 0
-            bb[0][k] = bb[2][k];
-            bb[1][k] = bb[3][k];
-          }
         }
       }
 
@@ -405,7 +403,7 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
       const int orow0 = U.nb * RPB + (GU ? 32 : 64) * w;  // first output row of the wave's tiles
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const int jrow = 16 * t + i;
+        const int jrow = 16 * (2 * t + half) + i;
         const bool ok = jrow < U.m;
         uint16_t *dst = out + (size_t)(U.p0 + (ok ? jrow : 0)) * Nout + orow0 + 16 * (q & 1) + 8 * (q >> 1);
         if constexpr (GU) {
@@ -430,13 +428,23 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         }
       }
     };
-    const int T = (U.m + 15) >> 4;
-    if (T == 1) run(IntC<1>{});
-    else if (SM == 32 || T == 2) run(IntC<2>{});
-    else if (T == 3) run(IntC<SM >= 48 ? 3 : 1>{});
-    else if (SM == 64 || T == 4) run(IntC<SM >= 64 ? 4 : 1>{});
-    else if (SM == 80 || T == 5) run(IntC<SM >= 80 ? 5 : 1>{});
-    else run(IntC<SM >= 96 ? 6 : 1>{});
+    const int nt = tiles_of(U);
+    if (nt == 0) {  // one tile, the other half's: the steps' barriers, then the next unit's first reads
+      for (int ks = 0; ks < KS; ++ks) {
+        ring_barrier();
+        g = g + 1 == Ring ? 0 : g + 1;
+      }
+      read_a(g, cb0 + NSC, 0);
+      read_b(g, 0, 0, bb[0]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) decode(r, 0);
+    } else if (SM == 32 || nt == 1) {
+      run(IntC<1>{});
+    } else if (SM == 64 || nt == 2) {
+      run(IntC<SM >= 64 ? 2 : 1>{});
+    } else {
+      run(IntC<SM >= 96 ? 3 : 1>{});
+    }
     U = Un;
     cb0 += NSC;
   }
