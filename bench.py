@@ -630,7 +630,7 @@ def roofline_entry(head, cfg, layers, measured, workload):
                 'achieved': head['hbm_GBps'], 'peak': 8000.0, 'unit': 'GB/s', 'frac': head['hbm_frac'],
                 'traffic': None}
     if workload == 'prefill':
-        return {'bound': 'mfma', 'kernel': 'k3moe::k_fgemm<gate/up> + k3moe::k_fgemm<down> (grouped GEMMs on '
+        return {'bound': 'mfma', 'kernel': 'k3moe::k_sgemm<gate/up, FP4> + k3moe::k_sgemm<down, FP4> (grouped GEMMs on '
                                            'v_mfma_scale_f32_16x16x128_f8f6f4: MXFP4 weights, two-term E4M3 '
                                            'activations) with the router, top-k, grouping, split and combine kernels',
                 'achieved': head['tflops'], 'peak': MFMA_USEFUL_TFLOPS, 'unit': 'TFLOP/s',

@@ -43,10 +43,9 @@ extern "C" {
  * otherwise; the other values force one (DECODE fails with K3MOE_EINVAL when
  * the shape does not fit it). All give the same expert sets. The multi-kernel
  * path (GENERAL) runs the expert projections as grouped GEMMs when
- * hidden/latent and inter are multiples of 128: streaming ones (bf16 MFMA on
- * the weights decoded in registers, units of 32 or 64 tokens of an expert; from
- * a latent of 512 on) while the experts average fewer than 64 tokens, then, when
- * latent is a multiple of 512 and inter of 256, GEMMs on the scaled FP4 MFMA
+ * hidden/latent and inter are multiples of 128 (latent from 512 on): on bf16
+ * MFMA with the weights decoded in registers, or, once the experts average 16
+ * tokens, latent a multiple of 512 and inter of 256, on the scaled FP4 MFMA
  * (MXFP4 weights as stored, activations as two E4M3 terms with E8M0 block
  * scales, which represent the bf16 values); other widths run as per-16-token
  * streams. GROUPED forces the FP4-MFMA GEMMs (on bf16 MFMA where the widths do

@@ -177,30 +177,24 @@ int allow_xgemm_lds() {
   return rc;
 }
 
-int allow_fgemm_lds() {
-  static int granted_gu = 0, granted_dn = 0;
-  int rc = grant_lds(reinterpret_cast<const void *>(&k_fgemm<true>), kFLds, granted_gu, "FP4 gate/up GEMM");
-  if (!rc) rc = grant_lds(reinterpret_cast<const void *>(&k_fgemm<false>), kFLds, granted_dn, "FP4 down GEMM");
-  return rc;
-}
-
 // The streaming grouped GEMMs' instantiations of a plan (pl.sgemm pairs per unit).
-typedef void (*StreamGemm)(Plan, const uint16_t *, const uint8_t *, const uint8_t *, const uint8_t *, const uint8_t *,
-                           char *);
+typedef void (*StreamGemm)(Plan, MxAct, const uint8_t *, const uint8_t *, const uint8_t *, const uint8_t *, char *);
 struct StreamGemms {
   StreamGemm gu, dn;
   int lds;
 };
-template <int SM, int Ring, int ScSteps>
+template <bool FP4, int SM, int Ring, int ScSteps>
 StreamGemms stream_gemms_of() {
-  return {k_sgemm<true, SM, Ring, ScSteps>, k_sgemm<false, SM, Ring, ScSteps>, SGeom<SM, Ring, ScSteps>::lds};
+  return {k_sgemm<true, FP4, SM, Ring, ScSteps>, k_sgemm<false, FP4, SM, Ring, ScSteps>,
+          SGeom<FP4, SM, Ring, ScSteps>::lds};
 }
 int stream_gemms(const Plan &p, StreamGemms &g) {
-  static int granted[2][2] = {{0, 0}, {0, 0}};
-  const int v = p.sgemm == 32 ? 0 : 1;
-  g = v == 0 ? stream_gemms_of<32, 5, 16>() : stream_gemms_of<64, 4, 8>();
-  int rc = grant_lds(reinterpret_cast<const void *>(g.gu), g.lds, granted[v][0], "streaming gate/up GEMM");
-  if (!rc) rc = grant_lds(reinterpret_cast<const void *>(g.dn), g.lds, granted[v][1], "streaming down GEMM");
+  static int granted[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  const int v = p.fgemm ? 2 : p.sgemm == 32 ? 0 : 1;
+  g = v == 0 ? stream_gemms_of<false, 32, 5, 16>() : v == 1 ? stream_gemms_of<false, 64, 4, 8>()
+                                                           : stream_gemms_of<true, 96, 3, 16>();
+  int rc = grant_lds(reinterpret_cast<const void *>(g.gu), g.lds, granted[v][0], "grouped gate/up GEMM");
+  if (!rc) rc = grant_lds(reinterpret_cast<const void *>(g.dn), g.lds, granted[v][1], "grouped down GEMM");
   return rc;
 }
 
@@ -446,7 +440,7 @@ int k3moe_workspace_layout(const k3moe_dims *dims, k3moe_layout *layout) {
   layout->pair_token = (int64_t)p.o_ptok;
   layout->pair_weight = (int64_t)p.o_pw;
   layout->pair_of = (int64_t)p.o_pof;
-  const bool split = p.fgemm && p.xgemm;
+  const bool split = p.fgemm;
   layout->pair_h = split ? -1 : (int64_t)p.o_h;
   layout->pair_y = (int64_t)p.o_y;
   layout->input_split = split ? (int64_t)p.o_xq : -1;
@@ -719,25 +713,31 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
   if ((rc = launch_check("group scan"))) return rc;
   hipLaunchKernelGGL(k_group_place, dim3(nch), dim3(256), 0, st, p, ws);
   if ((rc = launch_check("group place"))) return rc;
-  if (p.fgemm) {  // many tokens per expert: grouped GEMMs on the scaled FP4 MFMA
-    if ((rc = allow_fgemm_lds())) return rc;
-    uint8_t *xq = reinterpret_cast<uint8_t *>(ws + p.o_xq);
-    const long nxb = (long)p.B * (p.K / kBlockK);
-    MxAct ax{xq, xq + (size_t)p.B * p.K, xq + (size_t)2 * p.B * p.K, xq + (size_t)2 * p.B * p.K + nxb, p.K};
-    long qg = (nxb + 31) / 32;
-    if (qg > 8192) qg = 8192;
-    hipLaunchKernelGGL(k_quant, dim3((unsigned)qg), dim3(256), 0, st, xin, nxb, const_cast<uint8_t *>(ax.hi),
-                       const_cast<uint8_t *>(ax.lo), const_cast<uint8_t *>(ax.shi), const_cast<uint8_t *>(ax.slo));
-    if ((rc = launch_check("activation split"))) return rc;
-    hipLaunchKernelGGL(k_fgemm<true>, dim3(p.G), dim3(kFThreads), kFLds, st, p, ax, gate_blocks, gate_scales, up_blocks,
+  if (p.sgemm) {  // grouped GEMMs built around the weight stream
+    StreamGemms sg;
+    if ((rc = stream_gemms(p, sg))) return rc;
+    MxAct ax{reinterpret_cast<const uint8_t *>(xin), nullptr, nullptr, nullptr};
+    MxAct ah{reinterpret_cast<const uint8_t *>(ws + p.o_h), nullptr, nullptr, nullptr};
+    if (p.fgemm) {  // many tokens per expert: on the scaled FP4 MFMA
+      uint8_t *xq = reinterpret_cast<uint8_t *>(ws + p.o_xq);
+      const long nxb = (long)p.B * (p.K / kBlockK);
+      const size_t nx = (size_t)p.B * p.K;
+      long qg = (nxb + 31) / 32;
+      if (qg > 8192) qg = 8192;
+      hipLaunchKernelGGL(k_quant, dim3((unsigned)qg), dim3(256), 0, st, xin, nxb, xq, xq + nx, xq + 2 * nx,
+                         xq + 2 * nx + nxb);
+      if ((rc = launch_check("activation split"))) return rc;
+      ax = MxAct{xq, xq + nx, xq + 2 * nx, xq + 2 * nx + nxb};
+      const uint8_t *hq = reinterpret_cast<const uint8_t *>(ws + p.o_hq);
+      const size_t nh = (size_t)p.P * p.I;
+      ah = MxAct{hq, hq + nh, hq + 2 * nh, hq + 2 * nh + (size_t)p.P * (p.I / kBlockK)};
+    }
+    hipLaunchKernelGGL(sg.gu, dim3(p.G), dim3(kSThreads), sg.lds, st, p, ax, gate_blocks, gate_scales, up_blocks,
                        up_scales, ws);
-    if ((rc = launch_check("FP4 gate/up GEMM"))) return rc;
-    const uint8_t *hq = reinterpret_cast<const uint8_t *>(ws + p.o_hq);
-    const size_t nh = (size_t)p.P * p.I;
-    MxAct ah{hq, hq + nh, hq + 2 * nh, hq + 2 * nh + (size_t)p.P * (p.I / kBlockK), p.I};
-    hipLaunchKernelGGL(k_fgemm<false>, dim3(p.G), dim3(kFThreads), kFLds, st, p, ah, down_blocks, down_scales, nullptr,
-                       nullptr, ws);
-    if ((rc = launch_check("FP4 down GEMM"))) return rc;
+    if ((rc = launch_check("grouped gate/up GEMM"))) return rc;
+    hipLaunchKernelGGL(sg.dn, dim3(p.G), dim3(kSThreads), sg.lds, st, p, ah, down_blocks, down_scales, nullptr, nullptr,
+                       ws);
+    if ((rc = launch_check("grouped down GEMM"))) return rc;
   } else if (p.xgemm) {  // grouped GEMMs on bf16 MFMA, weights decoded in registers
     if ((rc = allow_xgemm_lds())) return rc;
     hipLaunchKernelGGL(k_xgemm<true>, dim3(p.G), dim3(kXThreads), kXLds, st, p, xin, gate_blocks, gate_scales,
@@ -746,15 +746,6 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
     hipLaunchKernelGGL(k_xgemm<false>, dim3(p.G), dim3(kXThreads), kXLds, st, p,
                        reinterpret_cast<const uint16_t *>(ws + p.o_h), down_blocks, down_scales, nullptr, nullptr, ws);
     if ((rc = launch_check("down GEMM"))) return rc;
-  } else if (p.sgemm) {  // few tokens per expert: grouped GEMMs built around the weight stream
-    StreamGemms sg;
-    if ((rc = stream_gemms(p, sg))) return rc;
-    hipLaunchKernelGGL(sg.gu, dim3(p.G), dim3(kSThreads), sg.lds, st, p, xin, gate_blocks, gate_scales, up_blocks,
-                       up_scales, ws);
-    if ((rc = launch_check("streaming gate/up GEMM"))) return rc;
-    hipLaunchKernelGGL(sg.dn, dim3(p.G), dim3(kSThreads), sg.lds, st, p,
-                       reinterpret_cast<const uint16_t *>(ws + p.o_h), down_blocks, down_scales, nullptr, nullptr, ws);
-    if ((rc = launch_check("streaming down GEMM"))) return rc;
   } else {
     const long ng = (long)p.Dmax * p.RTg * p.Sg;
     hipLaunchKernelGGL(k_gateup, dim3(cdiv(ng, kWavesPerBlock)), dim3(kThreads), 0, st, p, xin, gate_blocks,

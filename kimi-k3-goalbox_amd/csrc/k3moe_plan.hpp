@@ -27,7 +27,6 @@ constexpr int kMaxExperts = 1024;
 constexpr int kMaxTopk = 32;
 constexpr int kGroupChunk = 128;   // tokens per placement chunk in k_group
 constexpr int kXMinPairsPerExpert = 16;  // general path: token-expert pairs per expert from which units hold more than 32
-constexpr int kSMaxPairsPerExpert = 64;  // ... and from which the FP4-MFMA GEMMs take over
 constexpr int kSMinWidth = 512;  // general path: least K of the streaming grouped GEMMs (their loads run up to 4 k-steps ahead)
 constexpr int kMaxRouterSplits = 16;     // general path: router k-splits (partials summed by the top-k kernel)
 
@@ -133,9 +132,9 @@ struct Plan {
   int single;     // 1: the single-token kernel runs the step (k3moe_single.hpp)
   int redundant;  // 1: every workgroup routes every token (no barrier before grouping)
   int rgemm;      // general path: router logits by k_lgemm<2> (k3moe_lgemm.hpp)
-  int xgemm;      // general path: 1 = grouped-GEMM expert kernels, 0 = per-16-token streams
-  int sgemm;      // general path: the streaming grouped GEMMs (k3moe_sgemm.hpp) and their pairs per unit; 0: not them
-  int fgemm;      // grouped GEMMs on the scaled FP4 MFMA with two-term E4M3 activations (k3moe_fgemm.hpp)
+  int xgemm;      // general path: the grouped GEMMs of k3moe_xgemm.hpp (neither xgemm nor sgemm: per-16-token streams)
+  int sgemm;      // general path: the grouped GEMMs of k3moe_sgemm.hpp and their pairs per unit; 0: not them
+  int fgemm;      // ... on the scaled FP4 MFMA with two-term E4M3 activations (k3moe_fgemm.hpp)
   int lat_in;     // single-token or decode kernel: 1 = it also computes the latent block's inputs (latent, shared_h)
   int lat_S;      // ... the shared experts' width S
   int lat_out;    // single-token or decode kernel: 1 = it also computes the latent block's output (lat_in too)
@@ -359,27 +358,23 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
       p.B <= kDecMaxTokens && p.P <= kDecMaxPairs && (long)p.B * p.Epad * 8 <= part_room &&
       decode_lds(p) <= kDecMaxLds - kDecStaticLds)
     p.path = kPathDecode;
-  // general path expert kernels (widths allowing 128-k steps). By the pairs per
-  // expert n = P / E: the streaming GEMMs with 32 pairs per unit below
-  // kXMinPairsPerExpert and with 64 below kSMaxPairsPerExpert (or above it, where
-  // the widths do not fit the FP4-MFMA GEMMs), the FP4-MFMA GEMMs from there.
-  // Gate/up + down us on a TP8 rank's shard, 32 / 64 / FP4: n = 4: 149 + 82 /
-  // 154 + 89 / -, n = 15: 209 + 102 / 182 + 114 / -, n = 31: 271 + 156 / 262 +
-  // 158 / 262 + 231, n = 62: 386 + 248 / 329 + 239 / 314 + 303; unsharded experts,
-  // n = 85: - / 2700 + 1223 / 2678 + 1209. The Kimi rank, n = 14: 302 + 165 /
-  // 314 + 161, n = 27: 363 + 209 / 361 + 179.
+  // general path expert kernels (widths allowing 128-k steps): the grouped GEMMs of
+  // k3moe_sgemm.hpp, below kXMinPairsPerExpert pairs per expert (n = P / E) with 32
+  // pairs per unit, from there on the FP4 MFMA with 96 where the widths fit it (whole
+  // units of output rows, 512 of K and 256 of I), else with 64. Gate/up + down us on a
+  // TP8 rank's shard, 32 / 64 / FP4 96 (and the activation split): n = 4: 140 + 82 /
+  // 147 + 88 / 152 + 89 + 5, n = 15: 197 + 96 / 176 + 112 / 177 + 106 + 7, n = 31: 264 +
+  // 157 / 258 + 152 / 217 + 129 + 12, n = 62: 411 + 251 / 353 + 250 / 297 + 195 + 19. The
+  // unsharded experts, n = 85: 3508 + 1684 / 2741 + 1339 / 2260 + 1142 + 23; the Kimi rank,
+  // n = 14: 303 + 175 / 318 + 170, n = 27: 383 + 235 / 358 + 201. (FP4's fp32 sums are of
+  // truncated blocks: it is not taken where the exact ones were.)
   const bool widths = p.K % 128 == 0 && p.I % 128 == 0, fp4_widths = p.K % 512 == 0 && p.I % 256 == 0;
   const bool grouped = d.path == K3MOE_PATH_GROUPED || d.path == K3MOE_PATH_GROUPED_BF16;
   const bool many = (long)p.P >= (long)kXMinPairsPerExpert * p.E;
-  p.sgemm = 0;
-  if (!grouped && d.path != K3MOE_PATH_STREAMED && widths && p.K >= kSMinWidth) {
-    if (!many) p.sgemm = 32;
-    else if ((long)p.P < (long)kSMaxPairsPerExpert * p.E || !fp4_widths) p.sgemm = 64;
-  }
-  // the other grouped GEMMs, on the FP4 MFMA where the widths are whole units of
-  // output rows (256 of I for gate/up, 512 of K for down) and whole 128-k steps
-  p.xgemm = grouped || (d.path != K3MOE_PATH_STREAMED && widths && many && !p.sgemm);
-  p.fgemm = p.xgemm && d.path != K3MOE_PATH_GROUPED_BF16 && fp4_widths;
+  const bool gemms = grouped || (d.path != K3MOE_PATH_STREAMED && widths);
+  p.fgemm = gemms && (grouped || many) && d.path != K3MOE_PATH_GROUPED_BF16 && fp4_widths;
+  p.sgemm = p.fgemm ? 96 : gemms && !grouped && p.K >= kSMinWidth ? (many ? 64 : 32) : 0;
+  p.xgemm = !p.sgemm && gemms && (grouped || many);  // grouped GEMMs of k3moe_xgemm.hpp
   p.Srw = (int)(p.G / p.RTr);  // decode router units: (row tile, split), every token tile
   if (p.Srw > srw_cap) p.Srw = srw_cap;
   if (p.Srw < 1) p.Srw = 1;

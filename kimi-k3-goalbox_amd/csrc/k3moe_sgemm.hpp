@@ -1,46 +1,47 @@
-// Grouped expert GEMMs for batches past the decode kernel's (up to some 64
-// tokens per expert): gate/up and down projections of kimi.py:321-322, MXFP4
-// weights decoded in registers, bf16 MFMA with fp32 accumulation. The step is
-// bound by reading the experts' weights, so the kernel is built to keep that
-// stream going.
+// Grouped expert GEMMs of the general path (batches past the decode kernel's):
+// gate/up and down projections of kimi.py:321-322 as one GEMM per active expert, on
+// the bf16 MFMA with the MXFP4 weights decoded in registers, or (FP4) on the scaled
+// FP4 MFMA with the weights as stored and two-term activations (k3moe_fgemm.hpp).
 //
-// Unit = (group j, row block nb). A group is up to SM = 32 or 64 of one active
-// expert's token-expert pairs, an expert's groups of equal size (the group table
-// of k_group_scan); a row block is gate/up: 128 rows of I and the same up rows,
-// down: 256 rows of the hidden dimension. Eight waves, two per SIMD: waves 4-7
-// issue loads and nothing else, waves 0-3 decode and multiply. Loader 4 + w
-// feeds MFMA wave w's four 16-row weight tiles (gate/up: gate rows 32w + 16r,
-// r < 2, and the same up rows, so the activation is applied in registers; down:
-// rows 64w + 16r). Operands move one 128-k step at a time through Ring LDS
-// slots filled by direct-to-LDS loads Ring - 1 steps ahead, one barrier per
-// step: at SM = 32, 64 KiB of weights in flight per CU. The loaders run over
-// unit boundaries, so the stream goes on through the MFMA waves' epilogues;
-// their waits allow exactly the loads issued after the awaited step's.
+// Unit = (group j, row block nb). A group is up to SM = 32, 64 or 96 of one active
+// expert's token-expert pairs, an expert's groups of equal size (the group table of
+// k_group_scan); a row block is gate/up: 128 rows of I and the same up rows, down:
+// 256 rows of the hidden dimension. Twelve waves, three per SIMD: waves 8-11 issue
+// loads and nothing else, waves 0-7 multiply. Loader 8 + w feeds row group w's four
+// 16-row weight tiles (gate/up: gate rows 32w + 16r, r < 2, and the same up rows, so
+// the activation is applied in registers; down: rows 64w + 16r). Operands move one
+// 128-k step at a time through Ring LDS slots filled by direct-to-LDS loads Ring - 1
+// steps ahead, one barrier per step: at SM = 32, 64 KiB of weights in flight per CU.
+// The loaders run over unit boundaries, so the stream goes on through the MFMA
+// waves' epilogues; their waits allow exactly the loads issued after the awaited
+// step's.
 //
-// LDS slot: activation rows (SM x 256 bytes, the 16-byte chunk c of row r at
-// position c ^ s_swizzle(r)), then the 16 weight tiles (block q of row i at
-// position 4 i + (q ^ a_swizzle(i)), one MXFP4 block each). Only the 4-row blocks that hold
-// tokens are loaded; columns without a token multiply whatever the slot held
-// and are never stored (an MFMA's columns are independent). Weight scales:
-// rows of whole 16-byte words (KB % 16 == 0) go through two buffers in chunks
-// of ScSteps steps (4 ScSteps bytes of a row at a time), other rows 4 bytes per
-// step.
+// LDS slot: the activation rows (bf16: SM x 256 bytes, the 16-byte chunk c of row r at
+// position c ^ s_swizzle(r); FP4: the hi rows, then the lo rows, SM x 128 bytes each,
+// chunk c at c ^ ((r >> 1) & 7), then their scale dwords), then the 16 weight tiles
+// (block q of row i at position 4 i + (q ^ a_swizzle(i)), one MXFP4 block each). Only
+// the row blocks that hold tokens are loaded; columns without a token multiply
+// whatever the slot held and are never stored (an MFMA's columns are independent).
+// Weight scales: rows of whole 16-byte words (KB % 16 == 0) go through two buffers in
+// chunks of ScSteps steps (4 ScSteps bytes of a row at a time: read 4 bytes per step,
+// each line was fetched about ten times), other rows 4 bytes per step.
 //
-// Schedule: a persistent grid; XCD x takes the groups [J x / 8, J (x + 1) / 8)
-// and its workgroups the XCD's units in turn, so that the row blocks of a
-// group, and an expert's groups, run on one XCD at about the same time.
+// Schedule: a persistent grid; XCD x takes the groups [J x / 8, J (x + 1) / 8) and its
+// workgroups the XCD's units in turn, so that the row blocks of a group, and an
+// expert's groups, run on one XCD at about the same time.
 //
-// Measured on a TP8 rank's shard (384 experts, K 7168, I 256) at 203 tokens:
-// gate/up 149 us, 740 MB of weights at 5.0 TB/s, down 82 us, 370 MB at 4.5 TB/s;
-// the per-16-token streams it replaced took 286 and 100 us there, 620 and 154
-// (now 209 and 102) at 700 tokens. Timing builds at 203 tokens: without the
-// MFMAs 146 us, with every weight read from cache 105 us: HBM bounds it. At
-// SM = 64 the weights of an expert's second group come from memory again
-// (fetched bytes 2.0 x the weights at 85 tokens per expert), which bounds the
-// unsharded experts there.
+// Measured (gate/up + down us; per-16-token streams and the former FP4 GEMMs, whose
+// loads ran two steps ahead of four MFMA waves, in brackets): a TP8 rank's shard at 203
+// tokens 140 + 84 (286 + 100), at 700 197 + 96 (620 + 154), at 2999 297 + 195 (314 + 303);
+// the unsharded experts at 4096 2260 + 1142 (2678 + 1209), at 700 1290 + 644 (3658 +
+// 1489); the Kimi rank at 777 303 + 172 (754 + 245). At 203 tokens HBM bounds it (740
+// MB of gate/up weights at 5.3 TB/s). At 85 tokens per expert timing builds of the
+// bf16 form took 1604 us with neither loads nor decode (the matrix cores' rate of a
+// large library product), 1951 without the loads, 1777 without the MFMAs.
 #pragma once
 
 #include "k3moe_device.hpp"
+#include "k3moe_fgemm.hpp"
 #include "k3moe_plan.hpp"
 
 namespace k3moe {
@@ -48,18 +49,21 @@ namespace k3moe {
 constexpr int kSMfma = 8;                        // MFMA waves: 4 row groups x 2 halves of the token tiles
 constexpr int kSThreads = (kSMfma + 4) * 64;     // and 4 loaders
 
-// LDS layout of a variant: SM pairs per unit, Ring slots, ScSteps k-steps per weight-scale chunk.
-template <int SM, int Ring, int ScSteps>
+// LDS layout of a variant: operand form, SM pairs per unit, Ring slots, ScSteps k-steps per weight-scale chunk.
+template <bool FP4, int SM, int Ring, int ScSteps>
 struct SGeom {
   static constexpr int ahead = Ring - 1;          // k-steps of loads in flight ahead of the current one
-  static constexpr int off_w = SM * 256;          // weight tiles of a slot
+  static constexpr int off_xs = SM * 256;         // FP4: the rows' scale dwords, hi then lo
+  static constexpr int off_w = off_xs + (FP4 ? 1024 : 0);  // weight tiles of a slot
   static constexpr int slot = off_w + 16 * 1024;
   static constexpr int sc_buf = 256 * 4 * ScSteps;   // one chunk of the unit's 256 weight rows
   static constexpr int off_sc = Ring * slot;         // two chunk buffers, or Ring pieces of 1 KiB
   static constexpr int row_words = SM > 64 ? 128 : 64;
   static constexpr int off_row = off_sc + 2 * sc_buf;  // gate/up: each loader's token rows, two units
   static constexpr int lds = off_row + 4 * 2 * row_words * 4;
-  static constexpr int row_loads = SM / 16;  // a loader's activation loads per step, at most (4 rows each)
+  static constexpr int row_loads = FP4 ? SM / 32 : SM / 16;  // a loader's blocks of activation rows (FP4: 8 rows of each term; 4 rows)
+  static_assert(!FP4 || SM % 32 == 0);
+  static_assert(!FP4 || SM <= 128, "the scale dwords' KiB");
   static_assert(SM % 16 == 0 && SM <= 128 && (ScSteps == 16 || ScSteps == 8));
   static_assert(Ring * 1024 <= 2 * sc_buf, "the per-step scale pieces fit the chunk buffers");
   static_assert(lds <= kDecMaxLds);
@@ -125,15 +129,16 @@ __device__ __forceinline__ u32x2 pack_bf16x4(float a, float b, float c, float d)
                (uint32_t)f32_to_bf16_bits(c) | ((uint32_t)f32_to_bf16_bits(d) << 16)};
 }
 
-// GU: gate/up of the gathered rows of act [B, K] -> h (pl.act applied);
-// otherwise down of the pair rows of act = h [P, I] -> y.
-template <bool GU, int SM, int Ring, int ScSteps>
-__global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t *__restrict__ act,
+// GU: gate/up of the gathered rows of act [B, K] -> h (pl.act applied); otherwise
+// down of the pair rows of act = h [P, I] -> y. FP4: activations and h as two E4M3
+// terms, otherwise bf16.
+template <bool GU, bool FP4, int SM, int Ring, int ScSteps>
+__global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, MxAct act,
                                                        const uint8_t *__restrict__ blk0,
                                                        const uint8_t *__restrict__ scl0,
                                                        const uint8_t *__restrict__ blk1,
                                                        const uint8_t *__restrict__ scl1, char *ws) {
-  typedef SGeom<SM, Ring, ScSteps> Geo;
+  typedef SGeom<FP4, SM, Ring, ScSteps> Geo;
   constexpr int kSAhead = Geo::ahead, kSSlot = Geo::slot, kSOffW = Geo::off_w, kSOffSc = Geo::off_sc,
                 kSScBuf = Geo::sc_buf, kSRowLoads = Geo::row_loads, kRowWords = Geo::row_words;
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -183,8 +188,9 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
     struct LoadP {  // one unit's load addresses for this lane
       const uint8_t *w[4], *s[4];  // weight tile rows (the lane's block of its row), scale rows
       const uint8_t *sn;           // scale row of the lane's row (tile q, row i), for rows of no whole words
-      const uint16_t *x[kSRowLoads];
-      int nx;                      // activation loads of this loader
+      const uint8_t *x[kSRowLoads];  // bf16 rows; FP4: the hi rows
+      const uint8_t *xs;             // FP4: the lane's row of scales
+      int nx;                        // blocks of activation rows of this loader that hold tokens
     };
     auto load_params = [&](const UnitP &U, int buf) {
       LoadP P;
@@ -202,11 +208,18 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
       P.nx = 0;
 #pragma unroll
       for (int u = 0; u < kSRowLoads; ++u) {
-        const int r0 = 4 * (w + 4 * u), r = r0 + q;
+        const int r0 = (FP4 ? 8 : 4) * (w + 4 * u), r = r0 + (FP4 ? l >> 3 : q);
         P.nx += r0 < U.m ? 1 : 0;
         const int rc = min(r, U.m - 1);
         const size_t arow = GU ? (size_t)rows[buf * kRowWords + rc] : (size_t)(U.p0 + rc);
-        P.x[u] = act + arow * Kd + ((i ^ s_swizzle(r)) * 8);
+        if constexpr (FP4) P.x[u] = act.hi + arow * Kd + ((l & 7) ^ ((r >> 1) & 7)) * 16;
+        else P.x[u] = act.hi + (arow * Kd + (i ^ s_swizzle(r)) * 8) * 2;
+      }
+      if constexpr (FP4) {  // loader w: the scale dwords 64 w + L, the rows' hi ones, then their lo ones
+        const int d = 64 * w + l, r = d < SM ? d : d - SM;
+        const int rc = min(min(r, SM - 1), U.m - 1);
+        const size_t arow = GU ? (size_t)rows[buf * kRowWords + rc] : (size_t)(U.p0 + rc);
+        P.xs = (d < SM ? act.shi : act.slo) + arow * KB;
       }
       return P;
     };
@@ -217,7 +230,13 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
     // Returns their number.
     auto issue = [&](const LoadP &P, int ks, int sl, int cb0) -> int {
       char *base = lds + sl * kSSlot;
-      int n = 4 + P.nx;
+      int n = 4 + (FP4 ? 2 : 1) * P.nx;
+      if constexpr (FP4) {
+        if (64 * w < 2 * SM) {  // wave-uniform
+          load_lds<4>(P.xs + 4 * ks, base + Geo::off_xs + w * 256);
+          n += 1;
+        }
+      }
       if (!wide) {  // lane L: step ks's 4 scale bytes of row L of the 64
         load_lds<4>(P.sn + 4 * ks, lds + kSOffSc + sl * 1024 + w * 256);
         n += 1;
@@ -247,7 +266,14 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
       for (int r = 0; r < 4; ++r) load_lds<16>(P.w[r] + ks * 64, base + kSOffW + (4 * w + r) * 1024);
 #pragma unroll
       for (int u = 0; u < kSRowLoads; ++u)
-        if (u < P.nx) load_lds<16>(P.x[u] + ks * 128, base + 4 * (w + 4 * u) * 256);
+        if (u < P.nx) {
+          if constexpr (FP4) {
+            load_lds<16>(P.x[u] + ks * 128, base + 8 * (w + 4 * u) * 128);
+            load_lds<16>(P.x[u] + (act.lo - act.hi) + ks * 128, base + SM * 128 + 8 * (w + 4 * u) * 128);
+          } else {
+            load_lds<16>(P.x[u] + ks * 256, base + 4 * (w + 4 * u) * 256);
+          }
+        }
       return n;
     };
     // the stream: step iks of unit iu is the next to go out
@@ -312,8 +338,11 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
   uint16_t *out = reinterpret_cast<uint16_t *>(ws + (GU ? pl.o_h : pl.o_y));
   u32x4 wa[4];         // a step's weights as stored, and their scale bytes
   uint32_t sa[4];
-  bf16x8 av[4][2];     // the decoded half
+  u32x4 wn[4];         // FP4: the next step's
+  uint32_t sn[4];
+  bf16x8 av[4][2];     // bf16: the decoded half
   u32x4 bb[2][2];      // B operands of item n in slot n & 1
+  uint32_t sb[2];      // FP4: and their scale bytes
   int g = 0;           // ring slot of the step read last
   // LDS offsets of this lane, as values the compiler keeps whole (it would
   // otherwise hoist one address per tile and spill them): everything else of an
@@ -322,9 +351,11 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
   int ls = wide ? kSOffSc + (4 * w * 16 + i) * (4 * ScSteps) + q : kSOffSc + w * 256 + i * 4 + q;
   const int tile_scales = wide ? 64 * ScSteps : 64;  // bytes from one tile's scales to the next's
   const int lx = !wide ? 0 : ScSteps == 16 ? 16 * (i >> 2) : 16 * (i >> 3);  // the row's rotation
-  int lb = half * 4096 + i * 256 + (((4 * q) ^ s_swizzle(i)) * 16);  // chunk 4q; chunk 4q + kk: ^ 16 kk
+  // bf16: chunk 4q of the row (chunk 4q + kk: ^ 16 kk); FP4: chunk q (chunk 4 + q: ^ 64)
+  int lb = FP4 ? half * 2048 + i * 128 + ((q ^ ((i >> 1) & 7)) * 16)
+               : half * 4096 + i * 256 + (((4 * q) ^ s_swizzle(i)) * 16);
   asm("" : "+v"(la), "+v"(ls), "+v"(lb));
-  auto read_a = [&](int sl, int c, int ks) {
+  auto read_a = [&](int sl, int c, int ks, u32x4 (&wa)[4], uint32_t (&sa)[4]) {
     const char *base = lds + (sl * kSSlot + la);
 #pragma unroll
     for (int r = 0; r < 4; ++r) wa[r] = *reinterpret_cast<const u32x4 *>(base + r * 1024);
@@ -338,21 +369,32 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
     av[r][0] = fp4x8_to_bf16(wa[r][2 * kh], sc);
     av[r][1] = fp4x8_to_bf16(wa[r][2 * kh + 1], sc);
   };
-  // the wave's j-th token tile (2 j + half), k half kh
-  auto read_b = [&](int sl, int kh, int j, u32x4 (&b)[2]) {
+  // Item n of a step over NT tiles: bf16 (k half, tile), FP4 (tile, term). Operands of
+  // the wave's j-th token tile (2 j + half), k half or term h.
+  auto read_b = [&](int sl, int h, int j, int n) {
+    u32x4(&b)[2] = bb[n & 1];
+    if constexpr (FP4) {
+      const int base = sl * kSSlot + h * SM * 128 + j * 4096;
+      b[0] = *reinterpret_cast<const u32x4 *>(lds + (base + lb));
+      b[1] = *reinterpret_cast<const u32x4 *>(lds + (base + (lb ^ 64)));
+      sb[n & 1] = *reinterpret_cast<const uint8_t *>(lds + (sl * kSSlot + Geo::off_xs + h * SM * 4 + (2 * j + half) * 64) + (4 * i + q));
+    } else {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
-      b[k] = *reinterpret_cast<const u32x4 *>(lds + (sl * kSSlot + (lb ^ (16 * (2 * kh + k)))) + j * 8192);
+      for (int k = 0; k < 2; ++k)
+        b[k] = *reinterpret_cast<const u32x4 *>(lds + (sl * kSSlot + (lb ^ (16 * (2 * h + k)))) + j * 8192);
+    }
   };
   auto tiles_of = [&](const UnitP &U) { return (((U.m + 15) >> 4) + 1 - half) >> 1; };  // the wave's token tiles of a unit
 
   UnitP U = unit_at(0);
   int cb0 = 0;
   ring_barrier();
-  read_a(0, 0, 0);
-  read_b(0, 0, 0, bb[0]);
+  read_a(0, 0, 0, wa, sa);
+  read_b(0, 0, 0, 0);
+  if constexpr (!FP4) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) decode(r, 0);
+    for (int r = 0; r < 4; ++r) decode(r, 0);
+  }
   for (int u = 0; u < nu; ++u) {
     const bool last = u + 1 == nu;
     const UnitP Un = unit_at(last ? u : u + 1);
@@ -368,18 +410,26 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         const bool inner = ks + 1 < KS;
 #pragma unroll
         for (int n = 0; n < N2; ++n) {
-          const int kh = n / NT, t = n % NT;
-          if (n + 1 < N2) read_b(g, (n + 1) / NT, (n + 1) % NT, bb[(n + 1) & 1]);
+          const int h = FP4 ? n & 1 : n / NT, t = FP4 ? n >> 1 : n % NT;  // term, or k half
+          if (n + 1 < N2) read_b(g, FP4 ? (n + 1) & 1 : (n + 1) / NT, FP4 ? (n + 1) >> 1 : (n + 1) % NT, n + 1);
           if (n == N2 - 2) {
             ring_barrier();
             g = g + 1 == Ring ? 0 : g + 1;
           }
-          if (n == (NT > 1 ? N2 - 2 : 1))
-            read_a(g, inner ? cb0 + (ks + 1) / ScSteps : cb0 + NSC, inner ? ks + 1 : 0);
-          if (n + 1 == N2) read_b(g, 0, 0, bb[0]);
+          if (n == (NT > 1 || FP4 ? N2 - 2 : 1)) {
+            const int c = inner ? cb0 + (ks + 1) / ScSteps : cb0 + NSC, k1 = inner ? ks + 1 : 0;
+            if constexpr (FP4) read_a(g, c, k1, wn, sn);
+            else read_a(g, c, k1, wa, sa);
+          }
+          if (n + 1 == N2) read_b(g, 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
           u32x4(&b)[2] = bb[n & 1];
-          if (t + 1 < NT) {
+          if constexpr (FP4) {
+            const i32x8 b8 = {(int)b[0][0], (int)b[0][1], (int)b[0][2], (int)b[0][3],
+                              (int)b[1][0], (int)b[1][1], (int)b[1][2], (int)b[1][3]};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r][t] = mfma_fp4x8(wa[r], b8, sa[r], sb[n & 1], acc[r][t]);
+          } else if (t + 1 < NT) {
 #pragma unroll
             for (int k = 0; k < 2; ++k)
 #pragma unroll
@@ -392,10 +442,17 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
 #pragma unroll
                 for (int r = r0; r < r0 + 2; ++r) acc[r][t] = mfma16(av[r][k], as_bf16x8(b[k]), acc[r][t]);
 #pragma unroll
-              for (int r = r0; r < r0 + 2; ++r) decode(r, kh ^ 1);
+              for (int r = r0; r < r0 + 2; ++r) decode(r, h ^ 1);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (FP4) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            wa[r] = wn[r];
+            sa[r] = sn[r];
+          }
         }
       }
 
@@ -406,7 +463,32 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         const int jrow = 16 * (2 * t + half) + i;
         const bool ok = jrow < U.m;
         uint16_t *dst = out + (size_t)(U.p0 + (ok ? jrow : 0)) * Nout + orow0 + 16 * (q & 1) + 8 * (q >> 1);
-        if constexpr (GU) {
+        if constexpr (GU && FP4) {
+          // one 32-column block of I per token: gate tiles 0, 1 with up tiles 2, 3
+          float h[2][4];
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              h[s2][v] = round_bf16(fast_act(pl.act, round_bf16(acc[s2][t][v]), round_bf16(acc[2 + s2][t][v])));
+          uint32_t hw[2], lw[2], sh, sl;
+          mx8_split8(h, hw, lw, sh, sl);
+          // eight consecutive columns per lane: of tile q & 1, from 8 (q / 2)
+          const auto hs = __builtin_amdgcn_permlane16_swap(hw[0], hw[1], false, false);
+          const auto ls2 = __builtin_amdgcn_permlane16_swap(lw[0], lw[1], false, false);
+          if (ok) {
+            const size_t p = (size_t)(U.p0 + jrow), nh = (size_t)pl.P * pl.I;
+            uint8_t *const hq = reinterpret_cast<uint8_t *>(ws + pl.o_hq);
+            uint8_t *const dh = hq + p * pl.I + orow0 + 16 * (q & 1) + 8 * (q >> 1);
+            *reinterpret_cast<u32x2 *>(dh) = u32x2{hs[0], hs[1]};
+            *reinterpret_cast<u32x2 *>(dh + nh) = u32x2{ls2[0], ls2[1]};
+            if (q == 0) {
+              uint8_t *const ds = hq + 2 * nh + p * (pl.I / kBlockK) + orow0 / kBlockK;
+              ds[0] = (uint8_t)sh;
+              ds[(size_t)pl.P * (pl.I / kBlockK)] = (uint8_t)sl;
+            }
+          }
+        } else if constexpr (GU) {
           u32x2 hp[2];
 #pragma unroll
           for (int s2 = 0; s2 < 2; ++s2) {
@@ -434,10 +516,12 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, const uint16_t 
         ring_barrier();
         g = g + 1 == Ring ? 0 : g + 1;
       }
-      read_a(g, cb0 + NSC, 0);
-      read_b(g, 0, 0, bb[0]);
+      read_a(g, cb0 + NSC, 0, wa, sa);
+      read_b(g, 0, 0, 0);
+      if constexpr (!FP4) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) decode(r, 0);
+        for (int r = 0; r < 4; ++r) decode(r, 0);
+      }
     } else if (SM == 32 || nt == 1) {
       run(IntC<1>{});
     } else if (SM == 64 || nt == 2) {

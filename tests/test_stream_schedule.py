@@ -1,6 +1,8 @@
-"""CPU checks of two kernels' load schedules (restated here from their sources).
+"""CPU checks of kernels' load schedules (restated here from their sources).
 
-k_fgemm (csrc/k3moe_fgemm.hpp): units stream back to back; a loader issues the
+k_sgemm (csrc/k3moe_sgemm.hpp), its loader stream: test_sgemm_*, and, for the
+two steps ahead of the FP4 form with a fixed number of loads per step,
+test_fgemm_stream_schedule: units stream back to back; a loader issues the
 step two ahead at every barrier (the next unit's first two steps during the
 last two of the current one), waits before the barrier of step g until only
 the loads of step g + 1 may be outstanding, and puts weight-scale chunk c of a
@@ -61,38 +63,88 @@ def test_fgemm_stream_schedule(KS, nunits):
     fgemm_stream(KS, nunits)
 
 
-def fgemm_scale_reads(KB, rows, steps_per_chunk=16):
-    """(row, first byte, bytes) of every weight-scale load of a row tile whose rows are KB bytes, per chunk."""
-    nsc = (KB // 4 + steps_per_chunk - 1) // steps_per_chunk
-    for c in range(nsc):
-        if KB % 16 == 0:
-            for lane in range(64):
-                b = 64*c + 16*(lane % 4)
-                if b < KB:
-                    yield lane // 4, b, 16
-        else:
-            for u in range(4):
-                for lane in range(64):
-                    b = 64*c + 4*(lane % 16)
-                    if b < KB:
-                        yield 4*u + lane // 16, b, 4
+def sgemm_scale_reads(KB, sc_steps):
+    """(row of 16, first byte, bytes) of every weight-scale load of a row tile whose rows are KB bytes."""
+    if KB % 16:   # 4 bytes per step
+        for ks in range(KB // 4):
+            for row in range(16):
+                yield row, 4*ks, 4
+        return
+    words = sc_steps // 4   # 16-byte words of a row per chunk, each row's in a rotated order
+    for c in range(-(-KB // (16*words))):
+        for row in range(16):
+            for pos in range(words):
+                at = 16*words*c + 16*(pos ^ (row >> (2 if words == 4 else 3)))
+                if at < KB:
+                    yield row, at, 16
 
 
-@pytest.mark.parametrize('KB', [8, 16, 24, 40, 48, 56, 64, 72, 112, 224])
-def test_fgemm_scale_loads_stay_in_their_rows(KB):
+@pytest.mark.parametrize('KB', [4, 8, 12, 16, 20, 24, 48, 56, 64, 72, 112, 224])
+@pytest.mark.parametrize('sc_steps', [8, 16])
+def test_sgemm_scale_loads_stay_in_their_rows(KB, sc_steps):
     """Every scale byte of the tile is loaded once and no load leaves its row (the last row ends the tensor)."""
     seen = [[0]*KB for _ in range(16)]
-    for row, b, n in fgemm_scale_reads(KB, 16):
+    for row, b, n in sgemm_scale_reads(KB, sc_steps):
         assert b + n <= KB, (KB, row, b, n)
         for j in range(b, b + n):
             seen[row][j] += 1
     assert all(v == 1 for row in seen for v in row)
 
 
-@pytest.mark.parametrize('KS', [2, 6, 10, 18])
-def test_fgemm_stream_schedule_narrow_scales(KS):
-    """Rows that are not whole 16-byte words: four times the loads per chunk, the same order."""
-    fgemm_stream(KS, 3, ktiles=16)
+@pytest.mark.parametrize('ring,sc_steps', [(5, 16), (4, 8), (3, 16)])
+@pytest.mark.parametrize('KS', [1, 2, 3, 4, 5, 6, 8, 12, 16, 20, 24, 28, 48, 56, 64])
+@pytest.mark.parametrize('unit_rows', [[2], [1, 3, 2], [3, 1, 1, 2, 3, 1, 2]])
+def test_sgemm_stream_schedule(ring, sc_steps, KS, unit_rows):
+    """k_sgemm's loaders (csrc/k3moe_sgemm.hpp): steps issued ring - 1 ahead across units whose activation loads
+    differ, a wait that allows exactly the loads issued after the awaited step's, a step's slot and scale chunk free
+    when their loads go out, and (gate/up: at least ring - 1 steps) the next unit's rows landed when they are used."""
+    wide, gather, ahead = KS % 4 == 0, KS >= ring - 1, ring - 1
+    nsc = -(-KS // sc_steps)
+    total = KS*len(unit_rows)
+    issued, landed_rows = [], {}
+
+    def issue(g):
+        u, ks = divmod(g, KS)
+        n = 4 + unit_rows[u]
+        if gather and ks == 0:
+            if u > 0:   # the unit's rows came with step 0 of the unit before, which has been waited for
+                assert landed_rows[u] <= waited, (g, waited)
+            if u + 1 < len(unit_rows):
+                landed_rows[u + 1] = g
+                n += 1
+        chunk = None
+        if wide and (ks == 0 or (ks >= ahead and (ks - ahead) % sc_steps == 0 and (ks - ahead)//sc_steps + 1 < nsc)):
+            c = 0 if ks == 0 else (ks - ahead)//sc_steps + 1
+            chunk = u*nsc + c
+            n += 4
+        issued.append((g, n, chunk))
+
+    def chunk_of(g):
+        return g//KS*nsc + g % KS//sc_steps
+
+    waited = -1
+    counts = []
+    for g in range(min(ahead, total)):
+        issue(g)
+        counts.append(issued[-1][1])
+    later = sum(counts[1:])
+    counts = counts[1:] + [0]*(ahead - len(counts))
+    for g in range(total):
+        assert later == sum(n for gs, n, _ in issued if gs > g)
+        waited = g
+        done = g - 1   # at this barrier the MFMA waves have read every step up to this one
+        if wide:       # the step's chunk has been loaded, into the buffer it is read from
+            assert any(c == chunk_of(g) for gs, _, c in issued if gs <= g)
+        later -= counts[0]
+        counts = counts[1:] + [0]
+        if g + ahead < total:
+            issue(g + ahead)
+            assert g + ahead - ring <= done   # the slot's last step
+            chunk = issued[-1][2]
+            if chunk is not None:   # the buffer held chunk - 2: no unread step uses it
+                assert all(chunk_of(s) != chunk - 2 for s in range(done + 1, total))
+            counts[-1] = issued[-1][1]
+            later += counts[-1]
 
 
 def sk_order(lo, hi, KS):
