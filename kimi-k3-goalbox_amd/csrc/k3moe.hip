@@ -277,7 +277,7 @@ int lgemm_launch(LgPlan p, const LgemmArgs &a, hipStream_t st) {
   p.G = 1;
   while (p.G * 2 <= device_cus() && p.G * 2 <= 1024) p.G *= 2;
   if (p.RW == 8) return lgemm_launch_rows<OUT, 8>(p, a, st);
-  if (p.RW == 5) return lgemm_launch_rows<OUT, 5>(p, a, st);
+  if (p.RW == 6) return lgemm_launch_rows<OUT, 6>(p, a, st);
   if (p.RW == 4) return lgemm_launch_rows<OUT, 4>(p, a, st);
   return lgemm_launch_rows<OUT, 2>(p, a, st);
 }

@@ -10,8 +10,9 @@
 // once; run 64 rows at a time they reread the 136 MB of a TP8 rank per 64
 // tokens, 13 x 31 and 13 x 32 us at 777 tokens.)
 //
-// Tile = (32 RW weight rows, up to 32 TW tokens) of one workgroup: waves 0-3
-// multiply, 2 x 2, RW x TW 16x16x32 MFMA tiles each; waves 4-7 load. The
+// Tile = (32 RW weight rows, up to 32 TW tokens) of one workgroup: waves 0-7
+// multiply, 4 x 2, RW / 2 x TW 16x16x32 MFMA tiles each, two waves per SIMD (one's LDS
+// reads beside the other's MFMAs); waves 8-11 load. The
 // operands move 64 k at a time through Ring LDS slots filled by direct-to-LDS
 // loads Ring - 1 steps ahead, one barrier per step: rows of 128 bytes, the
 // 16-byte chunk c of row r at position c ^ ((r >> 1) & 7), so that the reads of
@@ -35,12 +36,12 @@
 // 64-token kernels' for every batch; inside the block the MoE step's, free before
 // and after it, takes the partials and the normalised rows.
 //
-// Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 26 + 7 us at 65
-// tokens (62 in two skinny launches), 109 at 777 (407), 213 at 2048 (988); <1> 24
-// + 5, 73 (416), 165 us (1024). Timing builds of <0> at 777: without the loads 83
-// us, without the MFMAs 80, without either 36: the LDS reads of the one MFMA wave
-// per SIMD (31 cycles for 16 bytes a lane) beside its MFMAs bound one side, the
-// loads (about 50 KB/us a CU, also with every line in L2) the other.
+// Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 22 + 7 us at 65
+// tokens (62 in two skinny launches), 100 at 777 (407), 209 at 2048 (988); <1> 20 +
+// 5, 75 + 7 (416), 169 + 11 us (1024); a large library product's rate would be 45 and
+// 118 us for <0>. With four MFMA waves <0> took 109 and 213 us; timing builds of that at
+// 777: without the loads 83 us, without the MFMAs 80, without either 36. The loads
+// move some 40 KB/us a CU whether their lines are in L2 or not.
 #pragma once
 
 #include "k3moe_device.hpp"
@@ -50,7 +51,8 @@
 
 namespace k3moe {
 
-constexpr int kLgThreads = 512;
+constexpr int kLgMfma = 8;  // MFMA waves, 4 x 2 over a tile's rows and tokens
+constexpr int kLgThreads = (kLgMfma + 4) * 64;
 constexpr int kLgCus = 256;  // the plans' compute units: tiles, splits and so the workspace do not depend on the device
 constexpr int kLgStepK = 64;
 constexpr int kLgMaxSplits = 8;         // (<2>: kMaxRouterSplits)
@@ -58,7 +60,7 @@ constexpr long kLgMaxPartials = 64L << 20;  // bytes of fp32 partials, at most
 
 struct LgPlan {
   int B, h, lh, S, act, out;
-  int RW, TW;    // MFMA tiles of a wave: 16 RW rows x 16 TW tokens
+  int RW, TW;    // a tile's 32 RW rows x 32 TW tokens (MFMA tiles of a wave: RW / 2 x TW)
   int N;         // weight rows: <0> lh + 2 S, <1> h, <2> the experts up to a whole tile (Plan::Epad)
   int NRB, NTG;  // row blocks, token groups
   int TG;        // tokens per group (a multiple of 16)
@@ -84,7 +86,7 @@ inline void lgemm_choose(LgPlan &p, int n_cus, int max_splits, long max_part) {
   const bool out = p.out == 1;
   const int KS = (out ? p.lh : p.h) / kLgStepK, KS0 = out ? p.S / kLgStepK : 0;
   const int TT = cdiv(p.B, 16);
-  const int rws[4] = {8, 5, 4, 2}, tws[3] = {4, 3, 2};
+  const int rws[4] = {8, 6, 4, 2}, tws[3] = {4, 3, 2};
   const int xcds = p.G < 8 ? p.G : 8, nslot = p.G / xcds;
   long best = -1;
   for (int rw : rws)
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, l = tid & 63, i = l & 15, q = l >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w = wv & 3;
+  const int w = wv & (kLgMfma - 1);  // the MFMA wave, or the loader 0 .. 3
   const int xcds = gridDim.x < 8 ? (int)gridDim.x : 8;
   const int xcd = blockIdx.x % xcds, nslot = gridDim.x / xcds, slot = blockIdx.x / xcds;
   const int j0 = (int)((long)pl.items * xcd / xcds), j1 = (int)((long)pl.items * (xcd + 1) / xcds);
@@ -203,37 +205,40 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
     return U;
   };
 
-  if (wv >= 4) {  // ------------------------------------------------ loader
-    // Loader w fills the 8-row blocks w + 4u of the weight rows and of the token
-    // rows: lane L covers row L / 8 of the block at position L % 8. Rows past the
-    // weights or the tokens repeat the last one (their results are not stored).
+  if (wv >= kLgMfma) {  // ------------------------------------------ loader
+    // Loader w fills the 8-row blocks w + 4u of the weight rows (whole blocks of one
+    // matrix: wave-uniform bases, to which a load adds the lane's offset itself) and of
+    // the token rows: lane L covers row L / 8 of the block at position L % 8. Blocks past
+    // the weights and rows past the tokens repeat the last one (their results are not
+    // stored).
     struct LoadP {
       const uint16_t *a[RW], *b[TW];
+      uint32_t al;  // the lane's byte offset in a weight block
     };
+    // position L % 8 of row r holds chunk (L % 8) ^ ((r >> 1) & 7); blocks are 8 rows: r >> 1 is 4 (block) + (L >> 4)
+    const uint32_t c0 = (uint32_t)((l & 7) ^ ((4 * (w & 1) + (l >> 4)) & 7)) * 16;
     auto load_params = [&](const UnitP &U) {
       LoadP P;
       const bool shared = OUT == 1 && U.seg == 0;
+      const int pitch = shared ? pl.S : OUT == 1 ? pl.lh : pl.h;  // elements of a weight row, and of a token row
+      const int rows = OUT == 2 ? pl.lh : pl.N;
+      P.al = (uint32_t)(l >> 3) * (uint32_t)pitch * 2u + c0;
 #pragma unroll
       for (int u = 0; u < RW; ++u) {
-        const int r = 8 * (w + 4 * u) + (l >> 3);
-        const int c = ((l & 7) ^ ((r >> 1) & 7)) * 8 + U.k0 * kLgStepK;
-        const int row = min(U.rb * 32 * RW + r, (OUT == 2 ? pl.lh : pl.N) - 1);
-        if (OUT == 2) {
-          P.a[u] = wa + (size_t)row * pl.h + c;
-        } else if (OUT == 1) {
-          P.a[u] = shared ? wb + (size_t)row * pl.S + c : wa + (size_t)row * pl.lh + c;
+        const int row = U.rb * 32 * RW + 8 * (w + 4 * u);
+        const uint16_t *base;
+        if (OUT == 0 && row < pl.N && row >= pl.lh) {  // pair tile sr / 16: 8 gate rows, then the same 8 up rows
+          const int sr = row - pl.lh;
+          base = ((sr & 8) ? wc : wb) + (size_t)(8 * (sr >> 4)) * pl.h;
         } else {
-          const int sr = row - pl.lh;  // pair tile sr / 16: 8 gate rows, then the same 8 up rows
-          const uint16_t *pair = (sr & 8) ? wc : wb;
-          P.a[u] = sr < 0 ? wa + (size_t)row * pl.h + c : pair + (size_t)(8 * (sr >> 4) + (sr & 7)) * pl.h + c;
+          base = (shared ? wb : wa) + (size_t)min(row, (OUT == 0 ? pl.lh : rows) - 8) * pitch;
         }
+        P.a[u] = base + U.k0 * kLgStepK;
       }
 #pragma unroll
       for (int u = 0; u < TW; ++u) {
-        const int r = 8 * (w + 4 * u) + (l >> 3);
-        const int c = ((l & 7) ^ ((r >> 1) & 7)) * 8 + U.k0 * kLgStepK;
-        const int t = min(U.tg * pl.TG + r, pl.B - 1);
-        P.b[u] = shared ? x2 + (size_t)t * pl.S + c : x + (size_t)t * (OUT == 1 ? pl.lh : pl.h) + c;
+        const int t = min(U.tg * pl.TG + 8 * (w + 4 * u) + (l >> 3), pl.B - 1);
+        P.b[u] = (shared ? x2 : x) + (size_t)t * pitch + c0 / 2 + U.k0 * kLgStepK;
       }
       return P;
     };
@@ -245,7 +250,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
       if (iu >= nu) return 0;
       char *base = lds + isl * Slot;
 #pragma unroll
-      for (int u = 0; u < RW; ++u) load_lds<16>(P.a[u] + iks * kLgStepK, base + (w + 4 * u) * 1024);
+      for (int u = 0; u < RW; ++u) load_lds<16>(reinterpret_cast<const char *>(P.a[u] + iks * kLgStepK) + P.al, base + (w + 4 * u) * 1024);
 #pragma unroll
       for (int u = 0; u < TW; ++u) load_lds<16>(P.b[u] + iks * kLgStepK, base + OffB + (w + 4 * u) * 1024);
       if (++isl == Ring) isl = 0;
@@ -276,14 +281,15 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
   }
 
   // ---------------------------------------------------------- MFMA wave
+  constexpr int RV = RW / 2;  // the wave's row tiles
   const int wr = w >> 1, wt = w & 1;
-  u32x4 fa[2][RW], fb[2][TW];  // operands of the step's two 32-k halves
+  u32x4 fa[2][RV], fb[2][TW];  // operands of the step's two 32-k halves
   int la[2], lb[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     la[kk] = i * 128 + (((4 * kk + q) ^ ((i >> 1) & 7)) * 16);
     lb[kk] = la[kk] + OffB + wt * TW * 2048;
-    la[kk] += wr * RW * 2048;
+    la[kk] += wr * RV * 2048;
   }
   asm("" : "+v"(la[0]), "+v"(la[1]), "+v"(lb[0]), "+v"(lb[1]));
   auto read = [&](int sl, int kk) {
@@ -291,23 +297,23 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
 #pragma unroll
     for (int t = 0; t < TW; ++t) fb[kk][t] = *reinterpret_cast<const u32x4 *>(pb + t * 2048);
 #pragma unroll
-    for (int r = 0; r < RW; ++r) fa[kk][r] = *reinterpret_cast<const u32x4 *>(pa + r * 2048);
+    for (int r = 0; r < RV; ++r) fa[kk][r] = *reinterpret_cast<const u32x4 *>(pa + r * 2048);
   };
-  f32x4 acc[RW][TW];
+  f32x4 acc[RV][TW];
   // The MFMAs of half kk, with the other half's operand reads spread between them:
   // a wave gets 16 bytes a lane from LDS in about 31 cycles (two MFMAs' time), and
   // reads issued in a row hold up its MFMAs.
   auto multiply = [&](int kk) {
 #pragma unroll
-    for (int r = 0; r < RW; ++r)
+    for (int r = 0; r < RV; ++r)
 #pragma unroll
       for (int t = 0; t < TW; ++t) acc[r][t] = mfma16(as_bf16x8(fa[kk][r]), as_bf16x8(fb[kk][t]), acc[r][t]);
 #pragma unroll
-    for (int n = 0; n < RW + TW; ++n) {
+    for (int n = 0; n < RV + TW; ++n) {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                            // an LDS read
-      __builtin_amdgcn_sched_group_barrier(0x8, (RW * TW) / (RW + TW), 0);          // MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x8, (RV * TW) / (RV + TW), 0);          // MFMAs
     }
-    __builtin_amdgcn_sched_group_barrier(0x8, RW * TW, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, RV * TW, 0);
   };
   int g = 0;
   ring_barrier();
@@ -315,7 +321,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
   for (int u = 0; u < nu; ++u) {
     const UnitP U = unit_at(u);
 #pragma unroll
-    for (int r = 0; r < RW; ++r)
+    for (int r = 0; r < RV; ++r)
 #pragma unroll
       for (int t = 0; t < TW; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int ks = U.k0; ks < U.k1; ++ks) {
@@ -329,14 +335,14 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
       __builtin_amdgcn_sched_barrier(0);
     }
     // lane (token column i, q) holds rows 4q .. 4q + 3 of each tile
-    const int row0 = U.rb * 32 * RW + wr * RW * 16;
+    const int row0 = U.rb * 32 * RW + wr * RV * 16;
     const int tend = min(pl.B, (U.tg + 1) * pl.TG);
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       const int tok = U.tg * pl.TG + (wt * TW + t) * 16 + i;
       const bool ok = tok < tend;
 #pragma unroll
-      for (int r = 0; r < RW; ++r) {
+      for (int r = 0; r < RV; ++r) {
         const int row = row0 + 16 * r;
         if (row >= pl.N) break;  // wave-uniform (N: whole tiles)
         const f32x4 c = acc[r][t];
