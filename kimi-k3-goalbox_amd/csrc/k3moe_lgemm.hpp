@@ -37,11 +37,11 @@
 // and after it, takes the partials and the normalised rows.
 //
 // Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 22 + 7 us at 65
-// tokens (62 in two skinny launches), 100 at 777 (407), 209 at 2048 (988); <1> 20 +
-// 5, 75 + 7 (416), 169 + 11 us (1024); a large library product's rate would be 45 and
-// 118 us for <0>. With four MFMA waves <0> took 109 and 213 us; timing builds of that at
-// 777: without the loads 83 us, without the MFMAs 80, without either 36. The loads
-// move some 40 KB/us a CU whether their lines are in L2 or not.
+// tokens (62 in two skinny launches), 96 at 777 (407), 203 at 2048 (988); <1> with
+// its norm 20 + 5, 74 + 7 (416), 165 + 11 us (1024). With four MFMA waves <0> took 26,
+// 109 and 213 us, <1> 24, 73 and 165; timing builds of that <0> at 777: without the
+// loads 83 us, without the MFMAs 80, without either 36, and the loads about 50 KB/us a
+// CU also with every line in L2.
 #pragma once
 
 #include "k3moe_device.hpp"

@@ -372,9 +372,8 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   const bool grouped = d.path == K3MOE_PATH_GROUPED || d.path == K3MOE_PATH_GROUPED_BF16;
   const bool many = (long)p.P >= (long)kXMinPairsPerExpert * p.E;
   const bool gemms = grouped || (d.path != K3MOE_PATH_STREAMED && widths);
-  const bool offsets = (long)p.B * p.K * 2 < (1L << 32);  // k_sgemm's 32-bit offsets of token rows
-  p.fgemm = gemms && (grouped || many) && d.path != K3MOE_PATH_GROUPED_BF16 && fp4_widths && offsets;
-  p.sgemm = p.fgemm ? 96 : gemms && !grouped && p.K >= kSMinWidth && offsets ? (many ? 64 : 32) : 0;
+  p.fgemm = gemms && (grouped || many) && d.path != K3MOE_PATH_GROUPED_BF16 && fp4_widths;
+  p.sgemm = p.fgemm ? 96 : gemms && !grouped && p.K >= kSMinWidth ? (many ? 64 : 32) : 0;
   p.xgemm = !p.sgemm && gemms && (grouped || many);  // grouped GEMMs of k3moe_xgemm.hpp
   p.Srw = (int)(p.G / p.RTr);  // decode router units: (row tile, split), every token tile
   if (p.Srw > srw_cap) p.Srw = srw_cap;

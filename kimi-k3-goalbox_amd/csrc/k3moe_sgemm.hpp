@@ -185,44 +185,41 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, MxAct act,
       for (int u = 0; u < kRowWords / 64; ++u)
         load_lds<4>(ptok + U.p0 + min(64 * u + l, U.m - 1), reinterpret_cast<char *>(rows + buf * kRowWords + 64 * u));
     };
-    // One unit's load addresses: wave-uniform bases (scalar registers; a load adds the
-    // lane's 32-bit offset itself) and the lane's rows of the activations.
-    struct LoadP {
-      const uint8_t *w[4], *s[4];  // the weight tiles, their scales
-      const uint8_t *x;            // the activations (down: from the unit's first pair)
-      uint32_t xo[kSRowLoads];     // the lane's offset of its row and chunk
-      uint32_t xso;                // FP4: the offset of the lane's scale dwords
-      int nx;                      // blocks of activation rows of this loader that hold tokens
+    struct LoadP {  // one unit's load addresses for this lane
+      const uint8_t *w[4], *s[4];  // weight tile rows (the lane's block of its row), scale rows
+      const uint8_t *sn;           // scale row of the lane's row (tile q, row i), for rows of no whole words
+      const uint8_t *x[kSRowLoads];  // bf16 rows; FP4: the hi rows
+      const uint8_t *xs;             // FP4: the lane's row of scales
+      int nx;                        // blocks of activation rows of this loader that hold tokens
     };
-    const uint32_t pitch = (uint32_t)KB * 16;  // bytes of a weight row's codes
-    const uint32_t wl = (uint32_t)(l >> 2) * pitch + (uint32_t)((l & 3) ^ a_swizzle(l >> 2)) * 16;
-    const uint32_t xpitch = (uint32_t)Kd * (FP4 ? 1 : 2);
-    const bool s_lo = 64 * w + l >= SM;  // FP4: loader w's scale dwords 64 w + L: the rows' hi ones, then their lo ones
-    // the lane's scale dwords: of row i of tile q, for rows of no whole words
-    const uint32_t snl = (uint32_t)(GU ? 16 * (q & 1) + i : 16 * q + i) * KB;
     auto load_params = [&](const UnitP &U, int buf) {
       LoadP P;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int orow = min(U.nb * RPB + (GU ? 32 * w + 16 * (r & 1) : 64 * w + 16 * r), Nout - 16);
         const size_t row = (size_t)U.e * Nout + orow;
-        P.w[r] = (GU && r >= 2 ? blk1 : blk0) + row * pitch;
+        P.w[r] = (GU && r >= 2 ? blk1 : blk0) + (row + (l >> 2)) * KB * 16 + ((l & 3) ^ a_swizzle(l >> 2)) * 16;
         P.s[r] = (GU && r >= 2 ? scl1 : scl0) + row * KB;
       }
-      P.x = GU ? act.hi : act.hi + (size_t)U.p0 * xpitch;
+      {
+        const int orow = min(U.nb * RPB + (GU ? 32 * w + 16 * (q & 1) : 64 * w + 16 * q), Nout - 16);
+        P.sn = (GU && q >= 2 ? scl1 : scl0) + ((size_t)U.e * Nout + orow + i) * KB;
+      }
       P.nx = 0;
 #pragma unroll
       for (int u = 0; u < kSRowLoads; ++u) {
         const int r0 = (FP4 ? 8 : 4) * (w + 4 * u), r = r0 + (FP4 ? l >> 3 : q);
         P.nx += r0 < U.m ? 1 : 0;
         const int rc = min(r, U.m - 1);
-        const uint32_t arow = GU ? (uint32_t)rows[buf * kRowWords + rc] : (uint32_t)rc;
-        P.xo[u] = arow * xpitch + (uint32_t)(FP4 ? (l & 7) ^ ((r >> 1) & 7) : i ^ s_swizzle(r)) * 16;
+        const size_t arow = GU ? (size_t)rows[buf * kRowWords + rc] : (size_t)(U.p0 + rc);
+        if constexpr (FP4) P.x[u] = act.hi + arow * Kd + ((l & 7) ^ ((r >> 1) & 7)) * 16;
+        else P.x[u] = act.hi + (arow * Kd + (i ^ s_swizzle(r)) * 8) * 2;
       }
-      if constexpr (FP4) {
-        const int d = 64 * w + l, r = min(d < SM ? d : d - SM, SM - 1);
-        const int rc = min(r, U.m - 1);
-        P.xso = (GU ? (uint32_t)rows[buf * kRowWords + rc] : (uint32_t)rc) * (uint32_t)KB;
+      if constexpr (FP4) {  // loader w: the scale dwords 64 w + L, the rows' hi ones, then their lo ones
+        const int d = 64 * w + l, r = d < SM ? d : d - SM;
+        const int rc = min(min(r, SM - 1), U.m - 1);
+        const size_t arow = GU ? (size_t)rows[buf * kRowWords + rc] : (size_t)(U.p0 + rc);
+        P.xs = (d < SM ? act.shi : act.slo) + arow * KB;
       }
       return P;
     };
@@ -236,19 +233,12 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, MxAct act,
       int n = 4 + (FP4 ? 2 : 1) * P.nx;
       if constexpr (FP4) {
         if (64 * w < 2 * SM) {  // wave-uniform
-          const size_t at = GU ? 0 : (size_t)(P.x - act.hi) / kBlockK;  // (an E4M3 row holds 32 bytes per scale)
-          load_lds<4>((s_lo ? act.slo : act.shi) + at + 4 * ks + P.xso, base + Geo::off_xs + w * 256);
+          load_lds<4>(P.xs + 4 * ks, base + Geo::off_xs + w * 256);
           n += 1;
         }
       }
-      if (!wide) {  // lane L: step ks's 4 scale bytes of row L of the 64 (a partial row block: the last whole tiles')
-        if (GU) {
-          load_lds<4>((q < 2 ? P.s[0] : P.s[2]) + 4 * ks + snl, lds + kSOffSc + sl * 1024 + w * 256);
-        } else {
-          const bool whole = P.s[3] == P.s[0] + (uint32_t)(48 * KB);  // wave-uniform
-          const uint8_t *sp = whole ? P.s[0] + snl : (q == 0 ? P.s[0] : q == 1 ? P.s[1] : q == 2 ? P.s[2] : P.s[3]) + (uint32_t)(i * KB);
-          load_lds<4>(sp + 4 * ks, lds + kSOffSc + sl * 1024 + w * 256);
-        }
+      if (!wide) {  // lane L: step ks's 4 scale bytes of row L of the 64
+        load_lds<4>(P.sn + 4 * ks, lds + kSOffSc + sl * 1024 + w * 256);
         n += 1;
       } else if (chunk_at(ks)) {
         // lane L: 16 bytes of one row's chunk (zero area past the row). ScSteps 16: row L / 4,
@@ -273,15 +263,15 @@ __global__ __launch_bounds__(kSThreads, 1) void k_sgemm(Plan pl, MxAct act,
         }
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) load_lds<16>(P.w[r] + ks * 64 + wl, base + kSOffW + (4 * w + r) * 1024);
+      for (int r = 0; r < 4; ++r) load_lds<16>(P.w[r] + ks * 64, base + kSOffW + (4 * w + r) * 1024);
 #pragma unroll
       for (int u = 0; u < kSRowLoads; ++u)
         if (u < P.nx) {
           if constexpr (FP4) {
-            load_lds<16>(P.x + ks * 128 + P.xo[u], base + 8 * (w + 4 * u) * 128);
-            load_lds<16>(P.x + (act.lo - act.hi) + ks * 128 + P.xo[u], base + SM * 128 + 8 * (w + 4 * u) * 128);
+            load_lds<16>(P.x[u] + ks * 128, base + 8 * (w + 4 * u) * 128);
+            load_lds<16>(P.x[u] + (act.lo - act.hi) + ks * 128, base + SM * 128 + 8 * (w + 4 * u) * 128);
           } else {
-            load_lds<16>(P.x + ks * 256 + P.xo[u], base + 4 * (w + 4 * u) * 256);
+            load_lds<16>(P.x[u] + ks * 256, base + 4 * (w + 4 * u) * 256);
           }
         }
       return n;
