@@ -71,8 +71,10 @@ struct LgPlan {
   long o_en, o_part;
 };
 
-// Cycles of one 64-k step: the MFMAs, or the LDS traffic (8 (RW + TW) KiB read,
-// 4 (RW + TW) KiB written, 128 bytes a cycle), whichever is longer.
+// Cycles of one 64-k step, to rank the variants by: the MFMAs, or the LDS traffic
+// (4 (RW + TW) KiB written, 8 (RW + TW) KiB read, 128 bytes a cycle), whichever is
+// longer. (The reads are those of 2 x 2 waves; the 4 x 2 that run read 8 RW + 16 TW
+// KiB. The times above are of the choices that this estimate makes.)
 inline long lgemm_step_cost(int RW, int TW) {
   const long mfma = 32L * RW * TW, lds = 96L * (RW + TW);
   return (mfma > lds ? mfma : lds) + 60;
@@ -206,14 +208,15 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
   };
 
   if (wv >= kLgMfma) {  // ------------------------------------------ loader
-    // Loader w fills the 8-row blocks w + 4u of the weight rows (whole blocks of one
-    // matrix: wave-uniform bases, to which a load adds the lane's offset itself) and of
-    // the token rows: lane L covers row L / 8 of the block at position L % 8. Blocks past
-    // the weights and rows past the tokens repeat the last one (their results are not
-    // stored).
+    // Loader w fills the 8-row blocks w + 4u of the weight rows (wave-uniform bases, to
+    // which a load adds the lane's offset itself) and of the token rows: lane L covers row
+    // L / 8 of the block at position L % 8. <0>, <1>: a block lies in one matrix, and
+    // blocks past the weights repeat the last one; <2>: any number of experts, so rows
+    // past the last repeat it, also inside a block. Rows past the tokens repeat the last
+    // (none of these results are used).
     struct LoadP {
       const uint16_t *a[RW], *b[TW];
-      uint32_t al;  // the lane's byte offset in a weight block
+      uint32_t al[OUT == 2 ? RW : 1];  // the lane's byte offset in a weight block
     };
     // position L % 8 of row r holds chunk (L % 8) ^ ((r >> 1) & 7); blocks are 8 rows: r >> 1 is 4 (block) + (L >> 4)
     const uint32_t c0 = (uint32_t)((l & 7) ^ ((4 * (w & 1) + (l >> 4)) & 7)) * 16;
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
       const bool shared = OUT == 1 && U.seg == 0;
       const int pitch = shared ? pl.S : OUT == 1 ? pl.lh : pl.h;  // elements of a weight row, and of a token row
       const int rows = OUT == 2 ? pl.lh : pl.N;
-      P.al = (uint32_t)(l >> 3) * (uint32_t)pitch * 2u + c0;
+      if (OUT != 2) P.al[0] = (uint32_t)(l >> 3) * (uint32_t)pitch * 2u + c0;
 #pragma unroll
       for (int u = 0; u < RW; ++u) {
         const int row = U.rb * 32 * RW + 8 * (w + 4 * u);
@@ -230,6 +233,10 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
         if (OUT == 0 && row < pl.N && row >= pl.lh) {  // pair tile sr / 16: 8 gate rows, then the same 8 up rows
           const int sr = row - pl.lh;
           base = ((sr & 8) ? wc : wb) + (size_t)(8 * (sr >> 4)) * pl.h;
+        } else if (OUT == 2) {
+          const int first = min(row, rows - 1);
+          base = wa + (size_t)first * pitch;
+          P.al[OUT == 2 ? u : 0] = (uint32_t)min(l >> 3, rows - 1 - first) * (uint32_t)pitch * 2u + c0;
         } else {
           base = (shared ? wb : wa) + (size_t)min(row, (OUT == 0 ? pl.lh : rows) - 8) * pitch;
         }
@@ -250,7 +257,7 @@ __global__ __launch_bounds__(kLgThreads, 1) void k_lgemm(LgPlan pl, const uint16
       if (iu >= nu) return 0;
       char *base = lds + isl * Slot;
 #pragma unroll
-      for (int u = 0; u < RW; ++u) load_lds<16>(reinterpret_cast<const char *>(P.a[u] + iks * kLgStepK) + P.al, base + (w + 4 * u) * 1024);
+      for (int u = 0; u < RW; ++u) load_lds<16>(reinterpret_cast<const char *>(P.a[u] + iks * kLgStepK) + P.al[OUT == 2 ? u : 0], base + (w + 4 * u) * 1024);
 #pragma unroll
       for (int u = 0; u < TW; ++u) load_lds<16>(P.b[u] + iks * kLgStepK, base + OffB + (w + 4 * u) * 1024);
       if (++isl == Ring) isl = 0;

@@ -12,8 +12,11 @@ import pytest
 import torch
 
 import k3moe
+from k3moe import synthetic
+from k3moe.configs import MoEConfig
 from oracle import latent_ref
 from test_gpu_latent import block_weights, near_oracle
+from test_gpu_moe import run_and_check
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +59,11 @@ def test_latent_gemms_match_64_row_launches(gpu, B):
         near_oracle(sh[rows], psh.cpu(), steps=2)
         pout = k3moe.latent_out(g['expert_sum'][rows].contiguous(), *wout, sh[rows].contiguous(), g['shared_down'])
         near_oracle(out[rows], pout.cpu(), steps=2, floor=2e-2)
+
+
+@pytest.mark.parametrize('E,k,B', [(3, 2, 5), (7, 3, 70), (9, 2, 2), (12, 6, 33), (20, 4, 129), (61, 8, 3)])
+def test_router_rows_of_no_whole_blocks(gpu, E, k, B):
+    """The router's rows end inside a loader's block of 8 (or before its first ends)."""
+    say(f'case: router E={E} k={k} B={B} seed=0')
+    cfg = MoEConfig(f'e{E}', E, k, 384, 256, B)
+    run_and_check(cfg, synthetic.moe_layer_inputs(cfg, 0, scale_mode='kimi'), gpu, path='general')
