@@ -1,11 +1,12 @@
-// General MoE-step path: a chain of six kernels, any token count.
+// General MoE-step path: a chain of eight to ten kernels, any token count.
 //
-//   k_router   router logits x . router^T on MFMA, split over k      (kimi.py:308)
+//   k_lgemm<2> router logits x . router^T on MFMA, split over k (k3moe_lgemm.hpp;
+//              k_router for widths of no whole 64-k steps)         (kimi.py:308)
 //   k_topk     FP32 gating + top-k + renormalised weights, 1 wave/token (kimi.py:308-316)
 //   k_group_*  expert histogram, active-expert list, token->expert pairs (kimi.py:319-320)
-//   k_gateup   gate and up projections of every active expert, FP4 dequant in
-//              registers, MFMA, activation epilogue -> bf16 h          (kimi.py:321-322)
-//   k_down     down projection of every active expert -> bf16 y       (kimi.py:322)
+//   k_sgemm    gate/up -> activation -> bf16 h and down -> bf16 y of every active
+//              expert (k3moe_sgemm.hpp; k3moe_xgemm.hpp on the forced grouped paths;
+//              k_gateup and k_down below where no 128-k steps fit, or forced) (kimi.py:321-322)
 //   k_combine  FP32 routing-weighted sum in ascending expert order    (kimi.py:318,323)
 #pragma once
 
