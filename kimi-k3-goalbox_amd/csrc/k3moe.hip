@@ -25,9 +25,9 @@
 #include "k3moe_general.hpp"
 #include "k3moe_latent.hpp"
 #include "k3moe_lgemm.hpp"
+#include "k3moe_persistent.hpp"
 #include "k3moe_plan.hpp"
 #include "k3moe_sgemm.hpp"
-#include "k3moe_single.hpp"
 #include "k3moe_xgemm.hpp"
 
 using namespace k3moe;
@@ -126,7 +126,6 @@ int launch_check(const char *what) {
   return K3MOE_OK;
 }
 
-// Lets the decode kernel use more than 64 KiB of dynamic LDS (once per process).
 // Raises kernel fn's dynamic LDS limit to `limit` bytes (once per kernel and process).
 int grant_lds(const void *fn, int limit, int &granted, const char *what) {
   if (granted >= limit) return K3MOE_OK;
@@ -136,38 +135,11 @@ int grant_lds(const void *fn, int limit, int &granted, const char *what) {
   return K3MOE_OK;
 }
 
-// The decode kernel instantiation for a plan: whole gate/up super-steps (K a
-// multiple of 512) and the expert-major down variant of its I.
-typedef void (*DecodeKernel)(Plan, DecodeArgs);
-DecodeKernel decode_kernel(const Plan &p, int &slot) {
-  // the latent block's phases (which need whole 512-column gate/up chunks, AL)
-  // in their own instantiations: row 2
-  static const DecodeKernel table[3][4] = {
-      {k_moe_decode<false, 0, false>, k_moe_decode<false, 2, false>, k_moe_decode<false, 3, false>,
-       k_moe_decode<false, 4, false>},
-      {k_moe_decode<true, 0, false>, k_moe_decode<true, 2, false>, k_moe_decode<true, 3, false>,
-       k_moe_decode<true, 4, false>},
-      {k_moe_decode<true, 0, true>, k_moe_decode<true, 2, true>, k_moe_decode<true, 3, true>,
-       k_moe_decode<true, 4, true>}};
-  const int al = (p.K / kBlockK) % 16 == 0 ? 1 : 0;
-  const int row = p.lat_in ? 2 : al;  // (lat_in plans are pinned: AL)
-  const int v = p.I == 256 ? 1 : p.I == 384 ? 2 : p.I == 512 ? 3 : 0;
-  slot = row * 4 + v;
-  return table[row][v];
-}
-
-// The single-token kernel's instantiation `slot` may use more than 64 KiB of dynamic LDS.
-int allow_single_lds(const void *fn, int slot, int bytes) {
-  static int granted[8] = {0};
+// Instantiation `slot` of the persistent kernels may use more than 64 KiB of dynamic LDS.
+int allow_lds(PersistentKernel fn, int slot, int bytes) {
+  static int granted[kPersistentKernels] = {0};
   if (bytes <= 65536) return K3MOE_OK;
-  return grant_lds(fn, kDecMaxLds - kDecStaticLds, granted[slot], "single-token");
-}
-
-int allow_lds(DecodeKernel fn, int slot, int bytes) {
-  static int granted[12] = {0};
-  if (bytes <= 65536) return K3MOE_OK;
-  // dynamic + static LDS must fit the 160 KiB of a workgroup
-  return grant_lds(reinterpret_cast<const void *>(fn), kDecMaxLds - kDecStaticLds, granted[slot], "decode");
+  return grant_lds(reinterpret_cast<const void *>(fn), kDecMaxLds - kDecStaticLds, granted[slot], "persistent");
 }
 
 int allow_xgemm_lds() {
@@ -653,33 +625,11 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
       a.lat_sd = reinterpret_cast<const uint16_t *>(lat->shared_down);
       a.lat_y = reinterpret_cast<uint16_t *>(lat->out);
     }
-    if (p.single) {
-      // instantiations: chosen experts per wave in the down phase (1: k <= 8, 2: k <= 16) and
-      // the down projection's k-steps (2: I <= 256, 4: I <= 512)
-      // (and the latent block's phases: a separate instantiation)
-      const bool je2 = p.k > kDecWaves, ks4 = p.I > 256, lat = p.lat_in != 0;
-      auto launch = [&](auto kernel) -> int {
-        int r = allow_single_lds(reinterpret_cast<const void *>(kernel), lat * 4 + je2 * 2 + ks4, p.lds_total);
-        if (r) return r;
-        hipLaunchKernelGGL(kernel, dim3(p.G), dim3(kDecThreads), p.lds_total, st, p, a);
-        return launch_check("single-token step");
-      };
-      if (lat) {
-        if (je2 && ks4) return launch(k_moe_single<2, 4, true>);
-        if (je2) return launch(k_moe_single<2, 2, true>);
-        if (ks4) return launch(k_moe_single<1, 4, true>);
-        return launch(k_moe_single<1, 2, true>);
-      }
-      if (je2 && ks4) return launch(k_moe_single<2, 4, false>);
-      if (je2) return launch(k_moe_single<2, 2, false>);
-      if (ks4) return launch(k_moe_single<1, 4, false>);
-      return launch(k_moe_single<1, 2, false>);
-    }
     int slot = 0;
-    const DecodeKernel fn = decode_kernel(p, slot);
+    const PersistentKernel fn = persistent_kernel(p, slot);
     if ((rc = allow_lds(fn, slot, p.lds_total))) return rc;
     hipLaunchKernelGGL(fn, dim3(p.G), dim3(kDecThreads), p.lds_total, st, p, a);
-    return launch_check("decode step");
+    return launch_check(p.single ? "single-token step" : "decode step");
   }
 
   if (p.rgemm) {

@@ -37,7 +37,6 @@
 
 #include "k3moe_barrier.hpp"
 #include "k3moe_device.hpp"
-#include "k3moe_general.hpp"
 #include "k3moe_plan.hpp"
 
 namespace k3moe {
@@ -1395,6 +1394,7 @@ __device__ __forceinline__ DecodeArgs load_args(uint64_t at) {
 // that path is not used). Each instantiation holds one variant of each, which
 // keeps the kernel's code (and its instruction-cache footprint) small.
 template <bool AL, int KSD, bool LAT>
+__attribute__((aligned(kPersistentAlign)))
 __global__ __launch_bounds__(kDecThreads, 1) void k_moe_decode(Plan pl_arg, DecodeArgs a_arg) {
   const uint64_t t_entry = __builtin_amdgcn_s_memrealtime();  // (stored when tracing)
   // The arguments, read through the touched segment (pl_arg at offset 0, a_arg after it).

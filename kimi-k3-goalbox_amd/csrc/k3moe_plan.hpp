@@ -30,6 +30,7 @@ constexpr int kXMinPairsPerExpert = 16;  // general path: token-expert pairs per
 constexpr int kSMinWidth = 512;  // general path: least K of the streaming grouped GEMMs (their loads run up to 4 k-steps ahead)
 constexpr int kMaxRouterSplits = 16;     // general path: router k-splits (partials summed by the top-k kernel)
 
+constexpr int kPersistentAlign = 32768;  // of the persistent kernels' code (k3moe_persistent.hip)
 constexpr int kDecWaves = 8;       // decode path: waves per workgroup
 constexpr int kDecThreads = kDecWaves * 64;
 constexpr int kDecMaxTokens = 64;

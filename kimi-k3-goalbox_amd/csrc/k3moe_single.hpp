@@ -77,6 +77,7 @@ struct SgDn {
 // JE: chosen experts per wave in the down phase (k <= 8 JE); KSD: the down
 // projection's k-steps of 128 (I <= 128 KSD).
 template <int JE, int KSD, bool LAT>
+__attribute__((aligned(kPersistentAlign)))
 __global__ __launch_bounds__(kDecThreads, 1) void k_moe_single(Plan pl_arg, DecodeArgs a_arg) {
   const uint64_t t_entry = __builtin_amdgcn_s_memrealtime();  // (stored when tracing)
   const uint64_t kargs = touch_kernargs<sizeof(Plan) + sizeof(DecodeArgs)>();

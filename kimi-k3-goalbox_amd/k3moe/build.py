@@ -5,8 +5,8 @@ depend on torch's headers or ABI. Packed FP32 instructions are disabled for
 the device code (-Xclang -target-feature -Xclang -packed-fp32-ops). hipcc hands
 that option to both compiler passes and the host (x86) pass prints
 "'-packed-fp32-ops' is not a recognized feature for this target"; the device
-pass applies it. Every build then disassembles the gfx950 code object of the
-new library and fails if a v_pk_add_f32, v_pk_mul_f32 or v_pk_fma_f32 is in it
+pass applies it. Every build then disassembles the gfx950 code objects of the
+new library and fails if a v_pk_add_f32, v_pk_mul_f32 or v_pk_fma_f32 is in them
 (`check_no_packed_fp32`), so the guard does not rest on the option alone.
 
 Floating-point contraction is off (-ffp-contract=off): every product and sum
@@ -22,6 +22,7 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG_ROOT = os.path.dirname(HERE)
@@ -30,8 +31,8 @@ REPO = os.path.dirname(PKG_ROOT)
 OUT = os.path.join(HERE, 'libk3moe.so')
 ARCH = os.environ.get('K3MOE_ARCH', 'gfx950')
 
-SOURCES = ['k3moe.hip']
-HEADERS = ['k3moe_device.hpp']
+# Translation units, each a code object of its own (k3moe_persistent.hip: why).
+SOURCES = ['k3moe.hip', 'k3moe_persistent.hip']
 
 
 def hipcc() -> str:
@@ -41,12 +42,12 @@ def hipcc() -> str:
     raise RuntimeError('hipcc not found')
 
 
-def command(out: str = OUT) -> list[str]:
-    return [hipcc(), f'--offload-arch={ARCH}', '-O3', '-std=c++17', '-fPIC', '-shared', '-ffp-contract=off',
+def command(out: str = OUT, source: str = SOURCES[0], how: str = '-shared') -> list[str]:
+    """The hipcc line that makes `out` (how: '-shared' a library, '-c' an object) of one source."""
+    return [hipcc(), f'--offload-arch={ARCH}', '-O3', '-std=c++17', '-fPIC', how, '-ffp-contract=off',
             '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
             '-Wno-unused-command-line-argument',
-            '-I', os.path.join(REPO, 'include'),
-            *[os.path.join(CSRC, s) for s in SOURCES], '-o', out]
+            '-I', os.path.join(REPO, 'include'), os.path.join(CSRC, source), '-o', out]
 
 
 HOST_PASS_NOTE = "'-packed-fp32-ops' is not a recognized feature for this target"
@@ -61,20 +62,32 @@ def llvm_tool(name: str) -> str:
     raise RuntimeError(f'{name} not found under the ROCm llvm tools')
 
 
-def device_disassembly(lib: str) -> str:
-    """The gfx950 code object of `lib`, disassembled (llvm-objdump, in a scratch directory)."""
-    import tempfile
+def code_objects(lib: str, tool: str, *args: str) -> list[str]:
+    """What an llvm tool prints for each gfx950 code object of `lib` (extracted in a scratch directory)."""
     with tempfile.TemporaryDirectory() as tmp:
         copy = os.path.join(tmp, 'lib.so')
         shutil.copyfile(lib, copy)
         subprocess.run([llvm_tool('llvm-objdump'), '--offloading', copy], cwd=tmp, check=True,
                        capture_output=True, text=True)
-        objs = [f for f in os.listdir(tmp) if f.endswith(f'amdgcn-amd-amdhsa--{ARCH}')]
-        if len(objs) != 1:
-            raise RuntimeError(f'expected one {ARCH} code object in {lib}, found {objs}')
-        res = subprocess.run([llvm_tool('llvm-objdump'), '-d', f'--mcpu={ARCH}', objs[0]], cwd=tmp,
-                             check=True, capture_output=True, text=True)
-        return res.stdout
+        objs = sorted(f for f in os.listdir(tmp) if f.endswith(f'amdgcn-amd-amdhsa--{ARCH}'))
+        if not objs:
+            raise RuntimeError(f'no {ARCH} code object in {lib}')
+        return [subprocess.run([llvm_tool(tool), *args, obj], cwd=tmp, check=True, capture_output=True,
+                               text=True).stdout for obj in objs]
+
+
+def device_disassembly(lib: str) -> str:
+    """The gfx950 code objects of `lib`, disassembled."""
+    return ''.join(code_objects(lib, 'llvm-objdump', '-d', f'--mcpu={ARCH}'))
+
+
+def kernel_addresses(lib: str = OUT) -> list[dict[str, int]]:
+    """Per code object of `lib`: its kernels' mangled names and their code's addresses in it."""
+    tables = []
+    for text in code_objects(lib, 'llvm-readelf', '-s', '-W'):
+        rows = (ln.split() for ln in text.splitlines())
+        tables.append({r[7]: int(r[1], 16) for r in rows if len(r) == 8 and r[3] == 'FUNC'})
+    return tables
 
 
 def check_no_packed_fp32(lib: str = OUT) -> int:
@@ -91,13 +104,20 @@ def build(verbose: bool = False) -> str:
     """Compile every HIP source into libk3moe.so (always rebuilds), check its
     device code for packed FP32 and return its path."""
     tmp = OUT + '.tmp'
-    cmd = command(tmp)
-    if verbose:
-        print(' '.join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError('hipcc failed:\n' + res.stderr)
-    lines = [ln for ln in res.stderr.splitlines() if ln.strip()]
+    with tempfile.TemporaryDirectory() as objects:
+        objs = [os.path.join(objects, s + '.o') for s in SOURCES]
+        cmds = [command(obj, src, '-c') for obj, src in zip(objs, SOURCES)]
+        if verbose:
+            print('\n'.join(' '.join(c) for c in cmds), flush=True)
+        runs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for c in cmds]
+        said = [r.communicate()[0] for r in runs]   # (both compile at once)
+        if any(r.returncode for r in runs):
+            raise RuntimeError('hipcc failed:\n' + '\n'.join(said))
+        link = subprocess.run([hipcc(), f'--offload-arch={ARCH}', '-shared', '-fPIC', *objs, '-o', tmp],
+                              capture_output=True, text=True)
+        if link.returncode != 0:
+            raise RuntimeError('hipcc failed to link:\n' + link.stderr)
+    lines = [ln for text in said for ln in text.splitlines() if ln.strip()]
     host_notes = [ln for ln in lines if HOST_PASS_NOTE in ln]
     other = [ln for ln in lines if HOST_PASS_NOTE not in ln]
     if verbose and host_notes:

@@ -193,6 +193,19 @@ def test_device_code_has_no_packed_fp32():
     assert build.check_no_packed_fp32(_native.LIB_PATH) > 100_000
 
 
+def test_persistent_kernels_lie_alone_at_their_alignment():
+    """The persistent kernels fill a code object of their own, each at a multiple of kPersistentAlign, so that no
+    other kernel's size moves them (their times depend on it: csrc/k3moe_persistent.hip)."""
+    from k3moe import build
+    plan = open(os.path.join(build.CSRC, 'k3moe_plan.hpp')).read()
+    align = int(re.search(r'kPersistentAlign = (\d+);', plan).group(1))
+    tables = [t for t in build.kernel_addresses(_native.LIB_PATH) if any('k_moe_' in name for name in t)]
+    assert len(tables) == 1 and len(tables[0]) == 20
+    for name, address in tables[0].items():
+        assert 'k_moe_decode' in name or 'k_moe_single' in name, name
+        assert address % align == 0, (name, address)
+
+
 PACKED_PROBE = r'''
 #include <hip/hip_runtime.h>
 extern "C" __global__ void probe(float2* a, const float2* b, int n) {
