@@ -96,7 +96,11 @@ typedef struct k3moe_dims {
 /* Device workspace bytes the step needs for `dims` (256-byte aligned base,
  * zero-initialised control block, see k3moe_workspace_init).
  * Replaces the temporaries of kimi.py:308-323 (logits, index lists, the
- * per-expert decoded weights, which this library never materialises). */
+ * per-expert decoded weights, which this library never materialises). Past the
+ * persistent kernels' batches (64 tokens) AUTO's bytes do not fall as tokens
+ * grow where topk x latent >= 32 x experts (and inter and latent are
+ * multiples of 128); elsewhere a workspace for several batches takes the
+ * largest of their sizes. */
 int k3moe_workspace_bytes(const k3moe_dims *dims, size_t *bytes);
 
 /* One MoE step (kimi.py:307-324 without the TP all-reduce of line 324):

@@ -634,7 +634,7 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
 
   if (p.rgemm) {
     LgPlan lp;
-    lgemm_router_plan(p.B, p.h, p.E, p.Epad, kLgCus, lp);
+    lgemm_router_plan(p, kLgCus, lp);
     rc = lgemm_launch<2>(lp, LgemmArgs{reinterpret_cast<const uint16_t *>(x), nullptr,
                                        reinterpret_cast<const uint16_t *>(router), nullptr, nullptr, nullptr, nullptr,
                                        reinterpret_cast<float *>(ws + p.o_logit)}, st);

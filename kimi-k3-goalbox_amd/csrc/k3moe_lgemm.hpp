@@ -53,99 +53,6 @@ namespace k3moe {
 
 constexpr int kLgMfma = 8;  // MFMA waves, 4 x 2 over a tile's rows and tokens
 constexpr int kLgThreads = (kLgMfma + 4) * 64;
-constexpr int kLgCus = 256;  // the plans' compute units: tiles, splits and so the workspace do not depend on the device
-constexpr int kLgStepK = 64;
-constexpr int kLgMaxSplits = 8;         // (<2>: kMaxRouterSplits)
-constexpr long kLgMaxPartials = 64L << 20;  // bytes of fp32 partials, at most
-
-struct LgPlan {
-  int B, h, lh, S, act, out;
-  int RW, TW;    // a tile's 32 RW rows x 32 TW tokens (MFMA tiles of a wave: RW / 2 x TW)
-  int N;         // weight rows: <0> lh + 2 S, <1> h, <2> the experts up to a whole tile (Plan::Epad)
-  int NRB, NTG;  // row blocks, token groups
-  int TG;        // tokens per group (a multiple of 16)
-  int splits;    // k splits of x (<0>, <2>) or en (<1>); 1: a workgroup does all of a tile and stores the outputs
-  int segs;      // k segments of a tile: <0>, <2> splits, <1> 1 + splits (the shared part first)
-  int items;     // work items of the grid
-  int G;
-  long o_en, o_part;
-};
-
-// Cycles of one 64-k step, to rank the variants by: the MFMAs, or the LDS traffic
-// (4 (RW + TW) KiB written, 8 (RW + TW) KiB read, 128 bytes a cycle), whichever is
-// longer. (The reads are those of 2 x 2 waves; the 4 x 2 that run read 8 RW + 16 TW
-// KiB. The times above are of the choices that this estimate makes.)
-inline long lgemm_step_cost(int RW, int TW) {
-  const long mfma = 32L * RW * TW, lds = 96L * (RW + TW);
-  return (mfma > lds ? mfma : lds) + 60;
-}
-
-// The variant and split count of the least estimated time on n_cus compute units
-// (the launch's grid follows the device).
-inline void lgemm_choose(LgPlan &p, int n_cus, int max_splits, long max_part) {
-  p.G = 1;
-  while (p.G * 2 <= n_cus && p.G * 2 <= 1024) p.G *= 2;
-  const bool out = p.out == 1;
-  const int KS = (out ? p.lh : p.h) / kLgStepK, KS0 = out ? p.S / kLgStepK : 0;
-  const int TT = cdiv(p.B, 16);
-  const int rws[4] = {8, 6, 4, 2}, tws[3] = {4, 3, 2};
-  const int xcds = p.G < 8 ? p.G : 8, nslot = p.G / xcds;
-  long best = -1;
-  for (int rw : rws)
-    for (int tw : tws)
-      for (int s = 1; s <= max_splits && s <= KS; ++s) {
-        const int nrb = cdiv(p.N, 32 * rw), ntg = cdiv(TT, 2 * tw);
-        const int segs = out ? 1 + s : s;
-        const long items = (long)nrb * ntg * (s > 1 ? segs : 1);
-        if (s > 1 && (long)segs * p.B * p.N * 4 > max_part) break;
-        const long rounds = cdiv(cdiv(items, xcds), nslot);
-        long t = rounds * ((s > 1 ? cdiv(KS, s) : KS + KS0) * lgemm_step_cost(rw, tw) + 2000);
-        if (s > 1 || p.out == 2) t += (long)segs * p.B * p.N / 2000;  // the partials out and in
-        if (s > 1 && p.out != 2) t += 12000;                          // and a launch
-        if (best < 0 || t < best) {
-          best = t;
-          p.RW = rw; p.TW = tw; p.splits = s; p.segs = segs; p.NRB = nrb; p.NTG = ntg; p.items = (int)items;
-          p.TG = cdiv(TT, ntg) * 16;
-        }
-      }
-}
-
-// Plan of k_lgemm<out> in `avail` bytes of workspace (at least the 64-token kernels',
-// whose area holds 64 normalised rows): the partials of its splits fit, and <1>
-// takes as many of the d.tokens rows at a time (p.B) as it can hold normalised, in
-// launches of equal size. avail follows from the dimensions alone, and so do the
-// splits and the order of the sums.
-inline void lgemm_plan(const k3moe_latent_dims &d, int n_cus, int out, long avail, LgPlan &p) {
-  p = LgPlan{};
-  p.B = d.tokens; p.h = d.hidden; p.lh = d.latent; p.S = d.shared; p.act = d.activation; p.out = out;
-  p.N = out ? p.h : p.lh + 2 * p.S;
-  long o = kInitBytes;
-  if (out) {
-    const long fit = (avail - o - 256) / (2L * p.lh) / 16 * 16;
-    const int launches = cdiv(p.B, fit);
-    p.B = cdiv(cdiv(p.B, launches), 16) * 16;
-    if (p.B > d.tokens) p.B = d.tokens;
-    p.o_en = o;
-    o = (long)align256((size_t)(o + (long)p.B * p.lh * 2));
-  }
-  p.o_part = o;
-  const long room = avail - o;
-  lgemm_choose(p, n_cus, kLgMaxSplits, room < kLgMaxPartials ? room : kLgMaxPartials);
-}
-
-// Plan of the router's k_lgemm<2> for a general-path step: B tokens of width h (a
-// multiple of 64) against E experts.
-inline void lgemm_router_plan(int B, int h, int E, int Epad, int n_cus, LgPlan &p) {
-  p = LgPlan{};
-  p.B = B; p.h = h; p.lh = E; p.N = Epad; p.out = 2;  // (lh: the weights' rows)
-  lgemm_choose(p, n_cus, kMaxRouterSplits, kLgMaxPartials);
-}
-
-inline int router_splits(int B, int h, int E, int Epad) {
-  LgPlan p;
-  lgemm_router_plan(B, h, E, Epad, kLgCus, p);
-  return p.splits;
-}
 
 template <int RW, int TW>
 struct LgGeom {

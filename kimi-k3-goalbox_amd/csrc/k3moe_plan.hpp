@@ -314,7 +314,112 @@ inline bool lat_out_plan(Plan &p) {
   return ok;
 }
 
-inline int router_splits(int B, int h, int E, int Epad);  // of lgemm_router_plan (k3moe_lgemm.hpp)
+// ------------------------------------- plans of k_lgemm (k3moe_lgemm.hpp) --
+
+constexpr int kLgCus = 256;  // the plans' compute units: tiles, splits and so the workspace do not depend on the device
+constexpr int kLgStepK = 64;
+constexpr int kLgMaxSplits = 8;         // (<2>: kMaxRouterSplits)
+constexpr long kLgMaxPartials = 64L << 20;  // bytes of fp32 partials, at most
+
+struct LgPlan {
+  int B, h, lh, S, act, out;
+  int RW, TW;    // a tile's 32 RW rows x 32 TW tokens (MFMA tiles of a wave: RW / 2 x TW)
+  int N;         // weight rows: <0> lh + 2 S, <1> h, <2> the experts up to a whole tile (Plan::Epad)
+  int NRB, NTG;  // row blocks, token groups
+  int TG;        // tokens per group (a multiple of 16)
+  int splits;    // k splits of x (<0>, <2>) or en (<1>); 1: a workgroup does all of a tile and stores the outputs
+  int segs;      // k segments of a tile: <0>, <2> splits, <1> 1 + splits (the shared part first)
+  int items;     // work items of the grid
+  int G;
+  long o_en, o_part;
+};
+
+// Cycles of one 64-k step, to rank the variants by: the MFMAs, or the LDS traffic
+// (4 (RW + TW) KiB written, 8 (RW + TW) KiB read, 128 bytes a cycle), whichever is
+// longer. (The reads are those of 2 x 2 waves; the 4 x 2 that run read 8 RW + 16 TW
+// KiB. The times above are of the choices that this estimate makes.)
+inline long lgemm_step_cost(int RW, int TW) {
+  const long mfma = 32L * RW * TW, lds = 96L * (RW + TW);
+  return (mfma > lds ? mfma : lds) + 60;
+}
+
+// The variant and split count of the least estimated time on n_cus compute units
+// (the launch's grid follows the device).
+inline void lgemm_choose(LgPlan &p, int n_cus, int max_splits, long max_part) {
+  p.G = 1;
+  while (p.G * 2 <= n_cus && p.G * 2 <= 1024) p.G *= 2;
+  const bool out = p.out == 1;
+  const int KS = (out ? p.lh : p.h) / kLgStepK, KS0 = out ? p.S / kLgStepK : 0;
+  const int TT = cdiv(p.B, 16);
+  const int rws[4] = {8, 6, 4, 2}, tws[3] = {4, 3, 2};
+  const int xcds = p.G < 8 ? p.G : 8, nslot = p.G / xcds;
+  long best = -1;
+  for (int rw : rws)
+    for (int tw : tws)
+      for (int s = 1; s <= max_splits && s <= KS; ++s) {
+        const int nrb = cdiv(p.N, 32 * rw), ntg = cdiv(TT, 2 * tw);
+        const int segs = out ? 1 + s : s;
+        const long items = (long)nrb * ntg * (s > 1 ? segs : 1);
+        if (s > 1 && (long)segs * p.B * p.N * 4 > max_part) break;
+        const long rounds = cdiv(cdiv(items, xcds), nslot);
+        long t = rounds * ((s > 1 ? cdiv(KS, s) : KS + KS0) * lgemm_step_cost(rw, tw) + 2000);
+        if (s > 1 || p.out == 2) t += (long)segs * p.B * p.N / 2000;  // the partials out and in
+        if (s > 1 && p.out != 2) t += 12000;                          // and a launch
+        if (best < 0 || t < best) {
+          best = t;
+          p.RW = rw; p.TW = tw; p.splits = s; p.segs = segs; p.NRB = nrb; p.NTG = ntg; p.items = (int)items;
+          p.TG = cdiv(TT, ntg) * 16;
+        }
+      }
+}
+
+// Plan of k_lgemm<out> in `avail` bytes of workspace (at least the 64-token kernels',
+// whose area holds 64 normalised rows): the partials of its splits fit, and <1>
+// takes as many of the d.tokens rows at a time (p.B) as it can hold normalised, in
+// launches of equal size. avail follows from the dimensions alone, and so do the
+// splits and the order of the sums.
+inline void lgemm_plan(const k3moe_latent_dims &d, int n_cus, int out, long avail, LgPlan &p) {
+  p = LgPlan{};
+  p.B = d.tokens; p.h = d.hidden; p.lh = d.latent; p.S = d.shared; p.act = d.activation; p.out = out;
+  p.N = out ? p.h : p.lh + 2 * p.S;
+  long o = kInitBytes;
+  if (out) {
+    const long fit = (avail - o - 256) / (2L * p.lh) / 16 * 16;
+    const int launches = cdiv(p.B, fit);
+    p.B = cdiv(cdiv(p.B, launches), 16) * 16;
+    if (p.B > d.tokens) p.B = d.tokens;
+    p.o_en = o;
+    o = (long)align256((size_t)(o + (long)p.B * p.lh * 2));
+  }
+  p.o_part = o;
+  const long room = avail - o;
+  lgemm_choose(p, n_cus, kLgMaxSplits, room < kLgMaxPartials ? room : kLgMaxPartials);
+}
+
+// k-splits of k_router: tiles of 64 tokens x 384 experts, at least 256 workgroups, at most 8 splits.
+inline int router_splits(const Plan &pl) {
+  int s = cdiv(256, (long)cdiv(pl.B, 64) * cdiv(pl.E, 384));
+  if (s > 8) s = 8;
+  if (s > pl.KSr) s = pl.KSr;
+  return s < 1 ? 1 : s;
+}
+
+// Bytes that the general path's router partials may take. They lie in the pair outputs' (y), which
+// are written after the top-k has summed them; room for k_router's splits is added where those need
+// more. With k latent >= 2 splits experts, as in expert layers of use, the partials then add nothing
+// and the workspace grows with the batch, however the splits fall.
+inline long router_room(const Plan &pl) {
+  const long y = (long)pl.P * pl.K * 2, partials = (long)router_splits(pl) * pl.B * pl.Epad * 4;
+  return y > partials ? y : partials;
+}
+
+// Plan of the router's k_lgemm<2> for a general-path step (h a multiple of 64), in router_room bytes.
+inline void lgemm_router_plan(const Plan &pl, int n_cus, LgPlan &p) {
+  p = LgPlan{};
+  p.B = pl.B; p.h = pl.h; p.lh = pl.E; p.N = pl.Epad; p.out = 2;  // (lh: the weights' rows)
+  const long room = router_room(pl);
+  lgemm_choose(p, n_cus, kMaxRouterSplits, room < kLgMaxPartials ? room : kLgMaxPartials);
+}
 
 // n_cus: compute units of the device (the persistent grid size); trace: reserve
 // a timestamp area (kTraceSlots x 8 bytes per workgroup, up to 1024 groups).
@@ -381,21 +486,20 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   if (p.Srw < 1) p.Srw = 1;
   decode_lds(p);
 
-  // general path: the router's splits (rgemm, k3moe_lgemm.hpp: widths of whole
-  // 64-k steps; otherwise tiles of 64 tokens x 384 experts, at least 256
-  // workgroups, at most 8 splits), gate/up streams about 2048 waves
+  // general path: the router's splits (rgemm, k3moe_lgemm.hpp: widths of whole 64-k steps;
+  // otherwise k_router's), gate/up streams about 2048 waves
   p.rgemm = p.h % 64 == 0;
-  p.Sr = cdiv(256, (long)cdiv(p.B, 64) * cdiv(p.E, 384));
-  if (p.Sr > 8) p.Sr = 8;
-  if (p.Sr > p.KSr) p.Sr = p.KSr;
-  if (p.Sr < 1) p.Sr = 1;
-  if (p.rgemm && p.path == kPathGeneral) p.Sr = router_splits(p.B, p.h, p.E, p.Epad);
+  p.Sr = router_splits(p);
+  if (p.rgemm && p.path == kPathGeneral) {
+    LgPlan r;
+    lgemm_router_plan(p, kLgCus, r);
+    p.Sr = r.splits;
+  }
   base = (long)p.Dmax * p.RTg;
   p.Sg = cdiv(2048, base);
   if (p.Sg > p.KSg) p.Sg = p.KSg;
   if (p.Sg < 1) p.Sg = 1;
-  const int logit_splits = p.path == kPathDecode ? 0 : p.Sr;  // decode: partials in the tag area
-  if (p.path == kPathDecode) p.Sr = p.Srw;
+  if (p.path == kPathDecode) p.Sr = p.Srw;  // (its partials lie in the tag area)
 
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o = align256(o + bytes); return at; };
@@ -403,7 +507,6 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   p.o_zero = take(kZeroBytes);
   take(kLatCntBytes);  // the latent block's counters, kept by MoE steps on a shared workspace
   take(kTagBytes);     // the persistent kernels' tagged exchange area
-  p.o_logit = take((size_t)logit_splits * p.B * p.Epad * 4);
   p.o_ids = take((size_t)p.P * 4);
   p.o_w = take((size_t)p.P * 4);
   p.o_nact = take(16);  // {active experts, groups}
@@ -419,15 +522,19 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   p.o_gcnt = take(streams ? (size_t)p.Dmax * p.RTg * 4 : 0);
   p.o_gchunk = take(general ? (size_t)cdiv(p.B, kGroupChunk) * p.E * 4 : 0);  // grouping: per-chunk counts
   // the streaming GEMMs' group table: {expert, first pair, pairs, -} per group
-  p.o_gtab = take(general && p.sgemm ? (size_t)(p.P / p.sgemm + p.Dmax) * 16 : 0);
+  // (room for units of 32, however many pairs they hold: the bytes grow with the batch)
+  p.o_gtab = take(general && p.sgemm ? (size_t)(p.P / 32 + p.Dmax) * 16 : 0);
   const bool fg = general && p.fgemm;
   p.o_h = take(fg ? 0 : (size_t)p.P * p.I * 2);
   // two-term E4M3 activations of the FP4-MFMA GEMMs: expert inputs [B, K] and h [P, I]
   // (hi, lo, then the hi and lo block scales)
   p.o_xq = take(fg ? (size_t)p.B * p.K * 2 + (size_t)p.B * (p.K / 32) * 2 : 0);
   p.o_hq = take(fg ? (size_t)p.P * p.I * 2 + (size_t)p.P * (p.I / 32) * 2 : 0);
-  // pair outputs: the general path, and the decode path's expert-major down (I = 256, 384, 512)
-  p.o_y = take((general || p.I == 256 || p.I == 384 || p.I == 512) ? (size_t)p.P * p.K * 2 : 0);
+  // pair outputs: the general path (its router partials before them), and the decode path's
+  // expert-major down (I = 256, 384, 512)
+  const size_t y = (size_t)p.P * p.K * 2, partials = (size_t)p.Sr * p.B * p.Epad * 4;
+  p.o_y = take(general ? (y > partials ? y : partials) : p.I == 256 || p.I == 384 || p.I == 512 ? y : 0);
+  p.o_logit = p.o_y;
   p.trace = trace && p.path == kPathDecode;
   p.stall = 0;
   p.lat_in = 0;

@@ -114,13 +114,30 @@ def test_latent_dims_struct_matches_header():
     assert fields == [f for f, _ in _native.LatentDims._fields_]
 
 
+SHIPPED = {   # experts, top-k, hidden, latent, inter; the largest batch that the library's own 16 MiB array must hold
+    'tp8': ((384, 8, 7168, 7168, 256), 110), 'kimi': ((896, 16, 7168, 3584, 384), 92),
+    'small': ((64, 8, 2048, 2048, 256), 320), 'unsharded': ((384, 8, 7168, 7168, 2048), 89)}
+
+
+@pytest.mark.parametrize('name', sorted(SHIPPED))
+def test_general_workspace_grows_with_the_batch(name):
+    """A workspace sized for a batch of the general path holds every smaller one, whatever splits the router takes."""
+    (E, k, h, K, I), fits = SHIPPED[name]
+    last = 0
+    for B in range(65, 4097):
+        n = moe.workspace_bytes(_native.Dims(tokens=B, experts=E, topk=k, hidden=h, latent=K, inter=I))
+        assert n >= last, (B, n, last)
+        assert n <= 16 << 20 or B > fits, (B, n)
+        last = n
+
+
 @pytest.mark.parametrize('B', [1, 8, 64, 200])
 def test_latent_workspace_bytes_kimi_rank(B):
     from k3moe import latent
     n = latent.latent_workspace_bytes(latent.latent_dims(B, 7168, 3584, 768))
     # at least the counters' area and one split's fp32 partials of every output row
     assert n % 256 == 0 and n >= 4096 + 65536 + 16384 + min(B, 64)*7168*4
-    if B > 64:   # launches of 64 token rows: the 64-row workspace serves them
+    if B > 64:   # GEMMs in the 64-row kernels' workspace
         assert n == latent.latent_workspace_bytes(latent.latent_dims(64, 7168, 3584, 768))
 
 
