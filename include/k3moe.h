@@ -79,7 +79,11 @@ extern "C" {
  * Expert tensor layouts are the reference's (kimi.py:116-119), all u8:
  *   gate_blocks, up_blocks [E, I, K/32, 16]   gate_scales, up_scales [E, I, K/32]
  *   down_blocks            [E, K, I/32, 16]   down_scales            [E, K, I/32]
- * Byte j of a 16-byte block holds element 2j (low nibble) and 2j+1 (high). */
+ * Byte j of a 16-byte block holds element 2j (low nibble) and 2j+1 (high).
+ * Tensors are contiguous. x, latent and the latent block's tensors start at a
+ * multiple of 16 bytes. So should the router and the expert tensors (scales
+ * whose rows are not whole 16-byte words: of 4): past the persistent kernels'
+ * batches those that do not take slower kernels, whichever path is forced. */
 typedef struct k3moe_dims {
     int32_t tokens;
     int32_t experts;
@@ -180,6 +184,8 @@ int k3moe_moe_step_noalloc(const k3moe_dims *dims,
  *                 hi u8 [B, K/32], lo u8 [B, K/32] (-1 on other paths)
  *   h_split       h in the same form: [B k, I] twice, then [B k, I/32] twice
  *                 (-1 on other paths; pair_h is then -1 too: h is kept only split)
+ *                 (a step whose tensors' start keeps it from these GEMMs, see
+ *                 k3moe_dims, leaves h there as pair_h's bf16)
  * The persistent decode path keeps its grouping in LDS; for dims that select
  * it this returns K3MOE_EINVAL. */
 typedef struct k3moe_layout {

@@ -302,20 +302,39 @@ int latent_launch(const k3moe_latent_dims *dims, int out, const LatArgs &a, size
     return fail(K3MOE_EWORKSPACE, "workspace of %zu bytes is smaller than the %zu required", workspace_bytes, need);
   if (reinterpret_cast<uintptr_t>(a.ws) % 256) return fail(K3MOE_EWORKSPACE, "workspace must be 256-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dims->tokens > kLatMaxTokens) {
+  if (dims->tokens > kLatMaxTokens && at_multiple(a.x, 16) && at_multiple(a.wa, 16) && at_multiple(a.wb, 16) &&
+      at_multiple(a.wc, 16)) {
     if (room > workspace_bytes) room = workspace_bytes;
     const long avail = (long)(room > need ? room : need);
     return out ? latent_gemm<1>(dims, a, avail, st) : latent_gemm<0>(dims, a, avail, st);
   }
+  // up to kLatMaxTokens rows, or, where a tensor starts inside a 16-byte word (the GEMMs read them
+  // by direct-to-LDS loads of 16 bytes), that many at a time
+  k3moe_latent_dims c = *dims;
+  if (c.tokens > kLatMaxTokens) c.tokens = kLatMaxTokens;
   LatPlan pin, pout;
-  if ((rc = latent_plans(dims, device_cus(), pin, pout))) return rc;
-  const LatPlan &p = out ? pout : pin;
-  if ((rc = allow_latent_lds(out, p.sk, p.lds_total))) return rc;
-  if (p.sk && out) hipLaunchKernelGGL(k_latent_sk<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
-  else if (p.sk) hipLaunchKernelGGL(k_latent_sk<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
-  else if (out) hipLaunchKernelGGL(k_latent<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
-  else hipLaunchKernelGGL(k_latent<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, a);
-  return launch_check(out ? "latent_out" : "latent_in");
+  if ((rc = latent_plans(&c, device_cus(), pin, pout))) return rc;
+  const long trace = (out ? pout : pin).o_trace;
+  for (int b0 = 0; b0 < dims->tokens; b0 += kLatMaxTokens) {  // token rows b0 .. b0 + c.tokens - 1
+    if (dims->tokens - b0 < c.tokens) {
+      c.tokens = dims->tokens - b0;
+      if ((rc = latent_plans(&c, device_cus(), pin, pout))) return rc;
+    }
+    LatPlan p = out ? pout : pin;
+    p.o_trace = trace;
+    LatArgs ac = a;
+    ac.x = a.x + (long)b0 * (out ? dims->shared : dims->hidden);
+    ac.ya = a.ya + (long)b0 * (out ? dims->hidden : dims->latent);
+    if (out) ac.esum = a.esum + (long)b0 * dims->latent;
+    else ac.yb = a.yb + (long)b0 * dims->shared;
+    if ((rc = allow_latent_lds(out, p.sk, p.lds_total))) return rc;
+    if (p.sk && out) hipLaunchKernelGGL(k_latent_sk<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
+    else if (p.sk) hipLaunchKernelGGL(k_latent_sk<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
+    else if (out) hipLaunchKernelGGL(k_latent<1>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
+    else hipLaunchKernelGGL(k_latent<0>, dim3(p.G), dim3(kLatThreads), p.lds_total, st, p, ac);
+    if ((rc = launch_check(out ? "latent_out" : "latent_in"))) return rc;
+  }
+  return K3MOE_OK;
 }
 
 // The expert GEMMs' activation, elementwise (debug entry point k3moe_activation).
@@ -596,6 +615,8 @@ static int moe_step_impl(const k3moe_dims *dims, const void *x, const void *late
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   char *ws = reinterpret_cast<char *>(workspace);
   const uint16_t *xin = reinterpret_cast<const uint16_t *>(latent ? latent : x);
+
+  place_plan(p, x, xin, router, gate_blocks, gate_scales, up_blocks, up_scales, down_blocks, down_scales);
 
   if (p.path == kPathDecode) {
     DecodeArgs a{};

@@ -383,7 +383,7 @@ __global__ __launch_bounds__(1024) void k_group_scan(Plan pl, char *ws) {
       }
     }
   }
-  if (!pl.xgemm && !pl.sgemm) {
+  if (!pl.xgemm && !pl.sgemm && pl.Sg > 1) {
     int *gcnt = reinterpret_cast<int *>(ws + pl.o_gcnt);
     for (int i = tid; i < pl.Dmax * pl.RTg; i += 1024) gcnt[i] = 0;
   }

@@ -550,4 +550,32 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   p.total = o;
 }
 
+// Whether v lies at a multiple of n bytes.
+inline bool at_multiple(const void *v, int n) { return reinterpret_cast<uintptr_t>(v) % n == 0; }
+
+// Fits a general-path plan to where the caller's tensors lie. The GEMMs read them by direct-to-LDS
+// loads, of 16 bytes (weight scales of rows that are no whole 16-byte words: of 4): tensors that
+// start inside such a word take the kernels with ordinary loads, k_router's for the router's rows
+// and the per-16-token streams (not split over k: the plan's workspace has no room for partials).
+inline void place_plan(Plan &p, const void *x, const void *xin, const void *router, const void *gate_blocks,
+                       const void *gate_scales, const void *up_blocks, const void *up_scales,
+                       const void *down_blocks, const void *down_scales) {
+  if (p.path != kPathGeneral) return;
+  if (p.rgemm && !(at_multiple(x, 16) && at_multiple(router, 16))) {
+    const int fits = p.Sr;
+    p.rgemm = 0;
+    p.Sr = router_splits(p);
+    if ((long)p.Sr * p.B * p.Epad * 4 > (long)p.P * p.K * 2 && p.Sr > fits) p.Sr = fits;
+  }
+  const int gu = p.K / 32 % 16 ? 4 : 16, dn = p.I / 32 % 16 ? 4 : 16;
+  if ((p.sgemm || p.xgemm) &&
+      !(at_multiple(xin, 16) && at_multiple(gate_blocks, 16) && at_multiple(up_blocks, 16) &&
+        at_multiple(down_blocks, 16) && at_multiple(gate_scales, gu) && at_multiple(up_scales, gu) &&
+        at_multiple(down_scales, dn))) {
+    if (p.fgemm) p.o_h = p.o_hq;
+    p.sgemm = p.xgemm = p.fgemm = 0;
+    p.Sg = 1;
+  }
+}
+
 }  // namespace k3moe

@@ -63,3 +63,54 @@ def test_streaming_gemms_token_counts(gpu, counts):
     routes = torch.tensor([[e, lo + t % (E - lo)] for t, e in enumerate(first)], dtype=torch.int64, device=gpu)
     say(f'case: {cfg.name} tokens per expert {counts} seed=1')
     check(*both(cfg, 1, gpu, routes))
+
+
+def moved(t, off, dev):
+    """t's copy on dev that starts off bytes past a 256-byte boundary."""
+    raw = torch.empty(t.numel()*t.element_size() + off, dtype=torch.uint8, device=dev)
+    view = raw[off:].view(t.dtype).view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize('name,off', [('gate_scales', 1), ('up_scales', 3), ('down_scales', 5), ('gate_blocks', 4),
+                                      ('down_blocks', 8), ('latent', 4), ('router', 4)])
+@pytest.mark.parametrize('cfg', [MoEConfig('sgemm-i128', 24, 4, 512, 128, 70, latent=512),
+                                 MoEConfig('sgemm-fp4', 16, 4, 512, 512, 96, gating='softmax', latent=1024)],
+                         ids=lambda c: c.name)
+def test_tensors_inside_a_word(gpu, cfg, name, off):
+    """A tensor that starts inside a 16-byte word (scales: at any byte) takes the kernels with ordinary loads."""
+    say(f'case: {cfg.name} {name} at byte {off}')
+    inputs = synthetic.moe_layer_inputs(cfg, 3, scale_mode='kimi')
+    g = {k: (v.to(gpu) if isinstance(v, torch.Tensor) else v) for k, v in inputs.items()}
+    kw = dict(topk=cfg.topk, gating=cfg.gating, activation=cfg.activation)
+    want = k3moe.moe_step(*synthetic.step_args(g), latent=g['latent'], path='streamed', **kw)
+    g[name] = moved(g[name], off, gpu)
+    got = k3moe.moe_step(*synthetic.step_args(g), latent=g['latent'], **kw)
+    if name == 'router':
+        # the logits' h = 512 products are summed by another kernel, in another order: two fp32 sums differ by at most
+        # 2 x 512 x 2^-24 of the products' magnitudes' sum (512 x E|x| x E|w| = 6.5; 9 covers its largest), 5.5e-4, and
+        # a weight by no more than its logits
+        assert float((got['route_weights'] - want['route_weights']).abs().max()) <= 5.5e-4
+        got = {**got, 'route_weights': want['route_weights']}
+    check(got, want)
+
+
+@pytest.mark.parametrize('name', ['latent_down', 'shared_up', 'latent_up', 'shared_down'])
+def test_latent_weights_inside_a_word(gpu, name):
+    """The latent block's projections past 64 tokens with such a weight: launches of 64 rows, on shapes whose 64-row
+    kernels read the weights by ordinary loads."""
+    from test_gpu_latent import block_weights, near_oracle
+    B, h, lh, S = 100, 512, 256, 128
+    say(f'case: latent B={B} h={h} lh={lh} S={S} {name} at byte 4')
+    g = {k: v.to(gpu) for k, v in block_weights(B, h, lh, S, 4).items()}
+
+    def both():
+        lat, sh = k3moe.latent_in(g['x'], g['latent_down'], g['shared_gate'], g['shared_up'])
+        return lat, sh, k3moe.latent_out(g['expert_sum'], g['latent_norm'], g['latent_up'], g['shared_h'],
+                                         g['shared_down'])
+    g['shared_h'] = k3moe.latent_in(g['x'], g['latent_down'], g['shared_gate'], g['shared_up'])[1]
+    want = [t.cpu() for t in both()]
+    g[name] = moved(g[name], 4, gpu)
+    for t, w, steps in zip(both(), want, (1, 2, 2)):
+        near_oracle(t, w, steps=steps, floor=2e-2)
