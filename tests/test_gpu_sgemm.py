@@ -1,13 +1,14 @@
-"""GPU checks of the streaming grouped GEMMs (k_sgemm; run with -m gpu).
+"""GPU checks of the streaming grouped GEMMs in their bf16 forms (k_sgemm; run with -m gpu).
 
-Batches past the decode kernel's whose experts average fewer than 16 tokens run
-them on the general path. Checked against the per-16-token streams on the same
-routing (the same products, summed in fp32 in another order, so the bf16
+Batches past the decode kernel's run them on the general path: with 32 pairs per
+unit below 16 tokens per expert, with 64 from there on where the widths do not fit
+the FP4 form (test_gpu_fgemm.py). Checked against the per-16-token streams on the
+same routing (the same products, summed in fp32 in another order, so the bf16
 roundings of gate, up, h and y flip now and then: the bar of the grouped GEMMs'
-comparison) at the edges of the units: 1 to 33 and 64 to 65 tokens of an expert
-(one or two 16-token tiles, one to three groups), reductions of 1 to 8 k-steps,
-odd counts, scale rows that are not whole 16-byte words, a partial row block,
-and no expert active twice in a row.
+comparison) at the edges of the units: 1 to 33, 48 and 49, 64 and 65 and 129 tokens
+of an expert (partly filled 16-token tiles, one to five groups), reductions of 1 to
+28 k-steps, odd counts, scale rows that are not whole 16-byte words, a partial row
+block, and no expert active twice in a row.
 """
 
 import pytest
@@ -45,7 +46,7 @@ def check(a, b):
     MoEConfig('sgemm-i128', 24, 4, 512, 128, 70),                               # 4 and 1 k-steps
     MoEConfig('sgemm-k640-i384', 32, 4, 640, 384, 100, activation='silu'),      # narrow scales, a partial row block
     MoEConfig('sgemm-i512', 16, 2, 1024, 512, 90, gating='softmax'),            # whole scale words in both
-    MoEConfig('sgemm-k3584-i384', 48, 16, 512, 384, 66, latent=3584),    # two scale chunks
+    MoEConfig('sgemm-k3584-i384', 48, 16, 512, 384, 66, latent=3584),           # 64 pairs per unit, four scale chunks
     MoEConfig('sgemm-b800', 896, 16, 256, 128, 800, latent=512),                # many groups
 ], ids=lambda c: c.name)
 def test_streaming_gemms_match_the_streams(gpu, cfg):
@@ -62,6 +63,21 @@ def test_streaming_gemms_token_counts(gpu, counts):
     lo = len(counts) + 1
     routes = torch.tensor([[e, lo + t % (E - lo)] for t, e in enumerate(first)], dtype=torch.int64, device=gpu)
     say(f'case: {cfg.name} tokens per expert {counts} seed=1')
+    check(*both(cfg, 1, gpu, routes))
+
+
+@pytest.mark.parametrize('K,I', [(640, 384), (640, 1536), (3584, 640)])
+@pytest.mark.parametrize('counts', [(33, 48, 49, 64, 65, 129), (1, 16, 17, 130, 31, 193)])
+def test_units_of_64_pairs_token_counts(gpu, counts, K, I):
+    """As above for the units of 64 pairs (at least 16 pairs per expert on average, widths that the FP4 form does not
+    take): scale rows of whole words and not in both GEMMs, a partial row block in each."""
+    B, E = sum(counts), 20
+    cfg = MoEConfig('sgemm64-counts', E, 2, K, I, B)
+    assert 2*B >= 16*E and (K % 512 or I % 256)
+    first = [e for e, n in enumerate(counts) for _ in range(n)]
+    lo = len(counts) + 1
+    routes = torch.tensor([[e, lo + t % (E - lo)] for t, e in enumerate(first)], dtype=torch.int64, device=gpu)
+    say(f'case: {cfg.name} K={K} I={I} tokens per expert {counts} seed=1')
     check(*both(cfg, 1, gpu, routes))
 
 
