@@ -1,14 +1,12 @@
 """CPU checks of kernels' load schedules (restated here from their sources).
 
-k_sgemm (csrc/k3moe_sgemm.hpp), its loader stream: test_sgemm_*, and, for the
-two steps ahead of the FP4 form with a fixed number of loads per step,
-test_fgemm_stream_schedule: units stream back to back; a loader issues the
-step two ahead at every barrier (the next unit's first two steps during the
-last two of the current one), waits before the barrier of step g until only
-the loads of step g + 1 may be outstanding, and puts weight-scale chunk c of a
-unit (16 steps each) into buffer (unit's first chunk number + c) & 1. Checked:
-the wait counts equal the loads issued after step g, and no chunk buffer is
-overwritten while a step still reads its older content.
+k_sgemm (csrc/k3moe_sgemm.hpp), its loader stream, in the bf16 forms (test_sgemm_*)
+and the FP4 form (test_fgemm_stream_schedule): units stream back to back; a
+loader issues the step ring - 1 ahead at every barrier, waits before it until only
+the loads of later steps may be outstanding, and puts weight-scale chunk c of a
+unit into buffer (unit's first chunk number + c) & 1. Checked: the wait counts equal
+the loads issued after the awaited step, no slot or chunk buffer is overwritten
+while a step still reads its older content, and a unit's rows are there when used.
 
 k_latent_sk (csrc/k3moe_latent.hpp): the (row tile, step) items are cut into G
 equal runs; a tile must be whole in one run or cut once, every cut tile's two
@@ -16,51 +14,6 @@ segments must carry the parts they store, and the second to count in must sum
 both into every step of the tile, each part exactly once.
 """
 import pytest
-
-
-def fgemm_stream(KS, nunits, kloads=11, ktiles=4, steps_per_chunk=16):
-    nsc = (KS + steps_per_chunk - 1) // steps_per_chunk
-    chunk_at = lambda s: s == 0 or (s >= 2 and (s - 2) % steps_per_chunk == 0
-                                    and (s - 2) // steps_per_chunk + 1 < nsc)
-    issued = []  # (global step, loads, (buffer, chunk number) or None)
-
-    def issue(ks, g, cb0):
-        chunk = None
-        if chunk_at(ks):
-            c = 0 if ks == 0 else (ks - 2) // steps_per_chunk + 1
-            chunk = ((cb0 + c) & 1, cb0 + c)
-        issued.append((g, kloads + (ktiles if chunk else 0), chunk))
-
-    reads = {u * KS + ks: (((u * nsc + ks // steps_per_chunk) & 1), u * nsc + ks // steps_per_chunk)
-             for u in range(nunits) for ks in range(KS)}
-    issue(0, 0, 0)
-    issue(1, 1, 0)
-    for u in range(nunits):
-        g0, cb0, have_next = u * KS, u * nsc, u + 1 < nunits
-        for ks in range(KS):
-            g = g0 + ks
-            if ks + 1 < KS:
-                allow = kloads + (ktiles if chunk_at(ks + 1) else 0)
-            else:
-                allow = kloads + ktiles if have_next else 0
-            after = sum(n for gs, n, _ in issued if gs > g)
-            assert after == allow, (KS, u, ks, after, allow)
-            if ks + 2 < KS:
-                issue(ks + 2, g + 2, cb0)
-            elif have_next:
-                issue(ks + 2 - KS, g + 2, cb0 + nsc)
-            else:
-                continue
-            if issued[-1][2] is not None:
-                buf, chunk = issued[-1][2]
-                # the MFMA waves may still read step g (and later ones): none of them older content
-                assert all(not (reads[gg][0] == buf and reads[gg][1] < chunk) for gg in range(g, nunits * KS))
-
-
-@pytest.mark.parametrize('KS', [4, 8, 12, 16, 20, 24, 28, 32, 48, 56, 64])
-@pytest.mark.parametrize('nunits', [1, 2, 3, 5])
-def test_fgemm_stream_schedule(KS, nunits):
-    fgemm_stream(KS, nunits)
 
 
 def sgemm_scale_reads(KB, sc_steps):
@@ -91,13 +44,9 @@ def test_sgemm_scale_loads_stay_in_their_rows(KB, sc_steps):
     assert all(v == 1 for row in seen for v in row)
 
 
-@pytest.mark.parametrize('ring,sc_steps', [(5, 16), (4, 8), (3, 16)])
-@pytest.mark.parametrize('KS', [1, 2, 3, 4, 5, 6, 8, 12, 16, 20, 24, 28, 48, 56, 64])
-@pytest.mark.parametrize('unit_rows', [[2], [1, 3, 2], [3, 1, 1, 2, 3, 1, 2]])
-def test_sgemm_stream_schedule(ring, sc_steps, KS, unit_rows):
-    """k_sgemm's loaders (csrc/k3moe_sgemm.hpp): steps issued ring - 1 ahead across units whose activation loads
-    differ, a wait that allows exactly the loads issued after the awaited step's, a step's slot and scale chunk free
-    when their loads go out, and (gate/up: at least ring - 1 steps) the next unit's rows landed when they are used."""
+def sgemm_stream(ring, sc_steps, KS, unit_rows, row_loads=1, step_loads=0, gather_loads=1):
+    """One loader's run over units with unit_rows blocks of activation rows each (row_loads loads a block; step_loads
+    more in every step): its waits, slots, scale chunks and gathered rows."""
     wide, gather, ahead = KS % 4 == 0, KS >= ring - 1, ring - 1
     nsc = -(-KS // sc_steps)
     total = KS*len(unit_rows)
@@ -105,18 +54,18 @@ def test_sgemm_stream_schedule(ring, sc_steps, KS, unit_rows):
 
     def issue(g):
         u, ks = divmod(g, KS)
-        n = 4 + unit_rows[u]
+        n = 4 + row_loads*unit_rows[u] + step_loads + (0 if wide else 1)
         if gather and ks == 0:
             if u > 0:   # the unit's rows came with step 0 of the unit before, which has been waited for
                 assert landed_rows[u] <= waited, (g, waited)
             if u + 1 < len(unit_rows):
                 landed_rows[u + 1] = g
-                n += 1
+                n += gather_loads
         chunk = None
         if wide and (ks == 0 or (ks >= ahead and (ks - ahead) % sc_steps == 0 and (ks - ahead)//sc_steps + 1 < nsc)):
             c = 0 if ks == 0 else (ks - ahead)//sc_steps + 1
             chunk = u*nsc + c
-            n += 4
+            n += 4 if sc_steps == 16 else 2   # (two tiles' chunks a load)
         issued.append((g, n, chunk))
 
     def chunk_of(g):
@@ -145,6 +94,24 @@ def test_sgemm_stream_schedule(ring, sc_steps, KS, unit_rows):
                 assert all(chunk_of(s) != chunk - 2 for s in range(done + 1, total))
             counts[-1] = issued[-1][1]
             later += counts[-1]
+
+
+@pytest.mark.parametrize('ring,sc_steps', [(5, 16), (4, 8), (3, 16)])
+@pytest.mark.parametrize('KS', [1, 2, 3, 4, 5, 6, 8, 12, 16, 20, 24, 28, 48, 56, 64])
+@pytest.mark.parametrize('unit_rows', [[2], [1, 3, 2], [3, 1, 1, 2, 3, 1, 2]])
+def test_sgemm_stream_schedule(ring, sc_steps, KS, unit_rows):
+    """The bf16 forms (units of 32 and 64 pairs; ring 3 as the FP4 form's): steps issued ring - 1 ahead across units
+    whose activation loads differ."""
+    sgemm_stream(ring, sc_steps, KS, unit_rows)
+
+
+@pytest.mark.parametrize('KS', [2, 4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 56, 64])
+@pytest.mark.parametrize('nunits', [1, 2, 3, 5])
+@pytest.mark.parametrize('scale_dwords', [0, 1])
+def test_fgemm_stream_schedule(KS, nunits, scale_dwords):
+    """The FP4 form (96 pairs, two steps ahead): each block of rows is loaded in both terms, three of the four loaders
+    also take the rows' scale dwords, and a unit's rows are gathered in two loads."""
+    sgemm_stream(3, 16, KS, [1 + u % 3 for u in range(nunits)], row_loads=2, step_loads=scale_dwords, gather_loads=2)
 
 
 def sk_order(lo, hi, KS):
