@@ -804,8 +804,12 @@ int k3moe_mxfp4_decode(const uint8_t *blocks, const uint8_t *scales, int64_t n_b
     // one pass of kDecUnroll words per thread up to kDecGrid workgroups
     long grid = (long)((n_blocks * (f32 ? 8 : 4) + 256 * kDecUnroll - 1) / (256 * kDecUnroll));
     if (grid > kDecGrid) grid = kDecGrid;
-    if (f32) hipLaunchKernelGGL(k_decode<true>, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out);
-    else hipLaunchKernelGGL(k_decode<false>, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out);
+    const bool nt = n_blocks * (f32 ? 128 : 64) > kDecKeep;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), 0, st, blocks, scales, n_blocks, out);
+    };
+    if (f32) nt ? launch(k_decode<true, true>) : launch(k_decode<true, false>);
+    else nt ? launch(k_decode<false, true>) : launch(k_decode<false, false>);
     return launch_check("decode");
   }
   long grid = (long)((n_blocks * 16 + 255) / 256);

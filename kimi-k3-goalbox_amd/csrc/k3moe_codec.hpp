@@ -145,12 +145,22 @@ __global__ __launch_bounds__(kEncThreads) void k_encode(const void *__restrict__
 // 16-byte store, 4 packed bytes for bf16 (8 values) and 2 for fp32 (4), through
 // the hardware conversion (exact for every scale byte but 255, whose values are
 // the quiet NaN), kDecUnroll of them a grid apart in flight. HBM-bound: 17 bytes
-// in, 64 or 128 out per block, stored past the caches (a larger output would only
-// evict the input: 310 -> 301 us, at 90000 x 2048 83 -> 66). A TP8 rank's gate
-// weights to bf16: 301 us, 5.9 TB/s (774 us with a byte per thread and the bit
-// construction).
+// in, 64 or 128 out per block. A TP8 rank's gate weights to bf16: 301 us, 5.9 TB/s
+// (774 us with a byte per thread and the bit construction).
+//
+// NT: outputs of more than kDecKeep bytes, which the caches do not hold, are stored
+// past them (they would only evict the input: the gate weights 310 -> 301 us, 90000
+// x 2048 to bf16 83 -> 66); smaller ones stay for the kernel that reads them. us of
+// the decode / with a torch amax after it / with a matrix product of 64 rows, kept
+// and (past the caches):
+//   bf16  16 MB   9.9 / 19.1 / 29.9 (9.6 / 19.1 / 33.7)      fp32  32 MB   9.9 / 30.2 (9.9 / 33.8)
+//         64 MB  14.0 / 47.1 / 38.2 (13.8 / 56.5 / 44.3)           64 MB  12.9 / 38.2 (11.5 / 44.5)
+//        128 MB  26.0 / 81.8 / 54.3 (26.5 / 103.0 / 65.4)         128 MB  23.8 / 56.3 (25.4 / 70.5)
+//        160 MB  37.4 / 104.4 / 69.1 (31.4 / 128.3 / 77.6)        192 MB  33.9 / 76.6 (33.2 / 95.6)
+//        256 MB  62.5 / 196.2 / 134.6 (49.9 / 203.2 / 121.7)      256 MB  57.8 / 125.8 (47.9 / 138.5)
 constexpr int kDecUnroll = 4;
-template <bool F32>
+constexpr int64_t kDecKeep = (int64_t)128 << 20;
+template <bool F32, bool NT>
 __global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ blocks, const uint8_t *__restrict__ scales,
                                                 int64_t n_blocks, void *__restrict__ out) {
   constexpr int LPB = F32 ? 8 : 4;  // lanes per block
@@ -182,7 +192,8 @@ __global__ __launch_bounds__(256) void k_decode(const uint8_t *__restrict__ bloc
         const uint32_t nan = F32 ? 0x7FC00000u : 0x7FC07FC0u;
         o = u32x4{nan, nan, nan, nan};
       }
-      __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(out) + u);
+      if constexpr (NT) __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(out) + u);
+      else reinterpret_cast<u32x4 *>(out)[u] = o;
     }
   }
 }

@@ -154,3 +154,18 @@ def test_decode_of_unaligned_blocks(gpu, n, offset, dtype):
     bits = torch.int32 if dtype == torch.float32 else torch.int16
     assert torch.equal(got.isnan(), want.isnan())
     assert torch.equal(torch.where(got.isnan(), 0, got.view(bits)), torch.where(want.isnan(), 0, want.view(bits)))
+
+
+@pytest.mark.parametrize('dtype,extra', [(torch.bfloat16, 0), (torch.bfloat16, 1), (torch.float32, 1)])
+def test_decode_on_both_sides_of_the_kept_size(gpu, dtype, extra):
+    """Outputs of 128 MiB and one block more (stored past the caches) equal their halves'."""
+    n = (128 << 20)//(64 if dtype == torch.bfloat16 else 128) + extra
+    say(f'case: decode {n} blocks to {dtype}')
+    g = torch.Generator(device=gpu).manual_seed(n)
+    blocks = torch.randint(0, 256, (n, 16), generator=g, dtype=torch.uint8, device=gpu)
+    scales = torch.randint(0, 256, (n,), generator=g, dtype=torch.uint8, device=gpu)
+    whole = k3moe.mxfp4_decode(blocks, scales, dtype).view(n, 32)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    for part in (slice(0, n//2), slice(n//2, n)):
+        half = k3moe.mxfp4_decode(blocks[part], scales[part], dtype).view(-1, 32)
+        assert torch.equal(whole[part].view(bits), half.view(bits))
