@@ -30,11 +30,11 @@ int main(int argc, char **argv) {  // per line: tokens experts topk hidden laten
     Plan p;
     make_plan(d, 256, p, 0);
     auto at = [&](int j) { return reinterpret_cast<const void *>((uintptr_t)4096 + v[7 + j]); };
-    const size_t y_end = p.o_ebf;  // the pair outputs' area ends where the next one starts
+    const size_t y_end = p.o_ids;  // the pair outputs' area ends where the next one starts
     place_plan(p, at(0), at(1), at(2), at(3), at(4), at(5), at(6), at(7), at(8));
     const size_t h = (size_t)p.P * p.I * 2;
     const bool split = p.fgemm, streams = !p.sgemm && !p.xgemm;
-    const size_t room = p.path != kPathGeneral ? 0 : (p.o_h == p.o_hq ? p.o_y - p.o_hq : p.o_xq - p.o_h);
+    const size_t room = p.path != kPathGeneral ? 0 : (p.o_h == p.o_hq ? p.o_ebf - p.o_hq : p.o_xq - p.o_h);
     printf("%d %d %d %d %d %d %d\n", p.path == kPathGeneral, p.rgemm, p.sgemm != 0, p.xgemm, p.fgemm,
            p.path != kPathGeneral || split || h <= room,
            p.path != kPathGeneral ||
