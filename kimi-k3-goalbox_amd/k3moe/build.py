@@ -31,6 +31,15 @@ REPO = os.path.dirname(PKG_ROOT)
 OUT = os.path.join(HERE, 'libk3moe.so')
 ARCH = os.environ.get('K3MOE_ARCH', 'gfx950')
 
+# Every kernel starts at a multiple of this many bytes of its code object (the persistent ones at their own): the
+# general path's kernels too depend on where they lie. us of a TP8 rank's step at 65 / 129 / 203 tokens and the Kimi
+# block at 128 / 777, medians of four runs: at 256 B (the compiler's) 222.2 / 252.0 / 264.3 / 453.9 / 672.2, 512 B
+# 222.2 / 252.1 / 264.3 / 453.7 / 670.4, 1 KiB 221.5 / 251.4 / 263.1 / 453.2 / 670.2, 2 KiB 222.2 / 252.0 / 263.2 /
+# 453.9 / 672.7, 8 KiB 222.2 / 252.2 / 263.7 / 452.9 / 671.5, 32 KiB 222.4 / 252.7 / 264.6 / 453.3 / 670.7; before the
+# persistent kernels left the code object 221.9 / 251.8 / 263.1 / 455.6 / 674.0 (a second run: 1 KiB 223.0 / 251.6 /
+# 263.7 / 452.6 / 668.7, before 221.9 / 250.8 / 262.6 / 456.0 / 669.8).
+KERNEL_ALIGN = 1024
+
 # Translation units, each a code object of its own (k3moe_persistent.hip: why).
 SOURCES = ['k3moe.hip', 'k3moe_persistent.hip']
 
@@ -46,7 +55,7 @@ def command(out: str = OUT, source: str = SOURCES[0], how: str = '-shared') -> l
     """The hipcc line that makes `out` (how: '-shared' a library, '-c' an object) of one source."""
     return [hipcc(), f'--offload-arch={ARCH}', '-O3', '-std=c++17', '-fPIC', how, '-ffp-contract=off',
             '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
-            '-Wno-unused-command-line-argument',
+            '-Xarch_device', f'-falign-functions={KERNEL_ALIGN}', '-Wno-unused-command-line-argument',
             '-I', os.path.join(REPO, 'include'), os.path.join(CSRC, source), '-o', out]
 
 

@@ -216,11 +216,13 @@ def test_persistent_kernels_lie_alone_at_their_alignment():
     from k3moe import build
     plan = open(os.path.join(build.CSRC, 'k3moe_plan.hpp')).read()
     align = int(re.search(r'kPersistentAlign = (\d+);', plan).group(1))
-    tables = [t for t in build.kernel_addresses(_native.LIB_PATH) if any('k_moe_' in name for name in t)]
-    assert len(tables) == 1 and len(tables[0]) == 20
-    for name, address in tables[0].items():
+    tables = build.kernel_addresses(_native.LIB_PATH)
+    persistent = [t for t in tables if any('k_moe_' in name for name in t)]
+    assert len(persistent) == 1 and len(persistent[0]) == 20
+    for name, address in persistent[0].items():
         assert 'k_moe_decode' in name or 'k_moe_single' in name, name
         assert address % align == 0, (name, address)
+    assert all(a % build.KERNEL_ALIGN == 0 for t in tables for a in t.values())
 
 
 PACKED_PROBE = r'''
