@@ -59,8 +59,8 @@ extern "C" {
 #define K3MOE_PATH_GROUPED 3
 #define K3MOE_PATH_STREAMED 4
 #define K3MOE_PATH_SINGLE 5 /* the single-token kernel (fails with K3MOE_EINVAL when the
-                             * shape does not fit it: one token, topk <= 8, experts <= 512,
-                             * latent a multiple of 512 up to 8192, inter <= 256) */
+                             * shape does not fit it: one token, topk <= 16, experts <= 1024,
+                             * latent a multiple of 512 up to 8192, inter <= 512) */
 #define K3MOE_PATH_GROUPED_BF16 6 /* grouped GEMMs on bf16 MFMA (same conditions as GROUPED) */
 
 /* Element type codes. */

@@ -104,7 +104,7 @@ int device_cus() {
 }
 
 // K3MOE_TRACE=1 in the environment makes decode steps record per-workgroup
-// phase timestamps (32 x uint64 per workgroup, 100 MHz) in the last 256 KiB
+// phase timestamps (kTraceSlots x uint64 per workgroup, 100 MHz) in the last 512 KiB
 // of the workspace, a profiling aid; the workspace size includes that area.
 // Test hook (k3moe_debug_stall): > 0 makes every later step's router-logit
 // waits give up after this many polls; 0, the default, leaves them bounded by

@@ -36,9 +36,9 @@
 // 64-token kernels' for every batch; inside the block the MoE step's, free before
 // and after it, takes the partials and the normalised rows.
 //
-// Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 22 + 7 us at 65
-// tokens (62 in two skinny launches), 96 at 777 (407), 203 at 2048 (988); <1> with
-// its norm 20 + 5, 74 + 7 (416), 165 + 11 us (1024). With four MFMA waves <0> took 26,
+// Measured on a Kimi K3 TP8 rank (h 7168, lh 3584, S 768): <0> 21 + 6 us at 65
+// tokens (62 in two skinny launches), 98 at 777 (407), 208 at 2048 (988); <1> with
+// its norm 20 + 5 + 5, 75 + 7 (416), 169 + 10 us (1024). With four MFMA waves <0> took 26,
 // 109 and 213 us, <1> 24, 73 and 165; timing builds of that <0> at 777: without the
 // loads 83 us, without the MFMAs 80, without either 36, and the loads about 50 KB/us a
 // CU also with every line in L2.

@@ -1,10 +1,12 @@
 // The persistent kernels, in a translation unit and so a code object of their
-// own, each at a multiple of kPersistentAlign: a decode step of 10 to 60 us
-// depends on where in its code object a kernel lies, by up to 2 % with the same
-// instructions (each phase fetches its code anew), so no other kernel may move
-// them. us of 64 experts x 2048 at 8 / 32 tokens, a TP8 rank at 8 / 64 tokens, the
-// Kimi rank's block at 1 / 6, medians of four runs in turn (of one layout they
-// differ by 0.1 %):
+// own, each at a multiple of kPersistentAlign: the time of a decode step of 10 to
+// 60 us depends on where in its code object the kernel lies, by up to 2 % with the
+// same instructions, so no other kernel may move them. (By which mechanism is not
+// known; where the buffers lie moves a time by up to 1 % too, so that layouts are
+// compared on the same buffers.) us of 64 experts x 2048 at 8 / 32 tokens, a TP8
+// rank at 8 / 64 tokens, the Kimi rank's block at 1 / 6, medians of four runs in
+// turn (of one layout they differ by 0.1 %; lines of other runs by their difference
+// from the first):
 //   the library before the grouped and latent GEMMs joined it
 //                             30.57  38.21  60.75  183.3  52.39  100.6
 //   beside those GEMMs        30.84  38.27  60.87  183.4  52.64  100.2
@@ -18,6 +20,9 @@
 //                    32 KiB   30.63  38.33  60.84  183.2  52.52  100.2
 //                    64 KiB   30.84  38.27  61.12  183.1  52.73  100.3
 // 32 KiB with the single-token kernels first: 30.61, 38.25, 60.87, 183.9, 52.72, 100.4.
+// Over nine placements of the buffers, 64 experts at 8 / 32, a TP8 rank at 8, the block at
+// 1: before those GEMMs 30.47, 38.22, 59.40, 51.25; beside them 30.74, 38.27, 59.56, 51.46;
+// here 30.55, 38.25, 59.59, 51.34.
 #include <hip/hip_runtime.h>
 
 #include "k3moe_persistent.hpp"

@@ -7,7 +7,7 @@
 //            per CU, phases handed over through tagged slots and at most two
 //            grid barriers (k3moe_decode.hpp)
 //   general  any B: a chain of eight to ten kernels (k3moe_general.hpp,
-//            k3moe_xgemm.hpp, k3moe_fgemm.hpp)
+//            k3moe_lgemm.hpp, k3moe_sgemm.hpp, k3moe_fgemm.hpp, k3moe_xgemm.hpp)
 // The workspace starts with a control block (kCtlBytes): the barrier counters
 // of the persistent kernel and a sticky error word. It must be zero before the
 // first step; the barrier counters only grow (32-bit, wrapping), and each
@@ -336,8 +336,11 @@ struct LgPlan {
 
 // Cycles of one 64-k step, to rank the variants by: the MFMAs, or the LDS traffic
 // (4 (RW + TW) KiB written, 8 (RW + TW) KiB read, 128 bytes a cycle), whichever is
-// longer. (The reads are those of 2 x 2 waves; the 4 x 2 that run read 8 RW + 16 TW
-// KiB. The times above are of the choices that this estimate makes.)
+// longer. A ranking, not a model of the time: the reads counted are those of 2 x 2 waves
+// (the 4 x 2 that run read 8 RW + 16 TW KiB), and the rate of the loads is not in it. At
+// 2.4 GHz it gives <0> 44 us at 777 tokens of a Kimi rank and <1> 32 (98 and 75
+// measured), 57 and 60 at 1500 (141, 139), 97 and 70 at 2048 (208, 169), 6.6 each at 65 (21,
+// 20). The choices it makes have not been compared with every other tile.
 inline long lgemm_step_cost(int RW, int TW) {
   const long mfma = 32L * RW * TW, lds = 96L * (RW + TW);
   return (mfma > lds ? mfma : lds) + 60;
@@ -472,8 +475,10 @@ inline void make_plan(const k3moe_dims &d, int n_cus, Plan &p, int trace = 0) {
   // 147 + 88 / 152 + 89 + 5, n = 15: 197 + 96 / 176 + 112 / 177 + 106 + 7, n = 31: 264 +
   // 157 / 258 + 152 / 217 + 129 + 12, n = 62: 411 + 251 / 353 + 250 / 297 + 195 + 19. The
   // unsharded experts, n = 85: 3508 + 1684 / 2741 + 1339 / 2260 + 1142 + 23; the Kimi rank,
-  // n = 14: 303 + 175 / 318 + 170, n = 27: 383 + 235 / 358 + 201. (FP4's fp32 sums are of
-  // truncated blocks: it is not taken where the exact ones were.)
+  // n = 14: 303 + 175 / 318 + 170, n = 27: 383 + 235 / 358 + 201. (Each line of one run on one
+  // card; medians of later runs differ by up to 10 %.) FP4's fp32 sums are of truncated
+  // blocks: it is not taken where the exact ones were. The form of 64 pairs is at its limit
+  // of 168 VGPRs, with 9 spilled in gate/up and 1 in down, outside the k-loop.
   const bool widths = p.K % 128 == 0 && p.I % 128 == 0, fp4_widths = p.K % 512 == 0 && p.I % 256 == 0;
   const bool grouped = d.path == K3MOE_PATH_GROUPED || d.path == K3MOE_PATH_GROUPED_BF16;
   const bool many = (long)p.P >= (long)kXMinPairsPerExpert * p.E;

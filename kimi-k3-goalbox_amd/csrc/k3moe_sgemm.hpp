@@ -32,10 +32,10 @@
 //
 // Measured (gate/up + down us; per-16-token streams and the former FP4 GEMMs, whose
 // loads ran two steps ahead of four MFMA waves, in brackets): a TP8 rank's shard at 203
-// tokens 140 + 84 (286 + 100), at 700 197 + 96 (620 + 154), at 2999 297 + 195 (314 + 303);
-// the unsharded experts at 4096 2260 + 1142 (2678 + 1209), at 700 1290 + 644 (3658 +
-// 1489); the Kimi rank at 777 303 + 172 (754 + 245). At 203 tokens HBM bounds it (740
-// MB of gate/up weights at 5.3 TB/s). At 85 tokens per expert timing builds of the
+// tokens 140 + 80 (286 + 100), at 700 199 + 101 (620 + 154), at 2999 304 + 200 (314 + 303); the
+// unsharded experts at 4096 2283 + 1199 (2678 + 1209), at 700 1299 + 653 (3658 + 1489); the
+// Kimi rank at 777 319 + 178 (754 + 245; 282 + 161 before the clock falls). At 203 tokens HBM
+// bounds it (740 MB of gate/up weights at 5.3 TB/s). At 85 tokens per expert timing builds of the
 // bf16 form took 1604 us with neither loads nor decode (the matrix cores' rate of a
 // large library product), 1951 without the loads, 1777 without the MFMAs.
 #pragma once
